@@ -758,6 +758,7 @@ void field_mesh(const kem_mesh* m, kem::FieldMesh& f)
     f.far6 = m->far6;
     f.far3 = m->far3;
     f.far6_cl = m->far6_cl;
+    f.triangles = m->all_triangles;
     f.axisym = m->has_axisym;
 }
 

@@ -62,6 +62,88 @@ __device__ __forceinline__ double rsqrt_acc(double a)
     return __builtin_fma(y * h, __builtin_fma(0.375, h, 0.5), y);
 }
 
+// ---------------------------------------------------------------- elementary functions
+// The closed forms take a square root per corner, a logarithm of a quotient per edge and one
+// arctangent per element.  These are written out so that a quotient costs one reciprocal, and
+// none of them the library's special cases: corrected hardware estimates, and polynomials that
+// interpolate the odd series of atanh and atan at Chebyshev nodes (worst error 5e-18 and 1.2e-18
+// of the function over the reduced range, computed with 60 digits).  One triangle: 6 logarithms, 9
+// square roots and an atan2 of the library before, 3 + 3 + 1 of these now.  With the wavefronts that
+// share a group of points (k_field_near_culled, k_assemble_near): the near pass of 64 points over 192
+// triangles 824 -> 84 us, of 4,096 points over 1,728 462 -> 90 us, the closed-form entries of 3,112
+// rows with dielectric ones 5.2 -> 0.67 ms.
+// Coefficients, highest power first (the log series ends with log 2).  Read through a pointer that the
+// compiler cannot see through, so that they stay scalar loads at each use: as literals they were kept in
+// vector registers over the element loops (196 of them, 2 wavefronts per SIMD).
+__constant__ const double kLogSeries[12] = {0.15631534707431224, 0.07491639460673266, 0.10845291032779812, 0.11734265179376593,
+                                            0.13335179661515711, 0.15384543917753166, 0.1818181989926796, 0.22222222198216113,
+                                            0.28571428571600266, 0.3999999999999952, 0.6666666666666666, 0.6931471805599453};
+__constant__ const double kAtanSeries[9] = {-0.03956743974276833, 0.05716019885233984, -0.0665491123778113,
+                                            0.07691817726923288, -0.09090897022088731, 0.11111110943517653,
+                                            -0.14285714284545636, 0.19999999999996856, -0.3333333333333333};
+__device__ __forceinline__ const double* opaque(const double* p)
+{
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
+// sqrt(a), a >= 0, to about an ulp: a * rsq(a) and one correction of its residual
+__device__ __forceinline__ double sqrt_acc(double a)
+{
+    const double y = rsqrt_acc(a);
+    const double s = a * y;
+    const double r = __builtin_fma(0.5 * y, __builtin_fma(-s, s, a), s);
+    return a == 0. ? 0. : r;
+}
+
+// a / b to about an ulp: v_rcp_f64 with one third-order correction, then the quotient's residual
+__device__ __forceinline__ double quot_acc(double a, double b)
+{
+    const double y0 = __builtin_amdgcn_rcp(b);
+    const double e = __builtin_fma(-b, y0, 1.0);
+    const double y = __builtin_fma(y0, __builtin_fma(e, e, e), y0);
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
+// log(a / b) for a > 0 (infinite for b = 0, not a number for b < 0): a is scaled by a power of two to within a
+// factor 2 of b, then log(a / b) = 2 atanh((a - b) / (a + b)), |(a - b) / (a + b)| <= 1/3
+__device__ __forceinline__ double log_quot(double a, double b)
+{
+    const int k = __builtin_amdgcn_frexp_exp(a) - __builtin_amdgcn_frexp_exp(b);
+    const double m = __builtin_ldexp(a, -k);
+    const double s = quot_acc(m - b, m + b);
+    const double z = s * s;
+    const double* c = opaque(kLogSeries);
+    double q = c[0];
+#pragma unroll
+    for (int i = 1; i < 11; i++) q = __builtin_fma(q, z, c[i]);
+    const double r = __builtin_fma(s * z, q, s + s);
+    const double l = __builtin_fma((double)k, c[11], r);
+    return b > 0. ? l : b == 0. ? __builtin_inf() : __builtin_nan("");
+}
+
+// the angle of (x, y), y >= 0, in [0, pi] (0 for x = y = 0): the smaller over the larger of |x| and y,
+// beyond tan(pi/12) turned back by pi/6, then the odd series on |t| <= tan(pi/12)
+__device__ __forceinline__ double angle_acc(double y, double x)
+{
+    const double ax = fabs(x);
+    const bool steep = y > ax;
+    const double lo = steep ? ax : y, hi = steep ? y : ax;
+    const bool turn = lo > 0.2679491924311227 * hi;
+    const double c = turn ? 0.5773502691896258 : 0.;  // tan(pi/6)
+    const double den = __builtin_fma(lo, c, hi);
+    const double t = quot_acc(__builtin_fma(-hi, c, lo), den == 0. ? 1. : den);
+    const double z = t * t;
+    const double* p = opaque(kAtanSeries);
+    double q = p[0];
+#pragma unroll
+    for (int i = 1; i < 9; i++) q = __builtin_fma(q, z, p[i]);
+    double r = __builtin_fma(t * z, q, t) + (turn ? kPi / 6. : 0.);
+    r = steep ? kPi / 2. - r : r;
+    return x < 0. ? kPi - r : r;
+}
+
 // ---------------------------------------------------------------- cubature
 // pref * sum_g w_g (P - Q_g)/|P - Q_g|^3 and pref * sum_g w_g/|P - Q_g| (..._TriNP / _RectNP)
 template <int NQ, bool FIELD>
@@ -140,7 +222,7 @@ __device__ __forceinline__ F4 line_analytic(const double* __restrict__ g, double
         }
     }
     F4 r;
-    r.p = dia / (4. * kEps0) * log((DaP + DbP + L) / (DaP + DbP - L));
+    r.p = dia / (4. * kEps0) * log_quot(DaP + DbP + L, DaP + DbP - L);
     double den = (DaE * (DaE + DbE + L) * (DaE + DbE - L) * DbE) * 4. * kEps0;
     den = -1. / den;
     const double s = 2. * L * dia * den;
@@ -150,107 +232,85 @@ __device__ __forceinline__ F4 line_analytic(const double* __restrict__ g, double
     return r;
 }
 
-// ---------------------------------------------------------------- solid angle
-// Van Oosterom-Strackee: Omega = 2 atan2(|u0.(u1 x u2)|, 1 + u0.u1 + u0.u2 + u1.u2), signed by h
-__device__ __forceinline__ double tri_omega(const double* __restrict__ V, double px, double py, double pz)
-{
-    double u[3][3];
-#pragma unroll
-    for (int v = 0; v < 3; v++) {
-        const double dx = V[3 * v] - px, dy = V[3 * v + 1] - py, dz = V[3 * v + 2] - pz;
-        const double im = rsqrt_acc(dx * dx + dy * dy + dz * dz);
-        u[v][0] = im * dx;
-        u[v][1] = im * dy;
-        u[v][2] = im * dz;
-    }
-    const double x = 1. + (u[0][0] * u[1][0] + u[0][1] * u[1][1] + u[0][2] * u[1][2]) +
-                     (u[0][0] * u[2][0] + u[0][1] * u[2][1] + u[0][2] * u[2][2]) +
-                     (u[1][0] * u[2][0] + u[1][1] * u[2][1] + u[1][2] * u[2][2]);
-    const double a0 = u[1][1] * u[2][2] - u[1][2] * u[2][1];
-    const double a1 = u[1][2] * u[2][0] - u[1][0] * u[2][2];
-    const double a2 = u[1][0] * u[2][1] - u[1][1] * u[2][0];
-    const double y = fabs(u[0][0] * a0 + u[0][1] * a1 + u[0][2] * a2);
-    return fabs(2. * atan2(y, x));
-}
-
-// KSolidAngle::SolidAngleTriangleAsArray (KSolidAngle.hh:58-144)
-__device__ __forceinline__ double solid_angle_tri(const double* __restrict__ g, double px, double py, double pz)
-{
-    const double cx = px - g[KG_HX], cy = py - g[KG_HY], cz = pz - g[KG_HZ];
-    const double h = g[KG_NX] * cx + g[KG_NY] * cy + g[KG_NZ] * cz;
-    double res = (sqrt(cx * cx + cy * cy + cz * cz) <= 1.e-12) ? 2. * kPi : tri_omega(g + KG_V, px, py, pz);
-    return h < 0. ? -res : res;
-}
-
-// KSolidAngle::SolidAngleRectangleAsArray (KSolidAngle.hh:166-305): two triangles P0P1P2 and P2P3P0;
-// in the plane: 2 pi inside, 0 outside
-__device__ __forceinline__ double solid_angle_rect(const double* __restrict__ g, double px, double py, double pz)
-{
-    const double h = g[KG_NX] * (px - g[KG_HX]) + g[KG_NY] * (py - g[KG_HY]) + g[KG_NZ] * (pz - g[KG_HZ]);
-    double res;
-    if (fabs(h) < 1.e-12) {
-        const double* V = g + KG_V;
-        const double* s1 = g + KG_SV;
-        const double* s2 = g + KG_SV + 3;
-        const double dx = V[0] - px, dy = V[1] - py, dz = V[2] - pz;
-        const double A = g[KG_A], B = g[KG_B];
-        const double l1 = (-1) * (dx * s1[0] + dy * s1[1] + dz * s1[2]) / (A * A);
-        const double l2 = (-1) * (dx * s2[0] + dy * s2[1] + dz * s2[2]) / (B * B);
-        res = (l1 > 0. && l1 < 1. && l2 > 0. && l2 < 1.) ? 2. * kPi : 0.;
-    } else {
-        const double* V = g + KG_V;
-        const double t1[9] = {V[0], V[1], V[2], V[3], V[4], V[5], V[6], V[7], V[8]};
-        const double t2[9] = {V[6], V[7], V[8], V[9], V[10], V[11], V[0], V[1], V[2]};
-        res = tri_omega(t1, px, py, pz) + tri_omega(t2, px, py, pz);
-    }
-    return h < 0. ? -res : res;
-}
-
 // ---------------------------------------------------------------- closed form (RWG)
-// Line-integral term IqLFieldAndPotential: returns (field part, potential part).  Edges are
-// visited in a rolled loop that re-reads the per-edge geometry (scalar loads) and recomputes
-// the two vertex distances of each edge, keeping register pressure low.
-template <int NE, bool FIELD>
-__device__ __forceinline__ F4 edge_logs(const double* __restrict__ g, double px, double py, double pz, int count,
-                                        int line, double dist)
+// One evaluation at P: the solid angle and the edge logarithms (IqLFieldAndPotential) from the corner
+// vectors a_v = V_v - P and their lengths, each taken once.
+//
+// Solid angle (KSolidAngle.hh:58-305), Van Oosterom and Strackee without normalising the corner vectors:
+// tan(Omega / 2) = |a0.(a1 x a2)| / (R0 R1 R2 + (a0.a1) R2 + (a1.a2) R0 + (a2.a0) R1), the triple product
+// being twice the area times |h|; a rectangle's two triangles P0P1P2 and P2P3P0 add as angles of complex
+// numbers; signed by h.  Triangle: 2 pi at the centroid; rectangle: in the plane 2 pi inside, 0 outside.
+//
+// NEAR: the pair is in the numeric policy's near set (within 4.6 sizes), and the logarithm is that of the
+// quotient.  The rwg policy also evaluates distant pairs, whose terms cancel like eps dr^2: there the difference
+// of two logarithms keeps the roundings of the reference (the quotient's is closer to the truth, and 1.4 times
+// further from the reference at dr = 2,000).
+template <int NE, bool FIELD, bool NEAR>
+__device__ __forceinline__ F4 closed_form_at(const double* __restrict__ g, double px, double py, double pz, int count,
+                                             int line, double dist)
 {
-    F4 acc{0., 0., 0., 0.};
+    const double nx = g[KG_NX], ny = g[KG_NY], nz = g[KG_NZ];
+    const double cx = px - g[KG_HX], cy = py - g[KG_HY], cz = pz - g[KG_HZ];
+    const double h = nx * cx + ny * cy + nz * cz;
+    double ax[NE], ay[NE], az[NE], R[NE];
+#pragma unroll
+    for (int v = 0; v < NE; v++) {
+        const double* V = g + KG_V + 3 * v;
+        ax[v] = V[0] - px;
+        ay[v] = V[1] - py;
+        az[v] = V[2] - pz;
+        R[v] = sqrt_acc(ax[v] * ax[v] + ay[v] * ay[v] + az[v] * az[v]);
+    }
+    double om;
+    {
+        auto dot = [&](int a, int b) { return ax[a] * ax[b] + ay[a] * ay[b] + az[a] * az[b]; };
+        auto low = [&](int a, int b, int c) {
+            return R[a] * R[b] * R[c] + dot(a, b) * R[c] + dot(b, c) * R[a] + dot(c, a) * R[b];
+        };
+        // g[KG_PREF] = area / (4 pi eps0): twice the triangle's area (each half of a rectangle: its area)
+        const double y = g[KG_PREF] * ((NE == 3 ? 2. : 1.) / kK) * fabs(h);
+        if (NE == 3) {
+            om = 2. * angle_acc(y, low(0, 1, 2));
+            if (cx * cx + cy * cy + cz * cz <= 1.e-24) om = 2. * kPi;
+        } else {
+            const double x1 = low(0, 1, 2), x2 = low(2, NE - 1, 0);
+            om = 2. * angle_acc(fabs(y * (x1 + x2)), __builtin_fma(x1, x2, -y * y));
+            if (fabs(h) < 1.e-12) {
+                const double A = g[KG_A], B = g[KG_B];
+                const double* s1 = g + KG_SV;
+                const double* s2 = g + KG_SV + 3;
+                const double l1 = (-1) * (ax[0] * s1[0] + ay[0] * s1[1] + az[0] * s1[2]) / (A * A);
+                const double l2 = (-1) * (ax[0] * s2[0] + ay[0] * s2[1] + az[0] * s2[2]) / (B * B);
+                om = (l1 > 0. && l1 < 1. && l2 > 0. && l2 < 1.) ? 2. * kPi : 0.;
+            }
+        }
+        om = h < 0. ? -om : om;
+    }
+    F4 acc{FIELD ? nx * om : 0., FIELD ? ny * om : 0., FIELD ? nz * om : 0., -h * om};
+    // a rolled loop with the corner vectors rotating through the same registers: unrolled, the edges' divisions
+    // and series interleave (k_assemble_near<true>: 143 vector registers and 3 wavefronts per SIMD, 125 and 4 so)
 #pragma unroll 1
     for (int e = 0; e < NE; e++) {
-        const int e1 = (e + 1 == NE) ? 0 : e + 1;
         const double* u = g + KG_U + 3 * e;
         const double* m = g + KG_M + 3 * e;
-        const double* mid = g + KG_MID + 3 * e;
-        const double* va = g + KG_V + 3 * e;
-        const double* vb = g + KG_V + 3 * e1;
-        const double ax = va[0] - px, ay = va[1] - py, az = va[2] - pz;
-        const double bx = vb[0] - px, by = vb[1] - py, bz = vb[2] - pz;
-        const double rM = sqrt(ax * ax + ay * ay + az * az);
-        const double rP = sqrt(bx * bx + by * by + bz * bz);
-        const double sM = ax * u[0] + ay * u[1] + az * u[2];
-        const double sP = bx * u[0] + by * u[1] + bz * u[2];
-        bool have = false;
-        double val = 0.;
-        if (line != e) {
-            double nom, den;
-            if ((rM + sM) > (rP - sP)) {
-                nom = rP + sP;
-                den = rM + sM;
-            } else {
-                nom = rM - sM;
-                den = rP - sP;
-            }
-            val = log(nom) - log(den);
-            have = true;
-        } else if (count == 1 && fabs(dist / sM) < kLogArgQuotient) {
-            // point on the edge line: second-order Taylor argument (LogArgTaylor)
+        const double rM = R[0], rP = R[1];
+        const double sM = ax[0] * u[0] + ay[0] * u[1] + az[0] * u[2];
+        const double sP = ax[1] * u[0] + ay[1] * u[1] + az[1] * u[2];
+        const bool up = (rM + sM) > (rP - sP);
+        double nom = up ? rP + sP : rM - sM;
+        double den = up ? rM + sM : rP - sP;
+        bool have = true;
+        if (line == e) {
+            // point on the edge line: second-order Taylor argument (LogArgTaylor), or no logarithm
             double q = fabs(dist / sM);
+            have = count == 1 && q < kLogArgQuotient;
             q = q < 1.e-14 ? 1.e-14 : q;
-            val = log(rP + sP) - log(0.5 * fabs(sM) * q * q);
-            have = true;
+            nom = rP + sP;
+            den = 0.5 * fabs(sM) * q * q;
         }
+        const double val = NEAR ? log_quot(nom, den) : log(nom) - log(den);
         if (have) {
-            const double t = m[0] * (px - mid[0]) + m[1] * (py - mid[1]) + m[2] * (pz - mid[2]);
+            const double t = m[0] * ax[0] + m[1] * ay[0] + m[2] * az[0];  // minus the point's distance from the edge
             if (FIELD) {
                 acc.x += m[0] * val;
                 acc.y += m[1] * val;
@@ -258,45 +318,46 @@ __device__ __forceinline__ F4 edge_logs(const double* __restrict__ g, double px,
             }
             acc.p += t * val;
         }
+        const double tx = ax[0], ty = ay[0], tz = az[0], tr = R[0];
+#pragma unroll
+        for (int v = 0; v + 1 < NE; v++) {
+            ax[v] = ax[v + 1];
+            ay[v] = ay[v + 1];
+            az[v] = az[v + 1];
+            R[v] = R[v + 1];
+        }
+        ax[NE - 1] = tx;
+        ay[NE - 1] = ty;
+        az[NE - 1] = tz;
+        R[NE - 1] = tr;
     }
     return acc;
 }
 
-template <int NE>
-__device__ __forceinline__ double solid_angle(const double* __restrict__ g, double px, double py, double pz)
-{
-    return NE == 3 ? solid_angle_tri(g, px, py, pz) : solid_angle_rect(g, px, py, pz);
-}
-
-template <int NE, bool FIELD>
-__device__ __forceinline__ F4 closed_form_at(const double* __restrict__ g, double px, double py, double pz, int count,
-                                             int line, double dist)
-{
-    const double nx = g[KG_NX], ny = g[KG_NY], nz = g[KG_NZ];
-    const double h = nx * (px - g[KG_HX]) + ny * (py - g[KG_HY]) + nz * (pz - g[KG_HZ]);
-    const double om = solid_angle<NE>(g, px, py, pz);
-    const F4 iL = edge_logs<NE, FIELD>(g, px, py, pz, count, line, dist);
-    return F4{nx * om + iL.x, ny * om + iL.y, nz * om + iL.z, (-h * om) - iL.p};
-}
-
 // KElectrostaticRWG{Triangle,Rectangle}Integrator::ElectricFieldAndPotential
-template <int NE, bool FIELD>
+template <int NE, bool FIELD, bool NEAR = false>
 __device__ __forceinline__ F4 closed_form(const double* __restrict__ g, double px, double py, double pz)
 {
     int count = 0, line = 99;
     double dmin = 0.;
+    // Only a point in the element's plane can lie on an edge: kMinDistToLine is far below the height bound,
+    // which leaves room for h's own rounding (a few ulps of the distance), so most wavefronts skip the test.
+    const double cx = px - g[KG_HX], cy = py - g[KG_HY], cz = pz - g[KG_HZ];
+    const double h = g[KG_NX] * cx + g[KG_NY] * cy + g[KG_NZ] * cz;
+    if (fabs(h) <= 1.e-12 + 1.e-14 * (fabs(cx) + fabs(cy) + fabs(cz))) {
 #pragma unroll 1
-    for (int e = 0; e < NE; e++) {
-        const double dx = g[KG_V + 3 * e] - px, dy = g[KG_V + 3 * e + 1] - py, dz = g[KG_V + 3 * e + 2] - pz;
-        const double* s = g + KG_SV + 3 * e;
-        const double il = g[KG_IL + e];
-        const double cx = s[1] * dz - s[2] * dy, cy = s[2] * dx - s[0] * dz, cz = s[0] * dy - s[1] * dx;
-        const double dl = sqrt(cx * cx + cy * cy + cz * cz) * il;
-        const double lam = ((-dx * s[0]) + (-dy * s[1]) + (-dz * s[2])) * (il * il);
-        if (dl < kMinDistToLine && lam >= -kTolLambda && lam <= (1. + kTolLambda)) {
-            dmin = dl;
-            count++;
-            line = e;
+        for (int e = 0; e < NE; e++) {
+            const double dx = g[KG_V + 3 * e] - px, dy = g[KG_V + 3 * e + 1] - py, dz = g[KG_V + 3 * e + 2] - pz;
+            const double* s = g + KG_SV + 3 * e;
+            const double il = g[KG_IL + e];
+            const double ex = s[1] * dz - s[2] * dy, ey = s[2] * dx - s[0] * dz, ez = s[0] * dy - s[1] * dx;
+            const double dl = sqrt(ex * ex + ey * ey + ez * ez) * il;
+            const double lam = ((-dx * s[0]) + (-dy * s[1]) + (-dz * s[2])) * (il * il);
+            if (dl < kMinDistToLine && lam >= -kTolLambda && lam <= (1. + kTolLambda)) {
+                dmin = dl;
+                count++;
+                line = e;
+            }
         }
     }
     // on a vertex (count == 2): mean of the points moved by +-1e-7 along the normal, without
@@ -312,7 +373,7 @@ __device__ __forceinline__ F4 closed_form(const double* __restrict__ g, double p
 #pragma unroll 1
     for (int r = 0; r < nrep; r++) {
         const double sg = r == 0 ? sh : -sh;
-        const F4 a = closed_form_at<NE, FIELD>(g, px + sg * g[KG_NX], py + sg * g[KG_NY], pz + sg * g[KG_NZ], count,
+        const F4 a = closed_form_at<NE, FIELD, NEAR>(g, px + sg * g[KG_NX], py + sg * g[KG_NY], pz + sg * g[KG_NZ], count,
                                                line, dmin);
         acc.x += a.x;
         acc.y += a.y;
@@ -481,11 +542,12 @@ __device__ __forceinline__ void element_far_wave_pot_n(const double* __restrict_
     return cubature_pot_n<7, T>(an + 5 * KEM_N7, pref, dx, dy, dz, d2, v);
 }
 
-// Near pass of one pair (closed forms).
+// Near pass of one pair (closed forms; NEAR as for closed_form).
+template <bool NEAR>
 __device__ __forceinline__ F4 element_near(const double* __restrict__ g, int type, double px, double py, double pz)
 {
-    if (type == KEM_TRIANGLE) return closed_form<3, true>(g, px, py, pz);
-    if (type == KEM_RECTANGLE) return closed_form<4, true>(g, px, py, pz);
+    if (type == KEM_TRIANGLE) return closed_form<3, true, NEAR>(g, px, py, pz);
+    if (type == KEM_RECTANGLE) return closed_form<4, true, NEAR>(g, px, py, pz);
     return line_analytic(g, px, py, pz);
 }
 
@@ -495,7 +557,7 @@ __device__ __forceinline__ F4 element_near_any(const double* __restrict__ g, int
                                                double pz)
 {
     if (type >= KEM_CONICSECTION) return axisym_eval<true>(g, type, px, py, pz);
-    return element_near(g, type, px, py, pz);
+    return element_near<true>(g, type, px, py, pz);
 }
 
 // ---------------------------------------------------------------- mixed precision (FP32 far field)

@@ -20,6 +20,7 @@ struct FieldMesh {
     const float* far6 = nullptr;       // 6-point far records in cluster order (kem::build_far6)
     const float* far3 = nullptr;       // 3-point far records in cluster order
     const double* far6_cl = nullptr;   // and the clusters' 6- and 3-point reach (KEM_FAR_CL_STRIDE)
+    bool triangles = false;            // holds nothing but triangles
     bool axisym = false;               // holds conic sections or rings (kernels with their integrators)
 };
 

@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "kem_device.hpp"
 #include "kem_kernels.h"
@@ -188,7 +189,7 @@ __global__ __launch_bounds__(kBlock) void k_field_near(const double* __restrict_
             const F4 v = PC == 1   ? dev::element_policy(g, recs + j * KEM_REC, policy, x, y, z)
                          : PC == 2 ? dev::element_any<true>(g, nodes + j * KEM_NODE_STRIDE, recs + j * KEM_REC,
                                                             policy, x, y, z)
-                                   : dev::element_near(g, (int)g[KG_TYPE], x, y, z);
+                                   : dev::element_near<false>(g, (int)g[KG_TYPE], x, y, z);
             const double sj = sg[MULTI ? j * nsets : j];
             dev::kahan_add(v.x, sj, s0, c0);
             dev::kahan_add(v.y, sj, s1, c1);
@@ -215,17 +216,18 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-// Near pass with cluster culling (numeric policy).  Each wavefront bounds its 64 points by the
-// sphere around their bounding box; a cluster of KEM_CLUSTER elements (Morton order) whose
-// sphere of near distances cannot reach it is skipped as a whole.  The pairs evaluated are
-// exactly the near set (the same dist2 test as the far pass); culling only removes clusters
-// proven to contain none.  Writes its own sums (one slice of the partial-sum layout that
-// k_field_combine adds), so it may run beside the far pass.  Blocks stride over the point
-// blocks, so a small grid keeps the pass's footprint to a few wavefronts per SIMD beside the
-// far kernel.  Capped at 168 VGPRs (3 wavefronts per SIMD, 16 bytes of spills): uncapped it
-// takes 173 and runs 2 per SIMD (4 M points in uneven batches 253 -> 247 ms with the cap).
-template <bool MULTI, bool AXI>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_field_near_culled(const double* __restrict__ geom,
+// Near pass with cluster culling (numeric policy).  W wavefronts share 64 points and take every W-th element
+// of a cluster; each bounds the points by the sphere around their bounding box, and a cluster of KEM_CLUSTER
+// elements (Morton order) whose sphere of near distances cannot reach it is skipped as a whole.  The pairs
+// evaluated are exactly the near set (the same dist2 test as the far pass); culling only removes clusters
+// proven to contain none.  The W sums are added in order through LDS, so the result is one slice of the
+// partial-sum layout that k_field_combine adds, and may run beside the far pass.  Blocks stride over the point
+// groups, so a small grid keeps the pass's footprint beside the far kernel.
+// What bounds it is the latency of one wavefront's elements in turn while the chip is not full (64 points:
+// one wavefront ran all of them): W = 16 up to 512 groups of points, 4 up to 4,096, 1 above.  SHAPES 0:
+// triangles only, whose kernel needs fewer registers; 1: any planar element or wire; 2: axisymmetric ones too.
+template <bool MULTI, int SHAPES, int W>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(SHAPES == 0 ? 4 : 3))) void k_field_near_culled(const double* __restrict__ geom,
                                                               const double* __restrict__ sigma,
                                                               const int32_t* __restrict__ pset, int64_t nsets,
                                                               const double* __restrict__ clusters, int64_t ncl,
@@ -236,8 +238,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
                                                               double* __restrict__ out0, double* __restrict__ out1,
                                                               double* __restrict__ out2, double* __restrict__ out3)
 {
-  for (int64_t pb = blockIdx.x; pb * kBlock < npts; pb += gridDim.x) {
-    int64_t i = pb * kBlock + threadIdx.x;
+  __shared__ double part[W > 1 ? W - 1 : 1][4][64];
+  const int lane = threadIdx.x & 63;
+  const int w = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  for (int64_t pb = blockIdx.x; pb * 64 < npts; pb += gridDim.x) {
+    int64_t i = pb * 64 + lane;
     const bool live = i < npts;
     if (!live) i = npts - 1;
     const double x = px[i], y = py[i], z = pz[i];
@@ -256,12 +261,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
         if (dx * dx + dy * dy + dz * dz > reach * reach) continue;
         int64_t e1 = (k + 1) * KEM_CLUSTER;
         if (e1 > nelem) e1 = nelem;
-        for (int64_t e = k * KEM_CLUSTER; e < e1; e++) {
+        for (int64_t e = k * KEM_CLUSTER + w; e < e1; e += W) {
             const int64_t j = order[e];
             const double* g = geom + j * KG_STRIDE;
             if (dev::is_near2(g, dev::dist2(g, x, y, z), 0)) {
-                const F4 v = AXI ? dev::element_near_any(g, (int)g[KG_TYPE], x, y, z)
-                                 : dev::element_near(g, (int)g[KG_TYPE], x, y, z);
+                const F4 v = SHAPES == 0   ? dev::closed_form<3, true, true>(g, x, y, z)
+                             : SHAPES == 1 ? dev::element_near<true>(g, (int)g[KG_TYPE], x, y, z)
+                                           : dev::element_near_any(g, (int)g[KG_TYPE], x, y, z);
                 const double sj = sg[MULTI ? j * nsets : j];
                 dev::kahan_add(v.x, sj, s0, c0);
                 dev::kahan_add(v.y, sj, s1, c1);
@@ -270,7 +276,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) voi
             }
         }
     }
-    if (live) {
+    if (W > 1) {
+        if (w > 0) {
+            part[w - 1][0][lane] = s0;
+            part[w - 1][1][lane] = s1;
+            part[w - 1][2][lane] = s2;
+            part[w - 1][3][lane] = s3;
+        }
+        __syncthreads();
+        if (w == 0) {
+            for (int q = 0; q < W - 1; q++) {
+                dev::kahan_add(part[q][0][lane], 1., s0, c0);
+                dev::kahan_add(part[q][1][lane], 1., s1, c1);
+                dev::kahan_add(part[q][2][lane], 1., s2, c2);
+                dev::kahan_add(part[q][3][lane], 1., s3, c3);
+            }
+        }
+        __syncthreads();  // part is free for the next group of points
+    }
+    if (live && w == 0) {
         out0[i] = s0;
         out1[i] = s1;
         out2[i] = s2;
@@ -543,26 +567,30 @@ __global__ __launch_bounds__(kBlock) void k_census_far32c(const double* __restri
     if (threadIdx.x < 10 && sc[threadIdx.x]) atomicAdd(&counts[threadIdx.x], sc[threadIdx.x]);
 }
 
-// Kahan-sum the per-range partials (ws[c][s][i], c = Ex, Ey, Ez, phi) in range order.
+// Kahan-sum the per-range partials (ws[c][s][i], c = Ex, Ey, Ez, phi) in range order, blockIdx.y =
+// component.  Eight loads are in flight ahead of the chain of sums (one thread per point and all components,
+// a load at a time: 36 us at 4,096 points and 55 slices).
 __global__ __launch_bounds__(kBlock) void k_field_combine(const double* __restrict__ ws, int nsplit, int64_t npts,
                                                           double* __restrict__ phi, double* __restrict__ ex,
                                                           double* __restrict__ ey, double* __restrict__ ez)
 {
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= npts) return;
-    double* outs[4] = {ex, ey, ez, phi};
-    for (int c = 0; c < 4; c++) {
-        if (!outs[c]) continue;
-        const double* p = ws + (int64_t)c * nsplit * npts;
-        double s = 0., comp = 0.;
-        for (int k = 0; k < nsplit; k++) {
-            const double yk = p[(int64_t)k * npts + i] - comp;
-            const double t = s + yk;
-            comp = (t - s) - yk;
-            s = t;
-        }
-        outs[c][i] = s;
+    const int c = blockIdx.y;
+    double* out = c == 0 ? ex : c == 1 ? ey : c == 2 ? ez : phi;
+    if (!out) return;
+    const double* p = ws + (int64_t)c * nsplit * npts + i;
+    double s = 0., comp = 0.;
+    int k = 0;
+    for (; k + 8 <= nsplit; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = p[(int64_t)(k + q) * npts];
+#pragma unroll
+        for (int q = 0; q < 8; q++) dev::kahan_add(v[q], 1., s, comp);
     }
+    for (; k < nsplit; k++) dev::kahan_add(p[(int64_t)k * npts], 1., s, comp);
+    out[i] = s;
 }
 
 // ------------------------------------------------------------------ element pairs
@@ -808,15 +836,19 @@ __global__ __launch_bounds__(kBlock) void k_asm_nodes(const double* __restrict__
 // Closed-form entries: targets in the Morton order of the element centres (order[k]), so a
 // wavefront's targets are compact; each wavefront bounds its targets by a sphere and skips the
 // element clusters that cannot hold a near pair of any of them (the culling of
-// k_field_near_culled); the entries it finds are written in place (a few per target).
+// k_field_near_culled); the entries it finds are written in place (a few per target).  The kAsmNearWaves
+// wavefronts of a block share 64 targets and take every kAsmNearWaves-th element of a cluster: 20,000
+// targets are 313 wavefronts, a third of the chip's SIMDs with one each.
+constexpr int kAsmNearWaves = 8;
 template <bool FIELD>
-__global__ __launch_bounds__(kBlock) void k_assemble_near(const double* __restrict__ geom,
+__global__ __launch_bounds__(64 * kAsmNearWaves) void k_assemble_near(const double* __restrict__ geom,
                                                           const double* __restrict__ targets,
                                                           const double* __restrict__ clusters, int64_t ncl,
                                                           const int32_t* __restrict__ order, int64_t n,
                                                           double* __restrict__ A64, float* __restrict__ A32)
 {
-    int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int64_t k = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
     const bool live = k < n;
     if (!live) k = n - 1;
     const int64_t i = order[k];
@@ -837,13 +869,13 @@ __global__ __launch_bounds__(kBlock) void k_assemble_near(const double* __restri
         if (dx * dx + dy * dy + dz * dz > reach * reach) continue;
         int64_t e1 = (c + 1) * KEM_CLUSTER;
         if (e1 > n) e1 = n;
-        for (int64_t e = c * KEM_CLUSTER; e < e1; e++) {
+        for (int64_t e = c * KEM_CLUSTER + w; e < e1; e += kAsmNearWaves) {
             const int64_t j = order[e];
             const double* g = geom + j * KG_STRIDE;
             if (!dev::is_near2(g, dev::dist2(g, cx, cy, cz), 0)) continue;
             const int type = (int)g[KG_TYPE];
-            const F4 v = type == KEM_TRIANGLE    ? dev::closed_form<3, FIELD>(g, cx, cy, cz)
-                         : type == KEM_RECTANGLE ? dev::closed_form<4, FIELD>(g, cx, cy, cz)
+            const F4 v = type == KEM_TRIANGLE    ? dev::closed_form<3, FIELD, true>(g, cx, cy, cz)
+                         : type == KEM_RECTANGLE ? dev::closed_form<4, FIELD, true>(g, cx, cy, cz)
                                                  : dev::line_analytic(g, cx, cy, cz);
             double a;
             if (!FIELD || dirichlet) {
@@ -1496,23 +1528,36 @@ void near_slice(hipStream_t st, const SideStream* side, const FieldMesh& m, cons
     }
     const int64_t ncl = (m.n + KEM_CLUSTER - 1) / KEM_CLUSTER;
     double* o = q + slice * np;
-    // beside the mixed far pass a grid of g_tuning.near_blocks blocks (0: one per point block):
+    const int64_t groups = (np + 63) / 64;
+    // beside the mixed far pass a grid of g_tuning.near_blocks * 4 wavefronts (0: one per group of points):
     // a few wavefronts per SIMD, which the far kernel's blocks do not crowd out, so the pass ends
     // with the far kernel instead of after it (measured on 1 M points x 20,000 triangles: 67.5 ms
     // with one block per point block, 64.9 ms with 64 to 512 blocks, 69.3 ms with 768).  The FP64
     // far pass runs long enough that a small grid only takes its occupancy (362 -> 367..402 ms),
     // and so does the near pass over several sets (4 M points in uneven batches: 253 -> 261 ms).
-    unsigned gn = nblocks(np);
-    if (s != st && mixed && !MULTI && g_tuning.near_blocks > 0 && (int64_t)gn > g_tuning.near_blocks)
-        gn = (unsigned)g_tuning.near_blocks;
+    unsigned gn = (unsigned)groups;
+    if (s != st && mixed && !MULTI && g_tuning.near_blocks > 0 && groups > 4 * g_tuning.near_blocks)
+        gn = (unsigned)(4 * g_tuning.near_blocks);
+    auto launch = [&](auto shapes, auto waves) {
+        constexpr int W = decltype(waves)::value;
+        k_field_near_culled<MULTI, decltype(shapes)::value, W><<<gn, 64 * W, 0, s>>>(
+            m.geom, sg, pset, nsets, m.clusters, ncl, m.order, m.n, px, py, pz, np, o, o + ns * np, o + 2 * ns * np,
+            o + 3 * ns * np);
+    };
+    auto by_waves = [&](auto shapes) {
+        if (groups <= 512)
+            launch(shapes, std::integral_constant<int, 16>());
+        else if (groups <= 4096)
+            launch(shapes, std::integral_constant<int, 4>());
+        else
+            launch(shapes, std::integral_constant<int, 1>());
+    };
     if (m.axisym)
-        k_field_near_culled<MULTI, true><<<gn, kBlock, 0, s>>>(m.geom, sg, pset, nsets, m.clusters, ncl,
-                                                                        m.order, m.n, px, py, pz, np, o,
-                                                                        o + ns * np, o + 2 * ns * np, o + 3 * ns * np);
+        by_waves(std::integral_constant<int, 2>());
+    else if (m.triangles)
+        by_waves(std::integral_constant<int, 0>());
     else
-        k_field_near_culled<MULTI, false><<<gn, kBlock, 0, s>>>(m.geom, sg, pset, nsets, m.clusters, ncl,
-                                                                         m.order, m.n, px, py, pz, np, o,
-                                                                         o + ns * np, o + 2 * ns * np, o + 3 * ns * np);
+        by_waves(std::integral_constant<int, 1>());
     if (s != st) (void)hipEventRecord(side->join, s);
 }
 
@@ -1587,7 +1632,7 @@ hipError_t field_passes(hipStream_t st, int policy, const FieldMesh& m, bool mix
             // joins and combines of earlier chunks), not the wait for the near pass
             if (far_end && p0 + np >= npts) (void)hipEventRecord(far_end, st);
             if (culled) join_side(st, side);
-            k_field_combine<<<gc, kBlock, 0, st>>>(ws, (int)ns, np, phi + p0, ex + p0, ey + p0, ez + p0);
+            k_field_combine<<<dim3(gc, 4), kBlock, 0, st>>>(ws, (int)ns, np, phi + p0, ex + p0, ey + p0, ez + p0);
         }
     } else {
         const unsigned gx = nblocks(npts);
@@ -1622,7 +1667,7 @@ hipError_t field_passes(hipStream_t st, int policy, const FieldMesh& m, bool mix
                                                                 o2, o3, stride);
         }
         if (culled) join_side(st, side);
-        if (p.partials > 0) k_field_combine<<<gx, kBlock, 0, st>>>(ws, (int)ns, npts, phi, ex, ey, ez);
+        if (p.partials > 0) k_field_combine<<<dim3(gx, 4), kBlock, 0, st>>>(ws, (int)ns, npts, phi, ex, ey, ez);
     }
     return hipSuccess;
 }
@@ -1774,9 +1819,10 @@ hipError_t assemble_kernels(hipStream_t st, int policy, bool field, const double
         sp = (n + per2 - 1) / per2;
         grid = dim3(gx, (unsigned)sp);
         const int64_t ncl = (n + KEM_CLUSTER - 1) / KEM_CLUSTER;
+        const unsigned gnear = (unsigned)((n + 63) / 64);
         if (field) {
             k_assemble_far<true><<<grid, kBlock, 0, st>>>(geom, nodes, targets, n, per2, A64, A32);
-            k_assemble_near<true><<<gx, kBlock, 0, st>>>(geom, targets, clusters, ncl, order, n, A64, A32);
+            k_assemble_near<true><<<gnear, 64 * kAsmNearWaves, 0, st>>>(geom, targets, clusters, ncl, order, n, A64, A32);
         } else {
             // kAsmTargets targets per lane: fewer row blocks, more column splits
             constexpr int TT = kAsmTargets;
@@ -1789,7 +1835,7 @@ hipError_t assemble_kernels(hipStream_t st, int policy, bool field, const double
             k_asm_nodes<<<nblocks(n * KEM_NODE_SLOTS), kBlock, 0, st>>>(geom, nodes, n, anodes);
             k_assemble_far_pot<TT><<<dim3(gx2, (unsigned)sp2), kBlock, 0, st>>>(geom, nodes, anodes, targets, n, per3,
                                                                               A64, A32);
-            k_assemble_near<false><<<gx, kBlock, 0, st>>>(geom, targets, clusters, ncl, order, n, A64, A32);
+            k_assemble_near<false><<<gnear, 64 * kAsmNearWaves, 0, st>>>(geom, targets, clusters, ncl, order, n, A64, A32);
         }
         return hipGetLastError();
     }

@@ -1,0 +1,49 @@
+"""The culled near pass at the sizes where it changes the number of wavefronts that share a group of 64
+points (16 up to 512 groups, 4 up to 4,096, 1 above), over triangles, planar elements with wires, and a mesh
+smaller than a cluster: fields against the oracle, at points close to the surfaces (closed forms) and away."""
+import numpy as np
+import pytest
+
+from kassiopeia_amd import geometry as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from kassiopeia_amd import kemfield as K
+
+    c = K.Context(0)
+    c.set_integrator("numeric")
+    yield c
+    c.close()
+
+
+def meshes(name):
+    if name == "triangles":
+        return G.cube_mesh(2)
+    if name == "one":
+        return G.cube_mesh(1).subset([0])
+    wire = G.line_records([[-0.2, -0.2, 0.7]], [[0.3, 0.2, 0.8]], 2e-3)
+    line = G.Mesh(np.full(1, G.LINESEGMENT, np.int32), wire, np.zeros(1, np.int32), np.zeros(1), np.zeros(1),
+                  np.zeros(1, np.int32))
+    return G.concat(G.cube_rect_mesh(2), G.cube_mesh(1, edge=0.5), line)
+
+
+@pytest.mark.parametrize("name,npts", [("one", 1), ("one", 65), ("triangles", 64), ("triangles", 32768),
+                                       ("triangles", 32769), ("triangles", 262145), ("mixed", 63),
+                                       ("mixed", 32769)])
+def test_near_pass_wavefronts(ctx, oracle, name, npts):
+    from kassiopeia_amd import kemfield as K
+
+    m = meshes(name)
+    cont = K.KSurfaceContainer(ctx, m)
+    sigma = np.random.default_rng(npts).normal(size=m.n) * 1e-9
+    pts = G.points_shell(npts, 0.87, 1.6, npts)
+    pts[0] = [0.5, 0.13, 0.07]  # in the plane of a face
+    E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma).ElectricFieldAndPotential(pts)
+    phr, Er = oracle.field(m.shapes, m.recs, sigma, pts)
+    # FP64 sums of a few hundred terms in another order: far inside the 1e-12 that the field tests hold
+    assert np.abs(phi - phr).max() <= 1e-12 * np.abs(phr).max()
+    assert np.linalg.norm(E - Er, axis=1).max() <= 1e-12 * np.linalg.norm(Er, axis=1).max()
+    cont.close()
