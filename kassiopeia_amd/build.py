@@ -25,6 +25,7 @@ COMMON = ["-O3", "-fPIC", "-std=c++17", "-Wall", f"--offload-arch={ARCH}", "-mun
 SOURCES = [
     ("kem_kernels.hip", True),
     ("kem_sort.hip", True),
+    ("kem_tree.hip", True),
     ("kem_batch.hip", True),
     ("kem_adjoint.hip", True),
     ("kem_zh.hip", True),

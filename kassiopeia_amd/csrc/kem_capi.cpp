@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -109,6 +110,7 @@ struct kem_mesh {
     float* far6 = nullptr;       // mixed far field: 6-point records in cluster order
     float* far3 = nullptr;       // 3-point records in cluster order
     double* far6_cl = nullptr;   // and the clusters' 6- and 3-point reach
+    double* tree = nullptr;      // hierarchical far field: runs of elements (meshes without axisymmetric shapes)
     std::vector<int32_t> shape, bc;
     std::vector<double> value, flux;
     bool has_neumann = false;
@@ -301,7 +303,7 @@ struct DVec {
     ~DVec() { dfree(p); }
 };
 
-// point counts from which field evaluation visits points in Morton order
+// point counts from which field evaluation visits points along a space-filling curve
 constexpr int64_t kSortMinPoints = 4096;
 
 // Workspace sizes of one field evaluation with `range` elements per XCD range
@@ -313,7 +315,9 @@ WsNeed field_ws_need(const kem_ctx* c, const kem_mesh* m, const kem::FieldMesh& 
                      int64_t npts, bool mixed, int64_t range)
 {
     WsNeed n;
-    n.ws = kem::field_workspace_doubles(c->policy, fm, mixed, c->mixed_fp64_ratio, multi, nsets, npts, range);
+    const kem::TreePlan tp = kem::plan_tree(c->policy, fm, mixed, c->mixed_fp64_ratio, multi, npts);
+    n.ws = tp.use ? tp.doubles()
+                  : kem::field_workspace_doubles(c->policy, fm, mixed, c->mixed_fp64_ratio, multi, nsets, npts, range);
     n.gsig = m->gstart ? nsets * m->nm : 0;
     if (npts >= kSortMinPoints && npts <= INT32_MAX) n.sort = kem::sort_workspace_bytes(npts);
     return n;
@@ -586,14 +590,22 @@ int mesh_build(kem_ctx* c, int64_t n, const int64_t* gs, int64_t nm, const int32
         const int64_t f = gs ? gs[i] : i;
         kem::prep_target(shape[f], data + 11 * f, m->bc[i], m->flux[i], t.data() + (size_t)i * KT_STRIDE);
     }
-    for (int64_t i = 0; i < nm; i++) {
-        if (kem::prep_element(shape[i], data + 11 * i, g.data() + (size_t)i * KG_STRIDE,
-                              nd.data() + (size_t)i * KEM_NODE_STRIDE) != 0) {
-            delete m;
-            return fail(c, KEM_E_GEOM, "mesh: degenerate or non-finite element " + std::to_string(i));
+    std::atomic<int64_t> bad{nm};  // the first element that cannot be prepared
+    kem::in_parts(nm, 2048, [&](int64_t begin, int64_t end) {
+        for (int64_t i = begin; i < end; i++) {
+            if (kem::prep_element(shape[i], data + 11 * i, g.data() + (size_t)i * KG_STRIDE,
+                                  nd.data() + (size_t)i * KEM_NODE_STRIDE) != 0) {
+                for (int64_t b = bad; i < b && !bad.compare_exchange_weak(b, i);) {
+                }
+                return;
+            }
+            kem::prep_nodes32(g.data() + (size_t)i * KG_STRIDE, nd.data() + (size_t)i * KEM_NODE_STRIDE,
+                              nd32.data() + (size_t)i * KEM_NODE32_STRIDE);
         }
-        kem::prep_nodes32(g.data() + (size_t)i * KG_STRIDE, nd.data() + (size_t)i * KEM_NODE_STRIDE,
-                          nd32.data() + (size_t)i * KEM_NODE32_STRIDE);
+    });
+    if (bad < nm) {
+        delete m;
+        return fail(c, KEM_E_GEOM, "mesh: degenerate or non-finite element " + std::to_string(bad));
     }
     std::vector<int32_t> order((size_t)nm);
     std::vector<double> clusters((size_t)(4 * ((nm + KEM_CLUSTER - 1) / KEM_CLUSTER)));
@@ -602,6 +614,13 @@ int mesh_build(kem_ctx* c, int64_t n, const int64_t* gs, int64_t nm, const int32
     std::vector<double> far6_cl(clusters.size() / 4 * KEM_FAR_CL_STRIDE);
     kem::build_far6(nm, g.data(), nd32.data(), order.data(), clusters.data(), far6.data(), far3.data(),
                     far6_cl.data());
+    std::vector<double> tree;
+    if (std::none_of(shape, shape + nm, [](int32_t t) { return t == KEM_CONICSECTION || t == KEM_RING; })) {
+        kem::TreeLevels tl;
+        kem::tree_levels(nm, tl);
+        tree.resize((size_t)(tl.first[tl.levels - 1] + tl.count[tl.levels - 1]) * KEM_TREE_STRIDE);
+        kem::build_tree(nm, g.data(), order.data(), tl, tree.data());
+    }
     std::vector<double> recs((size_t)nm * KEM_REC, 0.);
     for (int64_t i = 0; i < nm; i++)
         for (int k = 0; k < 11; k++) recs[(size_t)i * KEM_REC + k] = data[11 * i + k];
@@ -637,6 +656,9 @@ int mesh_build(kem_ctx* c, int64_t n, const int64_t* gs, int64_t nm, const int32
     if (e == hipSuccess) e = dalloc(&m->far6_cl, (int64_t)far6_cl.size());
     if (e == hipSuccess)
         e = hipMemcpy(m->far6_cl, far6_cl.data(), sizeof(double) * far6_cl.size(), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = dalloc(&m->tree, (int64_t)tree.size());
+    if (e == hipSuccess && m->tree)
+        e = hipMemcpy(m->tree, tree.data(), sizeof(double) * tree.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = dalloc(&m->nodes, (int64_t)nd.size());
     if (e == hipSuccess) e = dalloc(&m->targets, (int64_t)t.size());
     if (e == hipSuccess) e = dalloc(&m->nodes32, (int64_t)nd32.size());
@@ -694,6 +716,7 @@ void kem_mesh_destroy(kem_mesh* m)
     dfree(m->far6);
     dfree(m->far3);
     dfree(m->far6_cl);
+    dfree(m->tree);
     dfree(m->recs);
     dfree(m->rule);
     dfree(m->gstart);
@@ -758,6 +781,7 @@ void field_mesh(const kem_mesh* m, kem::FieldMesh& f)
     f.far6 = m->far6;
     f.far3 = m->far3;
     f.far6_cl = m->far6_cl;
+    f.tree = m->tree;
     f.triangles = m->all_triangles;
     f.axisym = m->has_axisym;
 }
@@ -786,7 +810,7 @@ int field_eval(kem_ctx* c, const kem_mesh* m, const double* sigma, const int32_t
     hipEvent_t t0, t1;
     timing_pair(c, &t0, &t1);
     if (need.sort) {
-        // visit the points in Morton order so the lanes of a wavefront share quadrature rules
+        // visit the points along a space-filling curve so the lanes of a wavefront share quadrature rules
         KEM_CK(c, kem::launch_field_sorted(c->stream, c->policy, fm, mixed, c->mixed_fp64_ratio, sigma, pset, nsets,
                                            x, y, z, npts, phi, ex, ey, ez, w.sort, w.sort_bytes, w.ws, w.ws_doubles,
                                            range, t0, t1, ss));

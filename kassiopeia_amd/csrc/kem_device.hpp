@@ -18,6 +18,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cstdint>
+
 #include "kem_layout.h"
 
 namespace kem {
@@ -81,10 +83,12 @@ __constant__ const double kLogSeries[12] = {0.15631534707431224, 0.0749163946067
 __constant__ const double kAtanSeries[9] = {-0.03956743974276833, 0.05716019885233984, -0.0665491123778113,
                                             0.07691817726923288, -0.09090897022088731, 0.11111110943517653,
                                             -0.14285714284545636, 0.19999999999996856, -0.3333333333333333};
-__device__ __forceinline__ const double* opaque(const double* p)
+typedef const __attribute__((address_space(4))) double* ScalarPtr;  // read-only data, loaded through scalar registers
+__device__ __forceinline__ ScalarPtr opaque(const double* p)
 {
-    asm volatile("" : "+s"(p));
-    return p;
+    ScalarPtr q = (ScalarPtr)(uintptr_t)p;
+    asm volatile("" : "+s"(q));
+    return q;
 }
 
 // sqrt(a), a >= 0, to about an ulp: a * rsq(a) and one correction of its residual
@@ -114,7 +118,7 @@ __device__ __forceinline__ double log_quot(double a, double b)
     const double m = __builtin_ldexp(a, -k);
     const double s = quot_acc(m - b, m + b);
     const double z = s * s;
-    const double* c = opaque(kLogSeries);
+    const ScalarPtr c = opaque(kLogSeries);
     double q = c[0];
 #pragma unroll
     for (int i = 1; i < 11; i++) q = __builtin_fma(q, z, c[i]);
@@ -135,7 +139,7 @@ __device__ __forceinline__ double angle_acc(double y, double x)
     const double den = __builtin_fma(lo, c, hi);
     const double t = quot_acc(__builtin_fma(-hi, c, lo), den == 0. ? 1. : den);
     const double z = t * t;
-    const double* p = opaque(kAtanSeries);
+    const ScalarPtr p = opaque(kAtanSeries);
     double q = p[0];
 #pragma unroll
     for (int i = 1; i < 9; i++) q = __builtin_fma(q, z, p[i]);
@@ -641,6 +645,51 @@ __device__ __forceinline__ void kahan_add(double v, double sj, double& s, double
     const double t = s + y;
     c = (t - s) - y;
     s = t;
+}
+
+// ---------------------------------------------------------------- wavefronts
+__device__ __forceinline__ double wave_min(double v)
+{
+    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
+    return v;
+}
+__device__ __forceinline__ double wave_max(double v)
+{
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    return v;
+}
+
+// A value every lane holds alike, moved to scalar registers so branches on it are uniform.
+__device__ __forceinline__ double uniform(double v)
+{
+    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+    return __hiloint2double(hi, lo);
+}
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// the double whose low and high words are the bits of lo and hi
+__device__ __forceinline__ double f2d(float lo, float hi)
+{
+    return __hiloint2double(__float_as_int(hi), __float_as_int(lo));
+}
+
+// weights of the degree-4 6-point rule's two orbits as the FP32 node table stores them
+constexpr float kW6a = (float)0.223381589678011, kW6b = (float)0.109951743655322;
+constexpr float kW3 = 1.f / 3.f;  // the degree-2 3-point rule (interior nodes)
+
+// one FP32 quadrature node at offset (ex, ey, ez) from the point, weight w (dev::cubature32)
+__device__ __forceinline__ void node32(float ex, float ey, float ez, float w, float& s0, float& s1, float& s2,
+                                       float& s3)
+{
+    const float ir = __builtin_amdgcn_rsqf(ex * ex + ey * ey + ez * ez);
+    const float wi = w * ir;
+    const float f = wi * ir * ir;
+    s0 += ex * f;
+    s1 += ey * f;
+    s2 += ez * f;
+    s3 += wi;
 }
 
 }  // namespace dev

@@ -6,6 +6,8 @@
 
 #include <cstdint>
 
+#include "kem_prep.h"
+
 namespace kem {
 
 // Device arrays of a mesh that the field passes read.
@@ -20,6 +22,7 @@ struct FieldMesh {
     const float* far6 = nullptr;       // 6-point far records in cluster order (kem::build_far6)
     const float* far3 = nullptr;       // 3-point far records in cluster order
     const double* far6_cl = nullptr;   // and the clusters' 6- and 3-point reach (KEM_FAR_CL_STRIDE)
+    const double* tree = nullptr;      // hierarchical far field: node records (kem::build_tree); null: flat passes
     bool triangles = false;            // holds nothing but triangles
     bool axisym = false;               // holds conic sections or rings (kernels with their integrators)
 };
@@ -53,6 +56,24 @@ struct FieldPlan {
 FieldPlan plan_field(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t nsets,
                      int64_t npts, int64_t range_elems, int64_t ws_doubles);
 
+// How launch_field evaluates far pairs hierarchically (kem_tree.hip; host arithmetic): expansions of moments
+// doubles at the start of ws, then the point groups' ranges, then partials doubles of partial sums, the latter two
+// for chunk points at a time.
+struct TreePlan {
+    bool use = false;
+    TreeLevels levels;
+    int per_lane = 1;      // points per lane
+    int slices = 1;        // blocks per group of 64 per_lane points, each with a slice of the partial sums
+    int64_t moments = 0, ranges = 0, partials = 0, chunk = 0;
+    int64_t doubles() const { return moments + ranges + partials; }
+};
+TreePlan plan_tree(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t npts);
+// Sums over all elements at npts points in curve order, in p.slices slices of the partial layout out (component c,
+// slice s, point i at (c * slices + s) * npts + i); moments: expand the charges into mom first.
+hipError_t launch_tree(hipStream_t st, const FieldMesh& m, const TreePlan& p, bool mixed, const double* sigma,
+                       const double* px, const double* py, const double* pz, int64_t npts, double* mom, double* ranges,
+                       double* out, bool moments);
+
 // phi/E at npts points (SoA) from the mesh's elements with charge densities sigma.  pset
 // (nullable): per-point index of the charge-density set, point i using
 // sigma[pset[i]*n + j], 0 <= pset[i] < nsets.  mixed selects the mixed-precision far field
@@ -73,7 +94,7 @@ hipError_t launch_field(hipStream_t st, int policy, const FieldMesh& m, bool mix
                         int64_t ws_doubles, int64_t range_elems, hipEvent_t far_begin = nullptr,
                         hipEvent_t far_end = nullptr, const SideStream* side = nullptr);
 
-// Same as launch_field with the points visited in Morton order (kem_sort.hip): sort keys,
+// Same as launch_field with the points visited along a space-filling curve (kem_sort.hip): sort keys,
 // gather (with the set indices), evaluate, scatter back.  sort_ws: sort_workspace_bytes(npts) bytes.
 size_t sort_workspace_bytes(int64_t npts);
 hipError_t launch_field_sorted(hipStream_t st, int policy, const FieldMesh& m, bool mixed, double fp64_ratio,
@@ -91,7 +112,7 @@ hipError_t launch_census(hipStream_t st, const double* geom, int64_t nelem, cons
                          const double* pz, int64_t npts, int mixed, double fp64_ratio, unsigned long long* counts);
 
 // path census of the mixed cluster far pass (single set) over points in visiting order
-// (10 counters, see k_census_far32c); launch_census_paths_sorted visits them in the Morton
+// (10 counters, see k_census_far32c); launch_census_paths_sorted visits them in the curve
 // order of a pass of npts >= 4096 points (sort_ws: sort_workspace_bytes(npts) bytes)
 hipError_t launch_census_paths(hipStream_t st, const FieldMesh& m, const double* px, const double* py,
                                const double* pz, int64_t npts, unsigned long long* counts);
@@ -104,7 +125,7 @@ hipError_t launch_pairs(hipStream_t st, int policy, const double* geom, const do
                         const int64_t* gstart = nullptr);
 
 // collocation matrix; with element clusters (centre, radius per KEM_CLUSTER elements in the
-// Morton order `order`) the numeric policy splits it into cubature and closed-form kernels, and
+// run order `order`) the numeric policy splits it into cubature and closed-form kernels, and
 // without Neumann rows (field = false) that split needs anodes, assemble_nodes_doubles(n)
 // doubles of workspace for the potential node table
 int64_t assemble_nodes_doubles(int64_t n);

@@ -205,20 +205,9 @@ __global__ __launch_bounds__(kBlock) void k_field_near(const double* __restrict_
     }
 }
 
-__device__ __forceinline__ double wave_min(double v)
-{
-    for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-    return v;
-}
-__device__ __forceinline__ double wave_max(double v)
-{
-    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
 // Near pass with cluster culling (numeric policy).  W wavefronts share 64 points and take every W-th element
 // of a cluster; each bounds the points by the sphere around their bounding box, and a cluster of KEM_CLUSTER
-// elements (Morton order) whose sphere of near distances cannot reach it is skipped as a whole.  The pairs
+// elements (a compact run) whose sphere of near distances cannot reach it is skipped as a whole.  The pairs
 // evaluated are exactly the near set (the same dist2 test as the far pass); culling only removes clusters
 // proven to contain none.  The W sums are added in order through LDS, so the result is one slice of the
 // partial-sum layout that k_field_combine adds, and may run beside the far pass.  Blocks stride over the point
@@ -248,8 +237,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(SHAPES =
     const double x = px[i], y = py[i], z = pz[i];
     const double* __restrict__ sg = MULTI ? sigma + pset[i] : sigma;  // element-major sets
     // bounding sphere of the wavefront's points
-    const double lx = wave_min(x), ly = wave_min(y), lz = wave_min(z);
-    const double hx = wave_max(x), hy = wave_max(y), hz = wave_max(z);
+    const double lx = dev::wave_min(x), ly = dev::wave_min(y), lz = dev::wave_min(z);
+    const double hx = dev::wave_max(x), hy = dev::wave_max(y), hz = dev::wave_max(z);
     const double wx = 0.5 * (lx + hx), wy = 0.5 * (ly + hy), wz = 0.5 * (lz + hz);
     const double wr = 0.5 * sqrt((hx - lx) * (hx - lx) + (hy - ly) * (hy - ly) + (hz - lz) * (hz - lz));
     double s0 = 0., s1 = 0., s2 = 0., s3 = 0.;
@@ -301,39 +290,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(SHAPES =
         out3[i] = s3;
     }
   }
-}
-
-// A value every lane holds alike, moved to scalar registers so branches on it are uniform.
-__device__ __forceinline__ double uniform(double v)
-{
-    const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
-    const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
-    return __hiloint2double(hi, lo);
-}
-
-typedef float v16f __attribute__((ext_vector_type(16)));
-
-// the double whose low and high words are the bits of lo and hi
-__device__ __forceinline__ double f2d(float lo, float hi)
-{
-    return __hiloint2double(__float_as_int(hi), __float_as_int(lo));
-}
-
-// weights of the degree-4 6-point rule's two orbits as the FP32 node table stores them
-constexpr float kW6a = (float)0.223381589678011, kW6b = (float)0.109951743655322;
-constexpr float kW3 = 1.f / 3.f;  // the degree-2 3-point rule (interior nodes)
-
-// one FP32 quadrature node at offset (ex, ey, ez) from the point, weight w (dev::cubature32)
-__device__ __forceinline__ void node32(float ex, float ey, float ez, float w, float& s0, float& s1, float& s2,
-                                       float& s3)
-{
-    const float ir = __builtin_amdgcn_rsqf(ex * ex + ey * ey + ez * ez);
-    const float wi = w * ir;
-    const float f = wi * ir * ir;
-    s0 += ex * f;
-    s1 += ey * f;
-    s2 += ez * f;
-    s3 += wi;
 }
 
 // Per-call element weights of the far pass, sets element-major (entry j*nsets + s for
@@ -392,11 +348,11 @@ __global__ __launch_bounds__(kBlock) void k_field_far32c(const double* __restric
     const double x = px[i], y = py[i], z = pz[i];
     const double* __restrict__ wl = MULTI ? wk + pset[i] : wk;  // element-major sets
     // bounding sphere of the wavefront's points, radius padded against rounding
-    const double lx = wave_min(x), ly = wave_min(y), lz = wave_min(z);
-    const double hx = wave_max(x), hy = wave_max(y), hz = wave_max(z);
-    const double wx = uniform(0.5 * (lx + hx)), wy = uniform(0.5 * (ly + hy)), wz = uniform(0.5 * (lz + hz));
+    const double lx = dev::wave_min(x), ly = dev::wave_min(y), lz = dev::wave_min(z);
+    const double hx = dev::wave_max(x), hy = dev::wave_max(y), hz = dev::wave_max(z);
+    const double wx = dev::uniform(0.5 * (lx + hx)), wy = dev::uniform(0.5 * (ly + hy)), wz = dev::uniform(0.5 * (lz + hz));
     const double wr =
-        uniform(0.5 * sqrt((hx - lx) * (hx - lx) + (hy - ly) * (hy - ly) + (hz - lz) * (hz - lz)) * (1. + 1e-9) +
+        dev::uniform(0.5 * sqrt((hx - lx) * (hx - lx) + (hy - ly) * (hy - ly) + (hz - lz) * (hz - lz)) * (1. + 1e-9) +
                 1e-12);
     const int64_t c0 = t.split * cl_per_split;
     int64_t c1 = c0 + cl_per_split;
@@ -418,12 +374,12 @@ __global__ __launch_bounds__(kBlock) void k_field_far32c(const double* __restric
             // degree-2 3-point rule (single-set passes: in the several-set kernel the branch
             // costs 3 % on the 4 M-point batches, which have no such clusters)
             for (int64_t k = c * KEM_CLUSTER; k < k1; k++) {
-                const v16f R = *reinterpret_cast<const v16f*>(far3 + k * KEM_FAR3_STRIDE);
+                const dev::v16f R = *reinterpret_cast<const dev::v16f*>(far3 + k * KEM_FAR3_STRIDE);
                 const double wj = wl[MULTI ? k * nsets : k];
                 float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-                node32(dx - R[0], dy - R[1], dz - R[2], kW3, s0, s1, s2, s3);
-                node32(dx - R[4], dy - R[5], dz - R[6], kW3, s0, s1, s2, s3);
-                node32(dx - R[8], dy - R[9], dz - R[10], kW3, s0, s1, s2, s3);
+                dev::node32(dx - R[0], dy - R[1], dz - R[2], dev::kW3, s0, s1, s2, s3);
+                dev::node32(dx - R[4], dy - R[5], dz - R[6], dev::kW3, s0, s1, s2, s3);
+                dev::node32(dx - R[8], dy - R[9], dz - R[10], dev::kW3, s0, s1, s2, s3);
                 a0 += (double)s0 * wj;
                 a1 += (double)s1 * wj;
                 a2 += (double)s2 * wj;
@@ -433,25 +389,25 @@ __global__ __launch_bounds__(kBlock) void k_field_far32c(const double* __restric
         }
         for (int64_t k = c * KEM_CLUSTER; k < k1; k++) {
             // the whole far record in two 16-dword loads: nodes 0-3, then nodes 4-5, centre, reach
-            const v16f* rv = reinterpret_cast<const v16f*>(far6 + k * KEM_FAR6_STRIDE);
-            const v16f A = rv[0], B = rv[1];
+            const dev::v16f* rv = reinterpret_cast<const dev::v16f*>(far6 + k * KEM_FAR6_STRIDE);
+            const dev::v16f A = rv[0], B = rv[1];
             const double wj = wl[MULTI ? k * nsets : k];
-            const double cx = f2d(B[8], B[9]), cy = f2d(B[10], B[11]), cz = f2d(B[12], B[13]);
+            const double cx = dev::f2d(B[8], B[9]), cy = dev::f2d(B[10], B[11]), cz = dev::f2d(B[12], B[13]);
             bool six = all6;
             if (!six) {
                 const double ux = wx - cx, uy = wy - cy, uz = wz - cz;
-                const double te = f2d(B[14], B[15]) + wr;
+                const double te = dev::f2d(B[14], B[15]) + wr;
                 six = ux * ux + uy * uy + uz * uz > te * te;
             }
             float s0, s1, s2, s3;
             if (six) {
                 s0 = s1 = s2 = s3 = 0.f;
-                node32(dx - A[0], dy - A[1], dz - A[2], kW6a, s0, s1, s2, s3);
-                node32(dx - A[4], dy - A[5], dz - A[6], kW6a, s0, s1, s2, s3);
-                node32(dx - A[8], dy - A[9], dz - A[10], kW6a, s0, s1, s2, s3);
-                node32(dx - A[12], dy - A[13], dz - A[14], kW6b, s0, s1, s2, s3);
-                node32(dx - B[0], dy - B[1], dz - B[2], kW6b, s0, s1, s2, s3);
-                node32(dx - B[4], dy - B[5], dz - B[6], kW6b, s0, s1, s2, s3);
+                dev::node32(dx - A[0], dy - A[1], dz - A[2], dev::kW6a, s0, s1, s2, s3);
+                dev::node32(dx - A[4], dy - A[5], dz - A[6], dev::kW6a, s0, s1, s2, s3);
+                dev::node32(dx - A[8], dy - A[9], dz - A[10], dev::kW6a, s0, s1, s2, s3);
+                dev::node32(dx - A[12], dy - A[13], dz - A[14], dev::kW6b, s0, s1, s2, s3);
+                dev::node32(dx - B[0], dy - B[1], dz - B[2], dev::kW6b, s0, s1, s2, s3);
+                dev::node32(dx - B[4], dy - B[5], dz - B[6], dev::kW6b, s0, s1, s2, s3);
             } else {
                 const int64_t j = order[k];
                 const double* g = geom + j * KG_STRIDE;
@@ -500,11 +456,11 @@ __global__ __launch_bounds__(kBlock) void k_census_far32c(const double* __restri
     const bool live = i < npts;
     if (!live) i = npts - 1;
     const double x = px[i], y = py[i], z = pz[i];
-    const double lx = wave_min(x), ly = wave_min(y), lz = wave_min(z);
-    const double hx = wave_max(x), hy = wave_max(y), hz = wave_max(z);
-    const double wx = uniform(0.5 * (lx + hx)), wy = uniform(0.5 * (ly + hy)), wz = uniform(0.5 * (lz + hz));
+    const double lx = dev::wave_min(x), ly = dev::wave_min(y), lz = dev::wave_min(z);
+    const double hx = dev::wave_max(x), hy = dev::wave_max(y), hz = dev::wave_max(z);
+    const double wx = dev::uniform(0.5 * (lx + hx)), wy = dev::uniform(0.5 * (ly + hy)), wz = dev::uniform(0.5 * (lz + hz));
     const double wr =
-        uniform(0.5 * sqrt((hx - lx) * (hx - lx) + (hy - ly) * (hy - ly) + (hz - lz) * (hz - lz)) * (1. + 1e-9) +
+        dev::uniform(0.5 * sqrt((hx - lx) * (hx - lx) + (hy - ly) * (hy - ly) + (hz - lz) * (hz - lz)) * (1. + 1e-9) +
                 1e-12);
     unsigned long long c[10] = {0};
     for (int64_t cc = 0; cc < ncl; cc++) {
@@ -521,12 +477,12 @@ __global__ __launch_bounds__(kBlock) void k_census_far32c(const double* __restri
             continue;
         }
         for (int64_t k = cc * KEM_CLUSTER; k < k1; k++) {
-            const v16f B = reinterpret_cast<const v16f*>(far6 + k * KEM_FAR6_STRIDE)[1];
+            const dev::v16f B = reinterpret_cast<const dev::v16f*>(far6 + k * KEM_FAR6_STRIDE)[1];
             bool six = all6;
             if (!six) {
-                const double cx = f2d(B[8], B[9]), cy = f2d(B[10], B[11]), cz = f2d(B[12], B[13]);
+                const double cx = dev::f2d(B[8], B[9]), cy = dev::f2d(B[10], B[11]), cz = dev::f2d(B[12], B[13]);
                 const double ux = wx - cx, uy = wy - cy, uz = wz - cz;
-                const double te = f2d(B[14], B[15]) + wr;
+                const double te = dev::f2d(B[14], B[15]) + wr;
                 six = ux * ux + uy * uy + uz * uz > te * te;
             }
             if (six) {
@@ -833,7 +789,7 @@ __global__ __launch_bounds__(kBlock) void k_asm_nodes(const double* __restrict__
     o[4] = q[3];
 }
 
-// Closed-form entries: targets in the Morton order of the element centres (order[k]), so a
+// Closed-form entries: targets in the order of the element runs (order[k]), so a
 // wavefront's targets are compact; each wavefront bounds its targets by a sphere and skips the
 // element clusters that cannot hold a near pair of any of them (the culling of
 // k_field_near_culled); the entries it finds are written in place (a few per target).  The kAsmNearWaves
@@ -858,8 +814,8 @@ __global__ __launch_bounds__(64 * kAsmNearWaves) void k_assemble_near(const doub
     const bool dirichlet = t[KT_BC] == 0.;
     const double f = t[KT_FLUX];
     const double diag = ((1. + f) / (1. - f)) / (2. * dev::kEps0);
-    const double lx = wave_min(cx), ly = wave_min(cy), lz = wave_min(cz);
-    const double hx = wave_max(cx), hy = wave_max(cy), hz = wave_max(cz);
+    const double lx = dev::wave_min(cx), ly = dev::wave_min(cy), lz = dev::wave_min(cz);
+    const double hx = dev::wave_max(cx), hy = dev::wave_max(cy), hz = dev::wave_max(cz);
     const double wx = 0.5 * (lx + hx), wy = 0.5 * (ly + hy), wz = 0.5 * (lz + hz);
     const double wr = 0.5 * sqrt((hx - lx) * (hx - lx) + (hy - ly) * (hy - ly) + (hz - lz) * (hz - lz));
     for (int64_t c = 0; c < ncl; c++) {
@@ -1727,6 +1683,27 @@ int64_t field_workspace_doubles(int policy, const FieldMesh& m, bool mixed, doub
     return partial + 2 * nsig;
 }
 
+namespace {
+// The hierarchical pass over points in curve order: expansions at the start of ws, then the point groups' ranges
+// and the partial sums of a chunk of points.
+hipError_t tree_field(hipStream_t st, const FieldMesh& m, const TreePlan& p, bool mixed, const double* sigma,
+                      const double* px, const double* py, const double* pz, int64_t npts, double* phi, double* ex,
+                      double* ey, double* ez, double* ws, hipEvent_t far_begin, hipEvent_t far_end)
+{
+    double* q = ws + p.moments + p.ranges;
+    if (far_begin) (void)hipEventRecord(far_begin, st);
+    for (int64_t p0 = 0; p0 < npts; p0 += p.chunk) {
+        const int64_t np = std::min(p.chunk, npts - p0);
+        const hipError_t e = launch_tree(st, m, p, mixed, sigma, px + p0, py + p0, pz + p0, np, ws, ws + p.moments, q,
+                                         p0 == 0);
+        if (e != hipSuccess) return e;
+        if (far_end && p0 + np >= npts) (void)hipEventRecord(far_end, st);
+        k_field_combine<<<dim3(nblocks(np), 4), kBlock, 0, st>>>(q, p.slices, np, phi + p0, ex + p0, ey + p0, ez + p0);
+    }
+    return hipSuccess;
+}
+}  // namespace
+
 hipError_t launch_field(hipStream_t st, int policy, const FieldMesh& m, bool mixed, double fp64_ratio,
                         const double* sigma, const int32_t* pset, int64_t nsets, const double* px, const double* py,
                         const double* pz, int64_t npts, double* phi, double* ex, double* ey, double* ez, double* ws,
@@ -1737,7 +1714,10 @@ hipError_t launch_field(hipStream_t st, int policy, const FieldMesh& m, bool mix
     if (nsets < 1 || !phi || !ex || !ey || !ez) return hipErrorInvalidValue;
     if (side && side->st && (!side->fork || !side->join)) return hipErrorInvalidValue;
     hipError_t e;
-    if (pset)
+    const TreePlan tp = plan_tree(policy, m, mixed, fp64_ratio, pset != nullptr, npts);
+    if (tp.use && tp.doubles() <= ws_doubles)
+        e = tree_field(st, m, tp, mixed, sigma, px, py, pz, npts, phi, ex, ey, ez, ws, far_begin, far_end);
+    else if (pset)
         e = field_passes<true>(st, policy, m, mixed, fp64_ratio, sigma, pset, nsets, px, py, pz, npts, phi, ex, ey,
                                ez, ws, ws_doubles, range_elems, far_begin, far_end, side);
     else

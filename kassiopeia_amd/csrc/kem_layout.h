@@ -77,7 +77,7 @@ enum kem_geom_field {
 #define KEM_NODE32_SLOTS 58
 #define KEM_NODE32_STRIDE (4 * KEM_NODE32_SLOTS)
 
-/* element clusters for the near pass: elements in Morton order of their centres, KEM_CLUSTER
+/* element clusters for the near pass: elements in compact runs (kem::build_clusters), KEM_CLUSTER
    per cluster; each cluster keeps (centre x, y, z, radius) with radius = max over its elements
    of |c_j - centre| + near distance of j, so a point farther than radius from the centre has no
    near pair in the cluster */
@@ -107,6 +107,16 @@ enum kem_geom_field {
    |c_j - centre| + KEM_FAR3_RATIO size_j over the cluster, infinite when it holds any other
    shape than triangles), 3 pad */
 #define KEM_FAR_CL_STRIDE 8
+
+/* hierarchical far field: runs of KEM_TREE_LEAF elements in cluster order, KEM_TREE_FAN of which make a run of
+   the next level, up to the first level of at most 64.  Node record (doubles): centre of the bounding box of
+   the elements' vertices, radius (largest vertex distance), near reach (largest |c_j - centre| + near distance),
+   1 / radius, 2 pad; levels one after the other, the lowest first. */
+#define KEM_TREE_LEAF 16
+#define KEM_TREE_FAN 4
+#define KEM_TREE_STRIDE 8
+#define KEM_TREE_LEVELS 13
+#define KEM_TREE_INDEX_BITS 27
 
 /* collocation target record (one per element): centre, unit normal, boundary type, flux */
 enum kem_target_field { KT_CX = 0, KT_CY, KT_CZ, KT_NX, KT_NY, KT_NZ, KT_BC, KT_FLUX, KT_STRIDE = 8 };

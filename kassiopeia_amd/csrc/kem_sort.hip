@@ -3,8 +3,10 @@
 // A wavefront evaluates one element against 64 points at a time and executes every
 // quadrature branch that any of its lanes needs.  Points in the caller's order are spatially
 // random, so a wavefront typically runs both the 12- and the 33-point loops (and the closed
-// form) for one element.  Sorting the points along a Morton (Z-order) curve of their bounding
-// box makes the 64 points of a wavefront neighbours, so they almost always share one regime.
+// form) for one element.  Sorting the points along a Hilbert curve of the cube around them makes the
+// 64 points of a wavefront neighbours, so they almost always share one regime, and close to each other, so
+// the hierarchical pass accepts more expansions for them.  (A Morton curve's jumps left groups of points up to
+// 8 times the usual size, whose wavefronts ran 20 times longer than the others.)
 // The results are gathered back to the caller's order; each point's value does not depend on
 // the ordering.
 #include <hip/hip_runtime.h>
@@ -62,30 +64,62 @@ __device__ __forceinline__ uint64_t spread3(uint64_t a)
     return v;
 }
 
-// 63-bit Morton key of each point in the box spanned by the block partials (points of several
-// charge-density sets sort together: the kernels read the sets element-major, so a wavefront
-// may mix sets)
-__global__ __launch_bounds__(kBlock) void k_morton(const double* __restrict__ x, const double* __restrict__ y,
-                                                   const double* __restrict__ z, int64_t n, const double* __restrict__ part, int nparts,
-                                                   uint64_t* __restrict__ key, int32_t* __restrict__ idx)
+// Hilbert key (kCurveBits bits per axis) of each point in the cube over the box spanned by the block
+// partials: J. Skilling, "Programming the Hilbert curve" (2004), axes to transposed index.  Points of several
+// charge-density sets sort together: the kernels read the sets element-major, so a wavefront may mix sets.
+constexpr int kCurveBits = 16;
+__global__ __launch_bounds__(kBlock) void k_curve(const double* __restrict__ x, const double* __restrict__ y,
+                                                  const double* __restrict__ z, int64_t n,
+                                                  const double* __restrict__ part, int nparts,
+                                                  uint64_t* __restrict__ key, int32_t* __restrict__ idx)
 {
+    // the box from the partials: thread t < nparts brings one of them
+    __shared__ double sh[6][kBoxParts];
+    for (int k = 0; k < 3; k++) {
+        const bool have = (int)threadIdx.x < nparts;
+        sh[k][threadIdx.x] = have ? part[threadIdx.x * 6 + k] : 1e300;
+        sh[3 + k][threadIdx.x] = have ? part[threadIdx.x * 6 + 3 + k] : -1e300;
+    }
+    __syncthreads();
+    for (int s = kBoxParts / 2; s > 0; s >>= 1) {
+        if ((int)threadIdx.x < s)
+            for (int k = 0; k < 3; k++) {
+                sh[k][threadIdx.x] = fmin(sh[k][threadIdx.x], sh[k][threadIdx.x + s]);
+                sh[3 + k][threadIdx.x] = fmax(sh[3 + k][threadIdx.x], sh[3 + k][threadIdx.x + s]);
+            }
+        __syncthreads();
+    }
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
-    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-    for (int b = 0; b < nparts; b++)
-        for (int k = 0; k < 3; k++) {
-            lo[k] = fmin(lo[k], part[b * 6 + k]);
-            hi[k] = fmax(hi[k], part[b * 6 + 3 + k]);
-        }
     const double v[3] = {x[i], y[i], z[i]};
-    uint64_t code = 0;
+    double span = 0.;
+    for (int k = 0; k < 3; k++) span = fmax(span, sh[3 + k][0] - sh[k][0]);
+    constexpr double kMost = (1 << kCurveBits) - 1;
+    uint32_t a[3];
     for (int k = 0; k < 3; k++) {
-        const double span = hi[k] - lo[k];
-        double q = span > 0. ? (v[k] - lo[k]) / span * 2097151.0 : 0.;
-        q = q < 0. ? 0. : (q > 2097151.0 ? 2097151.0 : q);
-        code |= spread3((uint64_t)q) << k;
+        double q = span > 0. ? (v[k] - sh[k][0]) / span * kMost : 0.;
+        q = q > 0. ? (q > kMost ? kMost : q) : 0.;
+        a[k] = (uint32_t)q;
     }
-    key[i] = code;
+    for (uint32_t q = 1u << (kCurveBits - 1); q > 1; q >>= 1) {
+        const uint32_t p = q - 1;
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            if (a[k] & q) {
+                a[0] ^= p;
+            } else {
+                const uint32_t t = (a[0] ^ a[k]) & p;
+                a[0] ^= t;
+                a[k] ^= t;
+            }
+        }
+    }
+    a[1] ^= a[0];
+    a[2] ^= a[1];
+    uint32_t t = 0;
+    for (uint32_t q = 1u << (kCurveBits - 1); q > 1; q >>= 1)
+        if (a[2] & q) t ^= q - 1;
+    key[i] = spread3(a[2] ^ t) | spread3(a[1] ^ t) << 1 | spread3(a[0] ^ t) << 2;
     idx[i] = (int32_t)i;
 }
 
@@ -172,8 +206,8 @@ hipError_t launch_field_sorted(hipStream_t st, int policy, const FieldMesh& m, b
     int nb = (int)((npts + kBlock - 1) / kBlock);
     if (nb > kBoxParts) nb = kBoxParts;
     k_bbox_part<<<nb, kBlock, 0, st>>>(px, py, pz, npts, box);
-    k_morton<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, box, nb, k0, i0);
-    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 63, st);
+    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, box, nb, k0, i0);
+    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 3 * kCurveBits, st);
     if (e != hipSuccess) return e;
     k_gather3<<<nblocks(npts), kBlock, 0, st>>>(i1, px, py, pz, pset, npts, sx, sy, sz, ss);
     e = launch_field(st, policy, m, mixed, fp64_ratio, sigma, pset ? ss : nullptr, nsets, sx, sy, sz, npts, o[0], o[1],
@@ -212,8 +246,8 @@ hipError_t launch_census_paths_sorted(hipStream_t st, const FieldMesh& m, const 
     int nb = (int)((npts + kBlock - 1) / kBlock);
     if (nb > kBoxParts) nb = kBoxParts;
     k_bbox_part<<<nb, kBlock, 0, st>>>(px, py, pz, npts, box);
-    k_morton<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, box, nb, k0, i0);
-    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 63, st);
+    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, box, nb, k0, i0);
+    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 3 * kCurveBits, st);
     if (e != hipSuccess) return e;
     k_gather3<<<nblocks(npts), kBlock, 0, st>>>(i1, px, py, pz, nullptr, npts, sx, sy, sz, ss);
     return launch_census_paths(st, m, sx, sy, sz, npts, counts);

@@ -1,0 +1,104 @@
+"""The hierarchical far field against the flat passes: fields at many points (hierarchical) and at batches of fewer than 4,096 of
+the same points (always flat), over meshes of triangles, of rectangles with wires and of symmetry groups, element counts
+that leave the last run partial, point counts around one and two points per lane and with ragged last groups, smooth
+densities and densities of random sign, and point sets that are hard to group: scattered clumps, one point many times,
+points far away, points that are not finite."""
+import numpy as np
+import pytest
+
+from kassiopeia_amd import geometry as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from kassiopeia_amd import kemfield as K
+
+    c = K.Context(0)
+    c.set_integrator("numeric")
+    yield c
+    c.close()
+
+
+def mesh_of(kind, n):
+    if kind == "triangles":
+        m = G.coax_mesh(nphi_in=24, nphi_out=48, nz=31, ncap_r=4, ncap_phi=33)
+        return m.subset(np.arange(min(n, m.n)))
+    if kind == "frame":
+        k = ((n - 40) / 6) ** 0.5
+        rect = G.cube_rect_mesh(int(k))
+        w = n - rect.n
+        x = np.linspace(-0.5, 0.5, w)
+        p0 = np.stack([x, np.full(w, -0.5), np.full(w, 0.8)], 1)
+        wires = G.line_records(p0, p0 + np.array([0.0, 1.0, 0.1]), 1e-4)
+        return G.concat(rect, G.Mesh(np.full(w, G.LINESEGMENT, np.int32), wires, np.zeros(w, np.int32), np.zeros(w),
+                                     np.zeros(w), np.zeros(w, np.int32)))
+    return G.mirror_groups(G.cube_mesh(round((n / 24) ** 0.5)), [0.0, 0.0, 1.5], [0.0, 0.0, 1.0])
+
+
+def points_of(kind, npts, seed):
+    if kind == "triangles":
+        return G.points_annulus(npts, 0.51, 0.99, 1.95, seed)
+    return G.points_shell(npts, 0.9, 2.5, seed)
+
+
+def flat(cont, sigma, pts, precision):
+    from kassiopeia_amd import kemfield as K
+
+    s = K.KIntegratingElectrostaticFieldSolver(cont, sigma, precision)
+    E, phi = zip(*[s.ElectricFieldAndPotential(pts[i:i + 4000]) for i in range(0, len(pts), 4000)])
+    return np.concatenate(E), np.concatenate(phi)
+
+
+@pytest.mark.parametrize("kind,n,npts,rough", [
+    ("triangles", 4007, 16001, False), ("triangles", 4007, 65536, True), ("triangles", 4007, 65537, True),
+    ("triangles", 3001, 65601, False), ("frame", 3219, 40001, True), ("frame", 3219, 131077, False),
+    ("groups", 4800, 33000, True)])
+def test_tree_against_flat(ctx, kind, n, npts, rough):
+    from kassiopeia_amd import kemfield as K
+
+    m = mesh_of(kind, n)
+    cont = K.KSurfaceContainer(ctx, m)
+    rng = np.random.default_rng(n + npts)
+    c = m.centroids()
+    sigma = 1e-9 * (rng.normal(size=m.n) if rough else 1.0 + 0.5 * np.sin(3.0 * c[:, 2] + c[:, 0]))
+    pts = points_of(kind, npts, npts)
+    some = np.unique(np.concatenate([[0, npts - 1], rng.integers(0, npts, 6000)]))
+    E0, p0 = flat(cont, sigma, pts[some], "fp64")
+    for precision, tol in (("fp64", 1e-13), ("mixed", 1e-6)):
+        E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, precision).ElectricFieldAndPotential(pts)
+        # FP64: expansions to 8e-14 of each run's field, before the decay of their coefficients; mixed: its bar
+        assert np.linalg.norm(E[some] - E0) <= tol * np.linalg.norm(E0), precision
+        assert np.linalg.norm(phi[some] - p0) <= tol * np.linalg.norm(p0), precision
+        assert np.abs(phi[some] - p0).max() <= 10 * tol * np.abs(p0).max(), precision
+    cont.close()
+
+
+def test_tree_hard_points(ctx):
+    from kassiopeia_amd import kemfield as K
+
+    m = mesh_of("triangles", 4007)
+    cont = K.KSurfaceContainer(ctx, m)
+    sigma = 1e-9 * np.random.default_rng(3).normal(size=m.n)
+    rng = np.random.default_rng(4)
+    clumps = rng.uniform(-2.0, 2.0, (40, 3))[rng.integers(0, 40, 30000)] + 1e-3 * rng.normal(size=(30000, 3))
+    sets = {"clumps": clumps, "one": np.tile([[0.7, 0.1, 0.2]], (20000, 1)),
+            "far": np.concatenate([clumps, 1e5 * rng.normal(size=(50, 3)), m.centroids()[:500]])}
+    for name, pts in sets.items():
+        E0, p0 = flat(cont, sigma, pts[::7], "fp64")
+        E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, "fp64").ElectricFieldAndPotential(pts)
+        assert np.linalg.norm(E[::7] - E0) <= 1e-13 * np.linalg.norm(E0), name
+        assert np.linalg.norm(phi[::7] - p0) <= 1e-13 * np.linalg.norm(p0), name
+    # points that are not finite give values that are not, and leave the others alone
+    pts = clumps.copy()
+    pts[[5, 77]] = np.nan
+    pts[[123, 20000], 1] = np.inf
+    bad = ~np.isfinite(pts).all(1)
+    E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, "fp64").ElectricFieldAndPotential(pts)
+    E0, p0 = flat(cont, sigma, clumps[::7], "fp64")
+    ok = ~bad[::7]
+    assert not np.isfinite(phi[np.isnan(pts).any(1)]).any()
+    assert np.linalg.norm(E[::7][ok] - E0[ok]) <= 1e-13 * np.linalg.norm(E0[ok])
+    assert np.linalg.norm(phi[::7][ok] - p0[ok]) <= 1e-13 * np.linalg.norm(p0[ok])
+    cont.close()
