@@ -31,7 +31,8 @@ def test_small_systems(ctx, n):
     for precision, restart in (("fp64", 0), ("fp64", 37), ("mixed", 0)):
         x, st, rc = A.solve(b, tolerance=1e-11, restart=restart, precision=precision, max_iterations=4000)
         assert rc == 0 and st.true_residual <= 2e-11, (precision, restart)
-        assert st.iterations <= n or restart
+        # a Krylov space has at most n dimensions; refinements and restarts each begin another
+        assert st.iterations <= n or precision == "mixed" or restart
         if not restart:  # 1e-11 on the residual times the conditioning of these meshes (below 1e3)
             assert np.linalg.norm(x - ref) <= 1e-7 * np.linalg.norm(ref), precision
     A.close()

@@ -45,3 +45,34 @@ def test_grid_equals_single_workgroup(coax12k):
     assert out[0][2] < 0.1
     r = np.abs(b - A.Multiply(out[0][0])).max() / np.abs(b).max()
     assert r < 0.1
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 256, 2048, 2049, 4097, 8191])
+def test_small_matches_host_sequence(n):
+    """The register kernel (up to 8,191 unknowns; 256, 512 and 1,024 threads, ragged last rows) against the same
+    corrections on the host: first argmax of |b - b_iter| (all residuals alike at first), the product and the sum of
+    each update fused as on the device."""
+    from kassiopeia_amd import kemfield as K
+
+    ctx = K.Context(0)
+    ctx.set_integrator("numeric")
+    m = G.coax_mesh(nphi_in=32, nphi_out=64, nz=60, ncap_r=4, ncap_phi=40).subset(np.arange(n))
+    m.bc_value[:] = 1.0
+    cont = K.KSurfaceContainer(ctx, m)
+    A = K.KBoundaryIntegralMatrix(cont)
+    steps = 40
+    x, st, rc = A.solve(cont.rhs(), method="robin_hood", tolerance=1e-300, check_interval=steps, max_iterations=1)
+    Ad = A.to_numpy()
+    xr, it, b = np.zeros(n), np.zeros(n), np.ones(n)
+    for _ in range(steps):
+        r = b - it
+        k = int(np.argmax(np.abs(r)))
+        c = r[k] / Ad[k, k]
+        xr[k] += c
+        it += Ad[:, k] * c
+    # the host rounds the product before the sum: 40 corrections of a few ulps each, on x of size one
+    assert st.sub_iterations == steps
+    assert np.abs(x - xr).max() <= 1e-13 * np.abs(xr).max()
+    A.close()
+    cont.close()
+    ctx.close()
