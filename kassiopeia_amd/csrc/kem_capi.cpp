@@ -27,6 +27,8 @@ constexpr double kMixedFp64RatioDefault = 0.0;
 // the inner tolerance of BF16-matrix solves: the BF16 product rounds its input vector to 8
 // significant bits, so an inner solve cannot reduce its true residual much below 2^-8
 constexpr double kBf16InnerTolerance = 1.0 / 256.0;
+// host-array calls of up to this size go through page-locked memory
+constexpr size_t kStageBytes = (size_t)16 << 20;
 // elements per XCD range of the large single-set far passes (kem::launch_field); 0 = no split
 constexpr int64_t kFarRangeDefault = 2560;
 
@@ -78,6 +80,11 @@ struct kem_ctx {
     double* scal = nullptr;  // small device scalars (dot products, Hessenberg column)
     int64_t scal_doubles = 0;
     FieldWs fws;  // workspace of eager field evaluations (grow-only)
+    // staging of host-array calls: device memory, and page-locked host memory for calls of up to kStageBytes (grow-only)
+    double* io = nullptr;
+    int64_t io_doubles = 0;
+    double* pin = nullptr;
+    int64_t pin_doubles = 0;
     double* acc4 = nullptr;  // one field's (phi, Ex, Ey, Ez) of a step-level sum over fields (grow-only)
     int64_t acc4_doubles = 0;
     // storage of destroyed matrices, kept for the next matrix of the same size: freeing and
@@ -380,6 +387,8 @@ void kem_ctx_destroy(kem_ctx* c)
     dfree(c->ws);
     dfree(c->scal);
     dfree(c->acc4);
+    dfree(c->io);
+    if (c->pin) (void)hipHostFree(c->pin);
     ws_release(c->fws);
     for (auto& b : c->store_cache) (void)hipFree(b.first);
     c->store_cache.clear();
@@ -1110,23 +1119,41 @@ int kem_field_eval(kem_ctx* c, const kem_mesh* m, const double* sigma, int64_t n
     if (!c || !m || !sigma || (npts > 0 && !P)) return KEM_E_ARG;
     if (npts <= 0) return KEM_OK;
     KEM_CK(c, enter(c));
-    std::vector<double> soa((size_t)npts * 3);
+    // sigma, x, y, z in one block of device memory, then phi, Ex, Ey, Ez; kept on the context, as is a page-locked
+    // block of host memory that small calls pass through in one copy each way (allocating, freeing and copying
+    // pageable memory took 120 us of a call of 64 points)
+    const int64_t in = m->n + 3 * npts, total = in + 4 * npts;
+    const bool staged = sizeof(double) * (size_t)total <= kStageBytes;
+    hipError_t e = hipSuccess;
+    if (c->io_doubles < total) {
+        dfree(c->io);
+        c->io_doubles = 0;
+        e = dalloc(&c->io, total);
+        if (e == hipSuccess) c->io_doubles = total;
+    }
+    if (e == hipSuccess && staged && c->pin_doubles < total) {
+        if (c->pin) (void)hipHostFree(c->pin);
+        c->pin = nullptr;
+        c->pin_doubles = 0;
+        e = hipHostMalloc((void**)&c->pin, sizeof(double) * (size_t)total, hipHostMallocDefault);
+        if (e == hipSuccess) c->pin_doubles = total;
+    }
+    if (e != hipSuccess) return fail(c, KEM_E_HIP, std::string("field_eval: ") + hipGetErrorString(e));
+    std::vector<double> pageable(staged ? 0 : (size_t)total);
+    double* h = staged ? c->pin : pageable.data();
+    std::memcpy(h, sigma, sizeof(double) * (size_t)m->n);
+    double* hx = h + m->n;
     for (int64_t i = 0; i < npts; i++)
-        for (int k = 0; k < 3; k++) soa[(size_t)k * npts + i] = P[3 * i + k];
-    double *dS = nullptr, *dP = nullptr, *dO = nullptr;
-    hipError_t e = dalloc(&dS, m->n);
-    if (e == hipSuccess) e = dalloc(&dP, 3 * npts);
-    if (e == hipSuccess) e = dalloc(&dO, 4 * npts);
-    if (e == hipSuccess) e = hipMemcpyAsync(dS, sigma, sizeof(double) * m->n, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(dP, soa.data(), sizeof(double) * 3 * npts, hipMemcpyHostToDevice, c->stream);
+        for (int k = 0; k < 3; k++) hx[(size_t)k * npts + i] = P[3 * i + k];
+    e = hipMemcpyAsync(c->io, h, sizeof(double) * (size_t)in, hipMemcpyHostToDevice, c->stream);
     int rc = KEM_OK;
     if (e == hipSuccess) {
-        rc = kem_field_eval_device(c, m, dS, npts, dP, dP + npts, dP + 2 * npts, precision, dO, dO + npts,
+        double *dP = c->io + m->n, *dO = c->io + in;
+        rc = kem_field_eval_device(c, m, c->io, npts, dP, dP + npts, dP + 2 * npts, precision, dO, dO + npts,
                                    dO + 2 * npts, dO + 3 * npts);
         if (rc == KEM_OK) {
-            std::vector<double> o((size_t)npts * 4);
-            e = hipMemcpyAsync(o.data(), dO, sizeof(double) * 4 * npts, hipMemcpyDeviceToHost, c->stream);
+            const double* o = h + in;
+            e = hipMemcpyAsync(h + in, dO, sizeof(double) * 4 * npts, hipMemcpyDeviceToHost, c->stream);
             if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
             if (e == hipSuccess) {
                 // device layout: phi, Ex, Ey, Ez planes of npts each
@@ -1136,11 +1163,10 @@ int kem_field_eval(kem_ctx* c, const kem_mesh* m, const double* sigma, int64_t n
                         for (int k = 0; k < 3; k++) E[3 * i + k] = o[(size_t)(k + 1) * npts + i];
                 }
             }
+        } else {
+            (void)hipStreamSynchronize(c->stream);  // the copy in still reads h
         }
     }
-    dfree(dS);
-    dfree(dP);
-    dfree(dO);
     if (rc != KEM_OK) return rc;
     if (e != hipSuccess) return fail(c, KEM_E_HIP, std::string("field_eval: ") + hipGetErrorString(e));
     return KEM_OK;

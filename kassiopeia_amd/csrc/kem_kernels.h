@@ -43,6 +43,7 @@ int64_t field_workspace_doubles(int policy, const FieldMesh& m, bool mixed, doub
 // How launch_field splits one evaluation (host arithmetic, no device access).
 struct FieldPlan {
     int kind = 0;          // far kernel: 0 FP64, 1 FP32 per pair, 2 FP32 over element clusters
+    bool small = false;    // one kernel over all pairs in FP64, ranges of a few elements
     bool xcd = false;      // 8 R element ranges, R per XCD, over chunks of points
     int64_t ranges = 1;    // element ranges of the far pass
     int64_t slices = 1;    // partial-sum slices: the ranges, and one for a culled near pass

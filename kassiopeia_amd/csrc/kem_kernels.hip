@@ -292,6 +292,52 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(SHAPES =
   }
 }
 
+// Small calls (plan_field): every pair of 64 points and the elements [j0, j0 + per) of a block of one wavefront, far
+// pairs by the FP64 rules and near ones by the closed forms, into the range's slice of the partial sums.  Such a
+// call is bound by how long one wavefront takes over its elements, not by the chip, so the elements are divided
+// into ranges of a few, the near pairs have no pass (and no second stream) of their own, and mixed precision, which
+// would save arithmetic that nothing waits for, takes the same kernel.
+template <int SHAPES>
+__global__ __launch_bounds__(64) void k_field_small(const double* __restrict__ geom, const double* __restrict__ nodes,
+                                                    const double* __restrict__ sigma, int64_t nelem, int64_t per,
+                                                    const double* __restrict__ px, const double* __restrict__ py,
+                                                    const double* __restrict__ pz, int64_t npts,
+                                                    double* __restrict__ out0, double* __restrict__ out1,
+                                                    double* __restrict__ out2, double* __restrict__ out3,
+                                                    int64_t out_stride)
+{
+    int64_t i = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    const bool live = i < npts;
+    if (!live) i = npts - 1;
+    const double x = px[i], y = py[i], z = pz[i];
+    const int64_t j0 = (int64_t)blockIdx.y * per, j1 = j0 + per < nelem ? j0 + per : nelem;
+    double s0 = 0., s1 = 0., s2 = 0., s3 = 0.;
+    double c0 = 0., c1 = 0., c2 = 0., c3 = 0.;
+    for (int64_t j = j0; j < j1; j++) {
+        const double* g = geom + j * KG_STRIDE;
+        const double r2 = dev::dist2(g, x, y, z);
+        F4 v;
+        if (dev::is_near2(g, r2, 0))
+            v = SHAPES == 0   ? dev::closed_form<3, true, true>(g, x, y, z)
+                : SHAPES == 1 ? dev::element_near<true>(g, (int)g[KG_TYPE], x, y, z)
+                              : dev::element_near_any(g, (int)g[KG_TYPE], x, y, z);
+        else
+            v = dev::element_far(g, nodes + j * KEM_NODE_STRIDE, (int)g[KG_TYPE], r2, x, y, z);
+        const double sj = sigma[j];
+        dev::kahan_add(v.x, sj, s0, c0);
+        dev::kahan_add(v.y, sj, s1, c1);
+        dev::kahan_add(v.z, sj, s2, c2);
+        dev::kahan_add(v.p, sj, s3, c3);
+    }
+    if (live) {
+        const int64_t o = (int64_t)blockIdx.y * out_stride + i;
+        out0[o] = s0;
+        out1[o] = s1;
+        out2[o] = s2;
+        out3[o] = s3;
+    }
+}
+
 // Per-call element weights of the far pass, sets element-major (entry j*nsets + s for
 // element j, set s; sigma is set-major, sigma[s*nelem + j]):
 //   wk[k*nsets + s] = prefactor * sigma of the k-th element in cluster order (order != null),
@@ -1770,7 +1816,32 @@ hipError_t field_passes(hipStream_t st, int policy, const FieldMesh& m, bool mix
     }
     const bool culled = culled_near(policy, m);
     const int64_t nr = p.ranges, ns = p.slices;
-    if (p.xcd) {
+    if (p.small) {
+        double *o0 = ex, *o1 = ey, *o2 = ez, *o3 = phi;
+        int64_t stride = 0;
+        if (p.partials > 0) {
+            o0 = ws;
+            o1 = ws + ns * npts;
+            o2 = ws + 2 * ns * npts;
+            o3 = ws + 3 * ns * npts;
+            stride = npts;
+        }
+        if (far_begin) (void)hipEventRecord(far_begin, st);
+        const dim3 grid((unsigned)((npts + 63) / 64), (unsigned)nr);
+        auto launch = [&](auto shapes) {
+            k_field_small<decltype(shapes)::value><<<grid, 64, 0, st>>>(m.geom, m.nodes, sg, nelem, p.per, px, py, pz,
+                                                                        npts, o0, o1, o2, o3, stride);
+        };
+        if (m.axisym)
+            launch(std::integral_constant<int, 2>());
+        else if (m.triangles)
+            launch(std::integral_constant<int, 0>());
+        else
+            launch(std::integral_constant<int, 1>());
+        if (far_end) (void)hipEventRecord(far_end, st);
+        if (p.partials > 0)
+            k_field_combine<<<dim3(nblocks(npts), 4), kBlock, 0, st>>>(ws, (int)ns, npts, phi, ex, ey, ez);
+    } else if (p.xcd) {
         // 8 R element ranges of at most range_elems elements, R per XCD; partial sums per
         // range (and of the near pass) over chunks of points
         if (far_begin) (void)hipEventRecord(far_begin, st);
@@ -1831,6 +1902,20 @@ hipError_t field_passes(hipStream_t st, int policy, const FieldMesh& m, bool mix
 }
 }  // namespace
 
+namespace {
+constexpr int64_t kSmallRange = 4;    // fewest elements of a range
+constexpr int64_t kSmallWaves = 8192;  // most wavefronts of a small call
+// Pairs up to which k_field_small is the faster way: FP64 as long as the passes do not fill the chip, mixed as long
+// as FP32 arithmetic is not what the time goes to.  Host-array calls, us with the passes / small: 192 elements x 64
+// points 238 / 50, 1,728 x 512 180 / 89, 4,800 x 1,500 474 / 357, 20,000 x 512 938 / 910 (FP64); 1,728 x 512 138 /
+// 89, 20,000 x 64 765 / 317, 4,800 x 512 207 / 184 with the passes after all (mixed).
+constexpr double kSmallPairsFp64 = 1e7, kSmallPairsMixed = 2e6;
+bool small_call(bool mixed, int64_t nelem, int64_t npts)
+{
+    return (double)nelem * (double)npts <= (mixed ? kSmallPairsMixed : kSmallPairsFp64);
+}
+}  // namespace
+
 FieldPlan plan_field(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t nsets,
                      int64_t npts, int64_t range_elems, int64_t ws_doubles)
 {
@@ -1840,6 +1925,20 @@ FieldPlan plan_field(int policy, const FieldMesh& m, bool mixed, double fp64_rat
     const bool clustered = policy == 0 && mixed && m.nodes32 && fp64_ratio == 0. && m.far6 && m.far3 &&
                            m.far6_cl && m.order;
     p.kind = clustered ? 2 : (policy == 0 && mixed && m.nodes32) ? 1 : 0;
+    if (!multi && culled_near(policy, m) && small_call(mixed, nelem, npts)) {
+        p.small = true;
+        p.kind = 0;
+        if (ws_doubles < 0)
+            ws_doubles = field_workspace_doubles(policy, m, mixed, fp64_ratio, multi, nsets, npts, range_elems);
+        const int64_t groups = (npts + 63) / 64;
+        int64_t r = std::max<int64_t>(1, std::min((nelem + kSmallRange - 1) / kSmallRange, kSmallWaves / groups));
+        while (r > 1 && 4 * r * npts > ws_doubles) r--;
+        p.per = (nelem + r - 1) / r;
+        p.ranges = p.slices = (nelem + p.per - 1) / p.per;
+        p.chunk = npts;
+        p.partials = p.slices > 1 ? 4 * p.slices * npts : 0;
+        return p;
+    }
     const int64_t nsig = (nsets * nelem + 31) / 32 * 32;
     p.weights = (clustered ? nsig : 0) + (multi ? nsig : 0);
     if (ws_doubles < 0)

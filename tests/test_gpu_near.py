@@ -47,3 +47,23 @@ def test_near_pass_wavefronts(ctx, oracle, name, npts):
     assert np.abs(phi - phr).max() <= 1e-12 * np.abs(phr).max()
     assert np.linalg.norm(E - Er, axis=1).max() <= 1e-12 * np.linalg.norm(Er, axis=1).max()
     cont.close()
+
+
+@pytest.mark.parametrize("precision,n,npts", [("fp64", 1, 1), ("fp64", 5, 63), ("fp64", 47, 65), ("fp64", 48, 4097),
+                                              ("mixed", 48, 130), ("mixed", 48, 41666), ("mixed", 48, 41667),
+                                              ("fp64", 48, 208333), ("fp64", 48, 208334)])
+def test_small_calls(ctx, oracle, precision, n, npts):
+    """Both sides of the sizes up to which one kernel takes all pairs (1e7 pairs FP64, 2e6 mixed), ragged ranges and
+    groups, a single element and point."""
+    from kassiopeia_amd import kemfield as K
+
+    m = meshes("triangles").subset(np.arange(n))
+    cont = K.KSurfaceContainer(ctx, m)
+    sigma = 1e-9 * np.random.default_rng(n).uniform(0.5, 1.5, size=m.n)
+    pts = G.points_shell(npts, 0.87, 1.6, npts)
+    E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, precision).ElectricFieldAndPotential(pts)
+    phr, Er = oracle.field(m.shapes, m.recs, sigma, pts)
+    tol = 1e-12 if precision == "fp64" or n * npts <= 2e6 else 1e-6  # the mixed bar where FP32 pairs are taken
+    assert np.abs(phi - phr).max() <= tol * np.abs(phr).max()
+    assert np.linalg.norm(E - Er, axis=1).max() <= tol * np.linalg.norm(Er, axis=1).max()
+    cont.close()
