@@ -264,52 +264,194 @@ __device__ __forceinline__ double wave_sum(double v)
 }
 
 // ------------------------------------------------------------------ field term
-// partV[s][j][10] = (sum_k g_k G_kj, sum_k g_k sigma_j dG_kj/dv) over the points of split s
-template <bool NEAR>
-__global__ __launch_bounds__(kBlock) void k_vjp_field(const double* __restrict__ geom,
-                                                      const double* __restrict__ sigma,
-                                                      const double* __restrict__ rule, int64_t n,
-                                                      const double* __restrict__ pts, const double* __restrict__ gk,
-                                                      int64_t npts, int64_t per_split, double* __restrict__ partV)
+// Far pairs of the field term: partV[s][j][10] = (sum_k g_k G_kj, sum_k g_k sigma_j dG_kj/dv) over the points of
+// split s.  Lane = element; the four wavefronts of a block share 64 elements and take 64 points of the split at a
+// time.  The sums over points are linear in the nodes' own sums A_q = sum_k g_k / R_kq and B_q = sum_k g_k r_kq /
+// R_kq^3, so a wavefront runs over the points inside and over the nodes outside: a pair costs 22 operations a
+// node, and the node's position and the nine derivatives are formed once per 64 points.  Bound by FP64 issue: 1.24 ms
+// for 5,000 elements and 10,000 points, 2.36 ms with the nodes inside (36 operations a node and each lane its own
+// rule).  All lanes take the rule with the most nodes that any of them needs for a point, as in the assembly; the
+// points are put in LDS by rule.  Near pairs are left out, and near[group * splits + s] says whether there were any,
+// so that k_vjp_field_near passes over the others (28 us where there are none, 230 us with its own test of each pair).
+constexpr int kVjpWaves = 4;
+__global__ __launch_bounds__(64 * kVjpWaves) void k_vjp_field_far(const double* __restrict__ geom,
+                                                                  const double* __restrict__ sigma,
+                                                                  const double* __restrict__ rule, int64_t n,
+                                                                  const double* __restrict__ pts,
+                                                                  const double* __restrict__ gk, int64_t npts,
+                                                                  int64_t per_split, double* __restrict__ partV,
+                                                                  int* __restrict__ near)
 {
-    const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (j >= n) return;
+    __shared__ double4 lp[kVjpWaves][64];
+    __shared__ int lk[kVjpWaves][64];
+    __shared__ double part[kVjpWaves - 1][10][64];
+    __shared__ int s_near[kVjpWaves];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int64_t j = (int64_t)blockIdx.x * 64 + lane;
+    const bool live = j < n;
+    if (!live) j = n - 1;
     const double* g = geom + j * KG_STRIDE;
     Elem E;
     load_elem(g, sigma[j], E);
+    const double cx = g[KG_CX], cy = g[KG_CY], cz = g[KG_CZ];
+    const double near2 = g[KG_NEAR2], ref7 = g[KG_REF7_2], ref12 = g[KG_REF12_2];
+    const bool act = live && E.tri;
+    const int64_t k0 = (int64_t)blockIdx.y * per_split;
+    const int64_t k1 = std::min<int64_t>(npts, k0 + per_split);
+    double4* P = lp[wv];
+    int* K = lk[wv];
+    double S = 0., F[3][3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
+    bool any_near = false;
+    for (int64_t c0 = k0 + 64 * wv; c0 < k1; c0 += 64 * kVjpWaves) {
+        const int cnt = (int)std::min<int64_t>(64, k1 - c0);
+        const int64_t kl = c0 + std::min(lane, cnt - 1);
+        const double4 mine{pts[3 * kl], pts[3 * kl + 1], pts[3 * kl + 2], gk[kl]};
+        // the rule that the wavefront takes for each point (lane k keeps point k's), and the lane's near pairs
+        int code = 0;
+        unsigned long long mask = 0;
+        for (int k = 0; k < cnt; k++) {
+            auto lane_of = [k](double v) {
+                return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                                        __builtin_amdgcn_readlane(__double2loint(v), k));
+            };
+            // dist2's operations, so the same pairs are near as in the forward pass
+            const double dx = cx - lane_of(mine.x), dy = cy - lane_of(mine.y), dz = cz - lane_of(mine.z);
+            const double r2 = __builtin_fma(dz, dz, __builtin_fma(dy, dy, dx * dx));
+            const bool isnear = !(r2 > near2), far = act && !isnear;
+            if (isnear) mask |= 1ull << k;
+            const int c = __builtin_amdgcn_ballot_w64(far && !(r2 > ref12)) != 0  ? 3
+                          : __builtin_amdgcn_ballot_w64(far && !(r2 > ref7)) != 0 ? 2
+                          : __builtin_amdgcn_ballot_w64(far) != 0                 ? 1
+                                                                                  : 0;
+            if (lane == k) code = c;
+        }
+        const bool some = __builtin_amdgcn_ballot_w64(act && mask != 0) != 0;
+        any_near = any_near || some;
+        __builtin_amdgcn_wave_barrier();
+        int at = 0;
+        int start[4];
+#pragma unroll
+        for (int c = 1; c <= 3; c++) {
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(code == c);
+            start[c - 1] = at;
+            if (code == c) {
+                const int to = at + __builtin_popcountll(m & ((1ull << lane) - 1));
+                P[to] = mine;
+                K[to] = lane;
+            }
+            at += __builtin_popcountll(m);
+        }
+        start[3] = at;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+        for (int c = 0; c < 3; c++) {
+            const int i0 = c == 0 ? start[0] : c == 1 ? start[1] : start[2];
+            const int i1 = c == 0 ? start[1] : c == 1 ? start[2] : start[3];
+            if (i0 == i1) continue;
+            const int nq = c == 0 ? 7 : c == 1 ? 12 : 33;
+            const double* t = rule + 4 * rule_slot(nq);
+            // two nodes at a time share the points' reads; the last of an odd rule runs beside itself with weight 0
+#pragma unroll 1
+            for (int q = 0; q < nq; q += 2) {
+                double bq[2][3], w[2], x[2], y[2], z[2], A[2], Bx[2], By[2], Bz[2];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const double* r = t + 4 * std::min(q + h, nq - 1);
+                    for (int m = 0; m < 3; m++) bq[h][m] = r[m];
+                    w[h] = q + h < nq ? r[3] : 0.;
+                    x[h] = bq[h][0] * E.v[0][0] + bq[h][1] * E.v[1][0] + bq[h][2] * E.v[2][0];
+                    y[h] = bq[h][0] * E.v[0][1] + bq[h][1] * E.v[1][1] + bq[h][2] * E.v[2][1];
+                    z[h] = bq[h][0] * E.v[0][2] + bq[h][1] * E.v[1][2] + bq[h][2] * E.v[2][2];
+                    A[h] = Bx[h] = By[h] = Bz[h] = 0.;
+                }
+                for (int i = i0; i < i1; i++) {
+                    const double4 p = P[i];
+                    const bool skip = some && ((mask >> K[i]) & 1);
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const double rx = p.x - x[h], ry = p.y - y[h], rz = p.z - z[h];
+                        double ir = dev::rsqrt_acc(rx * rx + ry * ry + rz * rz);
+                        if (skip) ir = 0.;
+                        const double a = p.w * ir;
+                        const double f = a * ir * ir;
+                        A[h] += a;
+                        Bx[h] = __builtin_fma(f, rx, Bx[h]);
+                        By[h] = __builtin_fma(f, ry, By[h]);
+                        Bz[h] = __builtin_fma(f, rz, Bz[h]);
+                    }
+                }
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    S = __builtin_fma(w[h], A[h], S);
+                    for (int m = 0; m < 3; m++) {
+                        const double wb = w[h] * bq[h][m];
+                        F[m][0] = __builtin_fma(wb, Bx[h], F[m][0]);
+                        F[m][1] = __builtin_fma(wb, By[h], F[m][1]);
+                        F[m][2] = __builtin_fma(wb, Bz[h], F[m][2]);
+                    }
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+    // the wavefronts' sums in order
+    if (lane == 0) s_near[wv] = any_near;
+    if (wv > 0) {
+        part[wv - 1][0][lane] = S;
+        for (int c = 0; c < 9; c++) part[wv - 1][1 + c][lane] = F[c / 3][c % 3];
+    }
+    __syncthreads();
+    if (wv > 0) return;
+    for (int k = 0; k < kVjpWaves - 1; k++) {
+        S += part[k][0][lane];
+        for (int c = 0; c < 9; c++) F[c / 3][c % 3] += part[k][1 + c][lane];
+    }
+    if (lane == 0) near[(int64_t)blockIdx.x * gridDim.y + blockIdx.y] = s_near[0] | s_near[1] | s_near[2] | s_near[3];
+    if (!live) return;
+    double* out = partV + ((int64_t)blockIdx.y * n + j) * 10;
+    out[0] = act ? E.pref * S : 0.;
+    for (int m = 0; m < 3; m++)
+        for (int c = 0; c < 3; c++)
+            out[1 + 3 * m + c] = act ? E.sig * (E.da[m][c] * S + E.pref * F[m][c]) : 0.;
+}
+
+// Near pairs of the field term, added to k_vjp_field_far's sums where it saw any
+__global__ __launch_bounds__(kBlock) void k_vjp_field_near(const double* __restrict__ geom,
+                                                           const double* __restrict__ sigma, int64_t n,
+                                                           const double* __restrict__ pts,
+                                                           const double* __restrict__ gk, int64_t npts,
+                                                           int64_t per_split, double* __restrict__ partV,
+                                                           const int* __restrict__ near)
+{
+    const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+    if (j >= n || !near[(j >> 6) * gridDim.y + blockIdx.y]) return;
+    const double* g = geom + j * KG_STRIDE;
+    Elem E;
+    load_elem(g, sigma[j], E);
+    if (!E.tri) return;
     const int64_t k0 = (int64_t)blockIdx.y * per_split;
     const int64_t k1 = std::min<int64_t>(npts, k0 + per_split);
     double acc[10];
     double* out = partV + ((int64_t)blockIdx.y * n + j) * 10;
-    for (int c = 0; c < 10; c++) acc[c] = NEAR ? out[c] : 0.;
-    if (E.tri) {
-        for (int64_t k = k0; k < k1; k++) {
-            const double px = pts[3 * k], py = pts[3 * k + 1], pz = pts[3 * k + 2], wk = gk[k];
-            const int reg = tri_regime_field(g, px, py, pz);
-            if (NEAR) {
-                if (reg != 0) continue;
-                Dual<9> V[3][3], P[3];
-                for (int m = 0; m < 3; m++)
-                    for (int c = 0; c < 3; c++) {
-                        V[m][c] = cst<9>(E.v[m][c]);
-                        V[m][c].d[3 * m + c] = 1.;
-                    }
-                P[0] = cst<9>(px);
-                P[1] = cst<9>(py);
-                P[2] = cst<9>(pz);
-                const Dual<9> G = tri_potential_cf<9>(P, V);
-                acc[0] += wk * G.v;
-                const double ws = wk * E.sig;
-                for (int c = 0; c < 9; c++) acc[1 + c] += ws * G.d[c];
-            } else {
-                if (reg == 0) continue;
-                double G, dv[9], dP[3];
-                far_derivs(E, rule, rule_slot(reg), reg, px, py, pz, G, dv, dP);
-                acc[0] += wk * G;
-                const double ws = wk * E.sig;
-                for (int c = 0; c < 9; c++) acc[1 + c] += ws * dv[c];
+    for (int c = 0; c < 10; c++) acc[c] = out[c];
+    for (int64_t k = k0; k < k1; k++) {
+        const double px = pts[3 * k], py = pts[3 * k + 1], pz = pts[3 * k + 2], wk = gk[k];
+        if (tri_regime_field(g, px, py, pz) != 0) continue;
+        Dual<9> V[3][3], P[3];
+        for (int m = 0; m < 3; m++)
+            for (int c = 0; c < 3; c++) {
+                V[m][c] = cst<9>(E.v[m][c]);
+                V[m][c].d[3 * m + c] = 1.;
             }
-        }
+        P[0] = cst<9>(px);
+        P[1] = cst<9>(py);
+        P[2] = cst<9>(pz);
+        const Dual<9> G = tri_potential_cf<9>(P, V);
+        acc[0] += wk * G.v;
+        const double ws = wk * E.sig;
+        for (int c = 0; c < 9; c++) acc[1 + c] += ws * G.d[c];
     }
     for (int c = 0; c < 10; c++) out[c] = acc[c];
 }
@@ -393,14 +535,25 @@ __global__ __launch_bounds__(kBlock) void k_vjp_matrix(const double* __restrict_
 __global__ __launch_bounds__(kBlock) void k_vjp_reduce_v(const double* __restrict__ partV, int nsplit, int64_t n,
                                                          double* __restrict__ dsig, double* __restrict__ dvert)
 {
+    // blockIdx.y = component; the loads of eight splits in flight
     const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (j >= n) return;
-    double s[10];
-    for (int c = 0; c < 10; c++) s[c] = 0.;
-    for (int k = 0; k < nsplit; k++)
-        for (int c = 0; c < 10; c++) s[c] += partV[((int64_t)k * n + j) * 10 + c];
-    if (dsig) dsig[j] = s[0];
-    for (int c = 0; c < 9; c++) dvert[j * 9 + c] = s[1 + c];
+    const int c = blockIdx.y;
+    if (j >= n || (c == 0 && !dsig)) return;
+    const double* p = partV + j * 10 + c;
+    double s = 0.;
+    int k = 0;
+    for (; k + 8 <= nsplit; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; q++) v[q] = p[(int64_t)(k + q) * n * 10];
+#pragma unroll
+        for (int q = 0; q < 8; q++) s += v[q];
+    }
+    for (; k < nsplit; k++) s += p[(int64_t)k * n * 10];
+    if (c == 0)
+        dsig[j] = s;
+    else
+        dvert[j * 9 + c - 1] = s;
 }
 
 // dvert[i*9 + 3m + c] += (sum_bx partP[bx][i][c]) / 3 for each corner m (c_i = mean of the vertices)
@@ -429,7 +582,8 @@ size_t vjp_workspace_doubles(int64_t n, int64_t npts)
 {
     const int64_t nbx = (n + kBlock - 1) / kBlock;
     const int sf = vjp_splits(nbx, npts), sm = vjp_splits(nbx, n);
-    return (size_t)std::max<int64_t>(sf, sm) * n * 10 + (size_t)nbx * n * 3;
+    // partial sums of the splits, the matrix term's sums per target, the field term's near flags
+    return (size_t)std::max<int64_t>(sf, sm) * n * 10 + (size_t)nbx * n * 3 + (size_t)((n + 63) / 64) * 128;
 }
 
 hipError_t launch_field_vjp(hipStream_t st, const double* geom, const double* sigma, const double* rule, int64_t n,
@@ -438,14 +592,17 @@ hipError_t launch_field_vjp(hipStream_t st, const double* geom, const double* si
 {
     if (n <= 0) return hipSuccess;
     if (ws_doubles < vjp_workspace_doubles(n, npts)) return hipErrorInvalidValue;
-    const int64_t nbx = nblocks(n);
-    const int s = npts > 0 ? vjp_splits(nbx, npts) : 1;
-    const int64_t per = npts > 0 ? (npts + s - 1) / s : 1;
-    const int ns = npts > 0 ? (int)((npts + per - 1) / per) : 1;
-    dim3 grid((unsigned)nbx, (unsigned)ns);
-    k_vjp_field<false><<<grid, kBlock, 0, st>>>(geom, sigma, rule, n, pts, gk, npts, per, ws);
-    k_vjp_field<true><<<grid, kBlock, 0, st>>>(geom, sigma, rule, n, pts, gk, npts, per, ws);
-    k_vjp_reduce_v<<<(unsigned)nbx, kBlock, 0, st>>>(ws, ns, n, dsig, dvert);
+    const int64_t nbx = nblocks(n), sf = vjp_splits(nbx, npts);
+    // splits of whole rounds of the block's wavefronts (256 points), within the workspace's and 256
+    constexpr int64_t kRound = 64 * kVjpWaves;
+    const int64_t rounds = std::max<int64_t>(1, (npts + kRound - 1) / kRound);
+    const int64_t per = (rounds + sf - 1) / sf * kRound;
+    const int ns = (int)std::max<int64_t>(1, (npts + per - 1) / per);
+    int* near = reinterpret_cast<int*>(ws + (size_t)sf * n * 10);
+    k_vjp_field_far<<<dim3((unsigned)((n + 63) / 64), (unsigned)ns), kRound, 0, st>>>(geom, sigma, rule, n, pts, gk, npts,
+                                                                                     per, ws, near);
+    k_vjp_field_near<<<dim3((unsigned)nbx, (unsigned)ns), kBlock, 0, st>>>(geom, sigma, n, pts, gk, npts, per, ws, near);
+    k_vjp_reduce_v<<<dim3((unsigned)nbx, 10), kBlock, 0, st>>>(ws, ns, n, dsig, dvert);
     return hipGetLastError();
 }
 
@@ -464,7 +621,7 @@ hipError_t launch_matrix_vjp(hipStream_t st, const double* geom, const double* t
     dim3 grid((unsigned)nbx, (unsigned)ns);
     k_vjp_matrix<false><<<grid, kBlock, 0, st>>>(geom, targets, rule, n, lw, u, per, partV, partP);
     k_vjp_matrix<true><<<grid, kBlock, 0, st>>>(geom, targets, rule, n, lw, u, per, partV, partP);
-    k_vjp_reduce_v<<<(unsigned)nbx, kBlock, 0, st>>>(partV, ns, n, nullptr, dvert);
+    k_vjp_reduce_v<<<dim3((unsigned)nbx, 10), kBlock, 0, st>>>(partV, ns, n, nullptr, dvert);
     k_vjp_reduce_p<<<(unsigned)nbx, kBlock, 0, st>>>(partP, (int)nbx, n, dvert);
     return hipGetLastError();
 }
