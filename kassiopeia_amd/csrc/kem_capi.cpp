@@ -322,7 +322,7 @@ WsNeed field_ws_need(const kem_ctx* c, const kem_mesh* m, const kem::FieldMesh& 
                      int64_t npts, bool mixed, int64_t range)
 {
     WsNeed n;
-    const kem::TreePlan tp = kem::plan_tree(c->policy, fm, mixed, c->mixed_fp64_ratio, multi, npts);
+    const kem::TreePlan tp = kem::plan_tree(c->policy, fm, mixed, c->mixed_fp64_ratio, multi, nsets, npts);
     n.ws = tp.use ? tp.doubles()
                   : kem::field_workspace_doubles(c->policy, fm, mixed, c->mixed_fp64_ratio, multi, nsets, npts, range);
     n.gsig = m->gstart ? nsets * m->nm : 0;

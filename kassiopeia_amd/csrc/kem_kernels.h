@@ -64,15 +64,18 @@ struct TreePlan {
     bool use = false;
     TreeLevels levels;
     int per_lane = 1;      // points per lane
+    int64_t sets = 1;      // charge-density sets, each with its expansions
     int slices = 1;        // blocks per group of 64 per_lane points, each with a slice of the partial sums
     int64_t moments = 0, ranges = 0, partials = 0, chunk = 0;
     int64_t doubles() const { return moments + ranges + partials; }
 };
-TreePlan plan_tree(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t npts);
+TreePlan plan_tree(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t nsets,
+                   int64_t npts);
 // Sums over all elements at npts points in curve order, in p.slices slices of the partial layout out (component c,
-// slice s, point i at (c * slices + s) * npts + i); moments: expand the charges into mom first.
+// slice s, point i at (c * slices + s) * npts + i); moments: expand the charges into mom first.  pset (a plan of
+// several sets): the points' sets, in ascending order, and the points in curve order within each.
 hipError_t launch_tree(hipStream_t st, const FieldMesh& m, const TreePlan& p, bool mixed, const double* sigma,
-                       const double* px, const double* py, const double* pz, int64_t npts, double* mom, double* ranges,
+                       const int32_t* pset, const double* px, const double* py, const double* pz, int64_t npts, double* mom, double* ranges,
                        double* out, bool moments);
 
 // phi/E at npts points (SoA) from the mesh's elements with charge densities sigma.  pset

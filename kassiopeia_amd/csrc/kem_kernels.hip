@@ -1988,15 +1988,15 @@ namespace {
 // The hierarchical pass over points in curve order: expansions at the start of ws, then the point groups' ranges
 // and the partial sums of a chunk of points.
 hipError_t tree_field(hipStream_t st, const FieldMesh& m, const TreePlan& p, bool mixed, const double* sigma,
-                      const double* px, const double* py, const double* pz, int64_t npts, double* phi, double* ex,
+                      const int32_t* pset, const double* px, const double* py, const double* pz, int64_t npts, double* phi, double* ex,
                       double* ey, double* ez, double* ws, hipEvent_t far_begin, hipEvent_t far_end)
 {
     double* q = ws + p.moments + p.ranges;
     if (far_begin) (void)hipEventRecord(far_begin, st);
     for (int64_t p0 = 0; p0 < npts; p0 += p.chunk) {
         const int64_t np = std::min(p.chunk, npts - p0);
-        const hipError_t e = launch_tree(st, m, p, mixed, sigma, px + p0, py + p0, pz + p0, np, ws, ws + p.moments, q,
-                                         p0 == 0);
+        const hipError_t e = launch_tree(st, m, p, mixed, sigma, pset ? pset + p0 : nullptr, px + p0, py + p0, pz + p0,
+                                         np, ws, ws + p.moments, q, p0 == 0);
         if (e != hipSuccess) return e;
         if (far_end && p0 + np >= npts) (void)hipEventRecord(far_end, st);
         k_field_combine<<<dim3(nblocks(np), 4), kBlock, 0, st>>>(q, p.slices, np, phi + p0, ex + p0, ey + p0, ez + p0);
@@ -2015,9 +2015,9 @@ hipError_t launch_field(hipStream_t st, int policy, const FieldMesh& m, bool mix
     if (nsets < 1 || !phi || !ex || !ey || !ez) return hipErrorInvalidValue;
     if (side && side->st && (!side->fork || !side->join)) return hipErrorInvalidValue;
     hipError_t e;
-    const TreePlan tp = plan_tree(policy, m, mixed, fp64_ratio, pset != nullptr, npts);
+    const TreePlan tp = plan_tree(policy, m, mixed, fp64_ratio, pset != nullptr, nsets, npts);
     if (tp.use && tp.doubles() <= ws_doubles)
-        e = tree_field(st, m, tp, mixed, sigma, px, py, pz, npts, phi, ex, ey, ez, ws, far_begin, far_end);
+        e = tree_field(st, m, tp, mixed, sigma, pset, px, py, pz, npts, phi, ex, ey, ez, ws, far_begin, far_end);
     else if (pset)
         e = field_passes<true>(st, policy, m, mixed, fp64_ratio, sigma, pset, nsets, px, py, pz, npts, phi, ex, ey,
                                ez, ws, ws_doubles, range_elems, far_begin, far_end, side);

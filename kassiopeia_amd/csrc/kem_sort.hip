@@ -65,11 +65,13 @@ __device__ __forceinline__ uint64_t spread3(uint64_t a)
 }
 
 // Hilbert key (kCurveBits bits per axis) of each point in the cube over the box spanned by the block
-// partials: J. Skilling, "Programming the Hilbert curve" (2004), axes to transposed index.  Points of several
-// charge-density sets sort together: the kernels read the sets element-major, so a wavefront may mix sets.
+// partials: J. Skilling, "Programming the Hilbert curve" (2004), axes to transposed index.  pset (nullable): the set
+// above the curve's bits, for the hierarchical pass.  The flat passes' points of several charge-density sets sort
+// together: their kernels read the sets element-major, so a wavefront may mix sets.
 constexpr int kCurveBits = 16;
 __global__ __launch_bounds__(kBlock) void k_curve(const double* __restrict__ x, const double* __restrict__ y,
                                                   const double* __restrict__ z, int64_t n,
+                                                  const int32_t* __restrict__ pset,
                                                   const double* __restrict__ part, int nparts,
                                                   uint64_t* __restrict__ key, int32_t* __restrict__ idx)
 {
@@ -119,7 +121,8 @@ __global__ __launch_bounds__(kBlock) void k_curve(const double* __restrict__ x, 
     uint32_t t = 0;
     for (uint32_t q = 1u << (kCurveBits - 1); q > 1; q >>= 1)
         if (a[2] & q) t ^= q - 1;
-    key[i] = spread3(a[2] ^ t) | spread3(a[1] ^ t) << 1 | spread3(a[0] ^ t) << 2;
+    const uint64_t set = pset ? (uint64_t)(uint32_t)pset[i] << (3 * kCurveBits) : 0;
+    key[i] = set | spread3(a[2] ^ t) | spread3(a[1] ^ t) << 1 | spread3(a[0] ^ t) << 2;
     idx[i] = (int32_t)i;
 }
 
@@ -206,8 +209,14 @@ hipError_t launch_field_sorted(hipStream_t st, int policy, const FieldMesh& m, b
     int nb = (int)((npts + kBlock - 1) / kBlock);
     if (nb > kBoxParts) nb = kBoxParts;
     k_bbox_part<<<nb, kBlock, 0, st>>>(px, py, pz, npts, box);
-    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, box, nb, k0, i0);
-    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 3 * kCurveBits, st);
+    // the hierarchical pass takes the points set by set (as launch_field decides)
+    int bits = 3 * kCurveBits;
+    const TreePlan tp = plan_tree(policy, m, mixed, fp64_ratio, pset != nullptr, nsets, npts);
+    const bool by_set = pset && tp.use && tp.doubles() <= ws_doubles;
+    if (by_set)
+        for (int64_t v = nsets - 1; v > 0; v >>= 1) bits++;
+    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, by_set ? pset : nullptr, box, nb, k0, i0);
+    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, bits, st);
     if (e != hipSuccess) return e;
     k_gather3<<<nblocks(npts), kBlock, 0, st>>>(i1, px, py, pz, pset, npts, sx, sy, sz, ss);
     e = launch_field(st, policy, m, mixed, fp64_ratio, sigma, pset ? ss : nullptr, nsets, sx, sy, sz, npts, o[0], o[1],
@@ -246,7 +255,7 @@ hipError_t launch_census_paths_sorted(hipStream_t st, const FieldMesh& m, const 
     int nb = (int)((npts + kBlock - 1) / kBlock);
     if (nb > kBoxParts) nb = kBoxParts;
     k_bbox_part<<<nb, kBlock, 0, st>>>(px, py, pz, npts, box);
-    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, box, nb, k0, i0);
+    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, nullptr, box, nb, k0, i0);
     hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 3 * kCurveBits, st);
     if (e != hipSuccess) return e;
     k_gather3<<<nblocks(npts), kBlock, 0, st>>>(i1, px, py, pz, nullptr, npts, sx, sy, sz, ss);

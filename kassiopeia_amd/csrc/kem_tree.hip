@@ -66,6 +66,48 @@ __device__ __forceinline__ bool order_of(int v, int& l, int& m)
     return l >= m && l <= P;
 }
 
+// one quadrature node (position about the run's centre, charge) into line m's sums, scaled as um = (2m-1)!! says
+template <int P>
+__device__ __forceinline__ void follow(const double4& node, int m, double um, double (&A)[P + 1], double (&B)[P + 1])
+{
+    const double x = node.x, y = node.y, z = node.z;
+    const double d2 = x * x + y * y + z * z;
+    // (x + i y)^m by its binary digits
+    double C = node.w, S = 0., bx = x, by = y;
+#pragma unroll
+    for (int bit = 1; bit < 32; bit <<= 1) {
+        if (m & bit) {
+            const double c = C * bx - S * by;
+            S = C * by + S * bx;
+            C = c;
+        }
+        const double c = bx * bx - by * by;
+        by = 2. * bx * by;
+        bx = c;
+    }
+    double u0 = 0., u1 = um, f = 2 * m + 1, gd = 0.;  // f = 2l + 1, gd = l^2 - m^2
+#pragma unroll
+    for (int i = 0; i <= P; i++) {
+        if (m + i <= P) {
+            A[i] = __builtin_fma(C, u1, A[i]);
+            B[i] = __builtin_fma(S, u1, B[i]);
+            const double u2 = __builtin_fma(f * z, u1, -(gd * d2) * u0);
+            u0 = u1;
+            u1 = u2;
+            gd += f;
+            f += 2.;
+        }
+    }
+}
+// from those sums to the stored coefficients of order (l, m)
+__device__ __forceinline__ double unscale_divisor(int l, int m)
+{
+    double f = m ? 0.5 : 1.;  // 2 for the pair of orders m and -m
+    for (int k = 2; k <= l + m; k++) f *= k;
+    for (int k = 2; k <= l - m; k++) f *= k;
+    return f;
+}
+
 // Expansion of each run of the lowest stored level: one block per run.  The quadrature nodes (33 per surface
 // element, 16 per wire) of 16 elements at a time are staged in LDS, as positions about the centre and charges; half a
 // wavefront follows one node, lane m its line m, with the sums in registers; the halves are added by a shuffle and
@@ -108,36 +150,7 @@ __global__ __launch_bounds__(kP2MBlock) void k_tree_p2m(const double* __restrict
             pt[q] = double4{(nd[0] - cx) * ia, (nd[1] - cy) * ia, (nd[2] - cz) * ia, w};
         }
         __syncthreads();
-        for (int q = half; q < nq; q += kP2MBlock / 32) {
-            const double x = pt[q].x, y = pt[q].y, z = pt[q].z;
-            const double d2 = x * x + y * y + z * z;
-            // (x + i y)^m by its binary digits
-            double C = pt[q].w, S = 0., bx = x, by = y;
-#pragma unroll
-            for (int bit = 1; bit < 32; bit <<= 1) {
-                if (m & bit) {
-                    const double c = C * bx - S * by;
-                    S = C * by + S * bx;
-                    C = c;
-                }
-                const double c = bx * bx - by * by;
-                by = 2. * bx * by;
-                bx = c;
-            }
-            double u0 = 0., u1 = um, f = 2 * m + 1, gd = 0.;  // f = 2l + 1, gd = l^2 - m^2
-#pragma unroll
-            for (int i = 0; i <= P; i++) {
-                if (m + i <= P) {
-                    A[i] = __builtin_fma(C, u1, A[i]);
-                    B[i] = __builtin_fma(S, u1, B[i]);
-                    const double u2 = __builtin_fma(f * z, u1, -(gd * d2) * u0);
-                    u0 = u1;
-                    u1 = u2;
-                    gd += f;
-                    f += 2.;
-                }
-            }
-        }
+        for (int q = half; q < nq; q += kP2MBlock / 32) follow<P>(pt[q], m, um, A, B);
     }
 #pragma unroll
     for (int i = 0; i <= P; i++) {
@@ -155,16 +168,98 @@ __global__ __launch_bounds__(kP2MBlock) void k_tree_p2m(const double* __restrict
         if (order_of<P>(v, l, mm)) {
             const int at = tri_index(l, mm);
             for (int k = 0; k < kWaves; k++) s += red[k][at][v & 1];
-            double f = mm ? 0.5 : 1.;  // 2 for the pair of orders m and -m
-            for (int k = 2; k <= l + mm; k++) f *= k;
-            for (int k = 2; k <= l - mm; k++) f *= k;
-            s /= f;
+            s /= unscale_divisor(l, mm);
         }
         o[v] = s;
     }
 }
 
-// Expansions of one level's runs from those of the level below: one block per run.  Two groups of 512 threads
+// The same for several charge-density sets: one block per run expands each of its elements at unit charge density once
+// (half a wavefront per element, its nodes as above) and leaves the coefficients in LDS; the sets' expansions are sums
+// of them, a thread per coefficient (64 sets of 20,000 triangles 0.56 ms, and 2.7 ms the levels above).
+template <int P>
+__global__ __launch_bounds__(kP2MBlock) void k_tree_p2m_sets(const double* __restrict__ geom,
+                                                             const double* __restrict__ nodes,
+                                                             const int32_t* __restrict__ order,
+                                                             const double* __restrict__ sigma, int64_t nsets,
+                                                             const double* __restrict__ tnode, int64_t nelem, int run,
+                                                             double* __restrict__ mom, int64_t mom_set)
+{
+    static_assert(P < 32, "a line per lane of half a wavefront");
+    constexpr int kNodes = 33, kElems = 8, T = tri_index(P, P) + 1, kSets = 32;
+    __shared__ double4 pt[kElems * kNodes];
+    __shared__ double unit[kElems][2 * T];
+    __shared__ double sg[kSets][kElems];
+    const int64_t node = blockIdx.x;
+    const double* t = tnode + node * KEM_TREE_STRIDE;
+    const double cx = t[0], cy = t[1], cz = t[2], ia = t[5];
+    const int64_t e0 = node * run;
+    const int ne = (int)(nelem - e0 < run ? nelem - e0 : run);
+    const int half = threadIdx.x >> 5, m = threadIdx.x & 31;
+    double um = 1.;
+    for (int i = 1; i <= m; i++) um *= 2 * i - 1;
+    for (int s0 = 0; s0 < ne; s0 += kElems) {
+        const int nq = min(ne - s0, kElems) * kNodes;
+        __syncthreads();
+        for (int q = threadIdx.x; q < kElems * kNodes; q += kP2MBlock) {
+            pt[q] = double4{0., 0., 0., 0.};
+            if (q >= nq) continue;
+            const int e = q / kNodes, k = q - e * kNodes;
+            const int64_t j = order[e0 + s0 + e];
+            const double* g = geom + j * KG_STRIDE;
+            const bool wire = (int)g[KG_TYPE] == KEM_LINESEGMENT;
+            const double* nd = nodes + j * KEM_NODE_STRIDE + 4 * (wire ? KEM_L16 + (k & 15) : KEM_N33 + k);
+            const double w = wire && k >= 16 ? 0. : nd[3] * g[KG_PREF];
+            pt[q] = double4{(nd[0] - cx) * ia, (nd[1] - cy) * ia, (nd[2] - cz) * ia, w};
+        }
+        __syncthreads();
+        {
+            double A[P + 1], B[P + 1];
+#pragma unroll
+            for (int i = 0; i <= P; i++) A[i] = B[i] = 0.;
+            for (int q = half * kNodes; q < (half + 1) * kNodes; q++) follow<P>(pt[q], m, um, A, B);
+#pragma unroll
+            for (int i = 0; i <= P; i++)
+                if (m + i <= P) {
+                    const int at = tri_index(m + i, m);
+                    unit[half][2 * at] = A[i];
+                    unit[half][2 * at + 1] = B[i];
+                }
+        }
+        for (int64_t c0 = 0; c0 < nsets; c0 += kSets) {
+            const int nc = (int)(nsets - c0 < kSets ? nsets - c0 : kSets);
+            __syncthreads();
+            {
+                const int e = threadIdx.x & (kElems - 1), c = threadIdx.x / kElems;
+                static_assert(kP2MBlock == kElems * kSets, "a charge density per thread");
+                sg[c][e] = s0 + e < ne && c < nc ? sigma[(c0 + c) * nelem + order[e0 + s0 + e]] : 0.;
+            }
+            __syncthreads();
+            for (int v = threadIdx.x; v < 2 * entries(P); v += kP2MBlock) {
+                int l, mm;
+                double u[kElems];
+                const bool have = order_of<P>(v, l, mm);
+                const int at = have ? 2 * tri_index(l, mm) + (v & 1) : 0;
+#pragma unroll
+                for (int e = 0; e < kElems; e++) u[e] = have ? unit[e][at] : 0.;
+                if (have) {
+                    const double f = unscale_divisor(l, mm);
+#pragma unroll
+                    for (int e = 0; e < kElems; e++) u[e] /= f;
+                }
+                double* o = mom + c0 * mom_set + node * (2 * entries(P)) + v;
+                for (int c = 0; c < nc; c++) {
+                    double s = s0 ? o[c * mom_set] : 0.;
+#pragma unroll
+                    for (int e = 0; e < kElems; e++) s = __builtin_fma(u[e], sg[c][e], s);
+                    o[c * mom_set] = s;
+                }
+            }
+        }
+    }
+}
+
+// Expansions of one level's runs from those of the level below: one block per run (and set, blockIdx.y).  Two groups of 512 threads
 // translate a child each at a time by the addition theorem of the R_l^m (exact up to order P), a thread per (l, m).
 // Both factors lie in LDS with their negative orders written out, so the sum over (k, j) is two 16-byte
 // reads and four multiply-adds a term.
@@ -173,8 +268,10 @@ template <int P>
 __global__ __launch_bounds__(2 * kM2MGroup) void k_tree_m2m(const double* __restrict__ tchild,
                                                             const double* __restrict__ tparent, int64_t nchild,
                                                             const double* __restrict__ mchild,
-                                                            double* __restrict__ mparent)
+                                                            double* __restrict__ mparent, int64_t mom_set)
 {
+    mchild += blockIdx.y * mom_set;
+    mparent += blockIdx.y * mom_set;
     constexpr int T = tri_index(P, P) + 1, N = (P + 1) * (P + 1);  // (l, m) at l^2 + l + m
     static_assert(T <= kM2MGroup, "a thread per order");
     __shared__ double2 R[2][N], Q[2][N];
@@ -363,17 +460,19 @@ struct Sums {
 // Ranges of a group's points that share a walk.  Usually the whole group; where the curve leaves the points' region and
 // comes back, or leaps over a gap, the group is halved until its halves are alike (one not under 0.4 of the whole's
 // radius) or hold kRangePoints, so that a few stray points do not blow up the sphere of all.  Record per
-// range: centre, radius, first and end point in the group; an empty range ends the list.
+// range: centre, radius, first and end point in the group; an empty range ends the list.  SETS: the points lie in curve
+// order within their charge-density sets, a range ends where the set changes, and its record holds the set too.
 constexpr int kRangePoints = 16;
-template <int NP>
+template <int NP, bool SETS>
 struct Ranges {
-    static constexpr int N = 64 * NP / kRangePoints;
-    double v[N][6];
+    static constexpr int N = SETS ? 64 * NP : 64 * NP / kRangePoints;
+    double v[N][SETS ? 7 : 6];
 };
-template <int NP>
+template <int NP, bool SETS>
 __global__ __launch_bounds__(64) void k_tree_ranges(const double* __restrict__ px, const double* __restrict__ py,
-                                                    const double* __restrict__ pz, int64_t npts,
-                                                    Ranges<NP>* __restrict__ out)
+                                                    const double* __restrict__ pz,
+                                                    const int32_t* __restrict__ pset, int64_t npts,
+                                                    Ranges<NP, SETS>* __restrict__ out)
 {
     const int lane = threadIdx.x;
     const int64_t grp = blockIdx.x;
@@ -412,9 +511,17 @@ __global__ __launch_bounds__(64) void k_tree_ranges(const double* __restrict__ p
         return dev::uniform(sqrt(far));
     };
     int a = 0, len = 64 * NP, k = 0;
-    Ranges<NP>* o = out + grp;
+    Ranges<NP, SETS>* o = out + grp;
+    auto set_of = [&](int at) {
+        const int64_t i = grp * NP * 64 + at;
+        return pset[i < npts ? i : npts - 1];
+    };
     while (a < 64 * NP) {
         const int b = a + len;
+        if (SETS && set_of(a) != set_of(b - 1)) {
+            len /= 2;
+            continue;
+        }
         if (len > kRangePoints) {
             const double r1 = sphere(a, a + len / 2), r2 = sphere(a + len / 2, b);
             const double r = sphere(a, b);
@@ -429,12 +536,13 @@ __global__ __launch_bounds__(64) void k_tree_ranges(const double* __restrict__ p
             o->v[k][3] = r;
             o->v[k][4] = a;
             o->v[k][5] = b;
+            if constexpr (SETS) o->v[k][6] = set_of(a);
         }
         k++;
         a = b;
         len = a ? a & -a : len;
     }
-    if (lane == 0 && k < Ranges<NP>::N) o->v[k][5] = 0.;
+    if (lane == 0 && k < Ranges<NP, SETS>::N) o->v[k][5] = 0.;
 }
 
 template <bool TRIANGLES>
@@ -459,14 +567,14 @@ constexpr int kTreeStack = 64 + 48 * (KEM_TREE_LEVELS + 1);
 // through LDS.  A run's coefficients pass through LDS too; the other wavefronts of the SIMD cover the wait for
 // them.  Three wavefronts per SIMD are asked for: a few registers spill, and the million mixed points over 20,000
 // triangles take 20.3 ms instead of 21.8 at two.  Bound by the vector ALU: half expansions, half pairs close by.
-template <bool MIXED, int NP, bool TRIANGLES>
+template <bool MIXED, int NP, bool TRIANGLES, bool SETS>
 __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_field_tree(
     const double* __restrict__ geom, const double* __restrict__ nodes, const float* __restrict__ nodes32,
     const float* __restrict__ far6, const double* __restrict__ far6_cl, const int32_t* __restrict__ order,
     const double* __restrict__ sigma, const double* __restrict__ tnode, const double* __restrict__ mom,
     TreeLevels T, int64_t nelem, const double* __restrict__ px, const double* __restrict__ py,
-    const double* __restrict__ pz, const Ranges<NP>* __restrict__ ranges, int64_t npts, int64_t ngroups,
-    int slices, double* __restrict__ out, int64_t comp_stride)
+    const double* __restrict__ pz, const Ranges<NP, SETS>* __restrict__ ranges, int64_t npts, int64_t ngroups,
+    int slices, double* __restrict__ out, int64_t comp_stride, int64_t mom_set)
 {
     using O = Orders<MIXED>;
     constexpr int E = entries(O::P);
@@ -496,11 +604,18 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
     }
     Sums<MIXED> sum[NP];
     int turn = 0;
-    for (int range = 0; range < Ranges<NP>::N; range++) {
+    for (int range = 0; range < Ranges<NP, SETS>::N; range++) {
         const double* rg = ranges[grp].v[range];
         const int ra = (int)rg[4], rb = (int)rg[5];
         if (rb == 0) break;
         const double wx = rg[0], wy = rg[1], wz = rg[2], wr = rg[3];
+        const double* sg = sigma;
+        const double* ms = mom;
+        if constexpr (SETS) {
+            const int64_t set = (int64_t)rg[6];
+            sg += set * nelem;
+            ms += set * mom_set;
+        }
         bool in[NP];  // the lane's points that belong to the range
 #pragma unroll
         for (int n = 0; n < NP; n++) in[n] = n * 64 + lane >= ra && n * 64 + lane < rb;
@@ -557,7 +672,7 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
                 const int node = __builtin_amdgcn_readlane(at, b);
                 const int p = max(1, __builtin_amdgcn_readlane(ord, b));
                 const double* u = tnode + (int64_t)node * KEM_TREE_STRIDE;
-                const Pair* src = reinterpret_cast<const Pair*>(mom) + (int64_t)(node - T.first[T.low]) * E;
+                const Pair* src = reinterpret_cast<const Pair*>(ms) + (int64_t)(node - T.first[T.low]) * E;
                 __builtin_amdgcn_wave_barrier();
                 for (int k = lane; k < line_start(O::P, p + 2); k += 64) co[k] = src[k];
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -584,7 +699,7 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
                     const int64_t j = order[k];
                     const double* g = geom + j * KG_STRIDE;
                     if (!MIXED) {
-                        const double sj = sigma[j];
+                        const double sj = sg[j];
 #pragma unroll
                         for (int n = 0; n < NP; n++) {
                             const double r2 = dev::dist2(g, x[n], y[n], z[n]);
@@ -601,7 +716,7 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
                     const dev::v16f* rv = reinterpret_cast<const dev::v16f*>(far6 + k * KEM_FAR6_STRIDE);
                     const dev::v16f A = rv[0], B = rv[1];
                     const double cx = dev::f2d(B[8], B[9]), cy = dev::f2d(B[10], B[11]), cz = dev::f2d(B[12], B[13]);
-                    const double sj = sigma[j], wj = g[KG_PREF] * sj;
+                    const double sj = sg[j], wj = g[KG_PREF] * sj;
                     const double ux = wx - cx, uy = wy - cy, uz = wz - cz;
                     const double te = dev::f2d(B[14], B[15]) + wr;
                     const bool six = ux * ux + uy * uy + uz * uz > te * te;
@@ -669,49 +784,57 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
 }
 
 template <bool MIXED>
-hipError_t tree_passes(hipStream_t st, const FieldMesh& m, const TreePlan& p, const double* sigma, const double* px,
-                       const double* py, const double* pz, int64_t npts, double* mom, double* ranges, double* out,
-                       bool moments)
+hipError_t tree_passes(hipStream_t st, const FieldMesh& m, const TreePlan& p, const double* sigma, const int32_t* pset,
+                       const double* px, const double* py, const double* pz, int64_t npts, double* mom, double* ranges,
+                       double* out, bool moments)
 {
     constexpr int P = Orders<MIXED>::P;
     const TreeLevels& T = p.levels;
     const int64_t stride = 2 * entries(P);
-    const int64_t base = T.first[T.low];
+    const int64_t base = T.first[T.low], mom_set = p.moments / p.sets;
     if (moments) {
-        k_tree_p2m<P><<<(unsigned)T.count[T.low], kP2MBlock, 0, st>>>(
-            m.geom, m.nodes, m.order, sigma, m.tree + base * KEM_TREE_STRIDE, m.n, T.run, mom);
+        const double* low = m.tree + base * KEM_TREE_STRIDE;
+        if (pset)
+            k_tree_p2m_sets<P><<<(unsigned)T.count[T.low], kP2MBlock, 0, st>>>(m.geom, m.nodes, m.order, sigma, p.sets,
+                                                                              low, m.n, T.run, mom, mom_set);
+        else
+            k_tree_p2m<P><<<(unsigned)T.count[T.low], kP2MBlock, 0, st>>>(m.geom, m.nodes, m.order, sigma, low, m.n,
+                                                                         T.run, mom);
         for (int k = T.low + 1; k < T.levels; k++)
-            k_tree_m2m<P><<<(unsigned)T.count[k], 2 * kM2MGroup, 0, st>>>(
+            k_tree_m2m<P><<<dim3((unsigned)T.count[k], (unsigned)p.sets), 2 * kM2MGroup, 0, st>>>(
                 m.tree + (int64_t)T.first[k - 1] * KEM_TREE_STRIDE, m.tree + (int64_t)T.first[k] * KEM_TREE_STRIDE,
-                T.count[k - 1], mom + (T.first[k - 1] - base) * stride, mom + (T.first[k] - base) * stride);
+                T.count[k - 1], mom + (T.first[k - 1] - base) * stride, mom + (T.first[k] - base) * stride, mom_set);
     }
     const int64_t groups = (npts + 64 * p.per_lane - 1) / (64 * p.per_lane);
     const int64_t unit = 8 * (int64_t)kTreeNeighbours * p.slices;
     const unsigned grid = (unsigned)((groups * p.slices + unit - 1) / unit * unit);
-    auto launch = [&](auto np) {
+    auto launch = [&](auto np, auto sets) {
         constexpr int NP = decltype(np)::value;
-        Ranges<NP>* rg = reinterpret_cast<Ranges<NP>*>(ranges);
-        k_tree_ranges<NP><<<(unsigned)groups, 64, 0, st>>>(px, py, pz, npts, rg);
+        constexpr bool SETS = decltype(sets)::value;
+        auto* rg = reinterpret_cast<Ranges<NP, SETS>*>(ranges);
+        k_tree_ranges<NP, SETS><<<(unsigned)groups, 64, 0, st>>>(px, py, pz, pset, npts, rg);
         auto run = [&](auto triangles) {
-            k_field_tree<MIXED, NP, decltype(triangles)::value><<<grid, 64 * kTreeWaves, 0, st>>>(
+            k_field_tree<MIXED, NP, decltype(triangles)::value, SETS><<<grid, 64 * kTreeWaves, 0, st>>>(
                 m.geom, m.nodes, m.nodes32, m.far6, m.far6_cl, m.order, sigma, m.tree, mom, T, m.n, px, py, pz, rg,
-                npts, groups, p.slices, out, p.slices * npts);
+                npts, groups, p.slices, out, p.slices * npts, mom_set);
         };
         if (m.triangles)
             run(std::true_type());
         else
             run(std::false_type());
     };
-    if (p.per_lane == 2)
-        launch(std::integral_constant<int, 2>());
+    if (pset)
+        launch(std::integral_constant<int, 1>(), std::true_type());
+    else if (p.per_lane == 2)
+        launch(std::integral_constant<int, 2>(), std::false_type());
     else
-        launch(std::integral_constant<int, 1>());
+        launch(std::integral_constant<int, 1>(), std::false_type());
     return hipGetLastError();
 }
 
 }  // namespace
 
-// The hierarchical pass serves single charge-density sets of planar elements and wires under the numeric policy
+// The hierarchical pass serves planar elements and wires under the numeric policy
 // (in mixed precision without an FP64 band), at 4,096 points or more, which the caller has put in curve order.
 // Below these sizes the flat pass is the faster one: its cost grows with elements times points, while here the
 // expansions take 0.2 ms and a group's walk its elements close by.  Measured, us flat / hierarchical:
@@ -725,6 +848,20 @@ inline bool tree_pays(bool mixed, double n, double m)
 {
     if (mixed) return n >= 3000. && n * m >= 1e8;
     return n >= 1536. && (m >= 8192. ? n * m >= 5e7 : n * m >= 1.5e8);
+}
+// Points of several sets are visited set by set, so the groups are less compact the fewer points a set has, and each set
+// has its expansions: the pass serves them from a product of elements and points per set on.  Measured on the coax, us
+// flat / hierarchical (elements x points x sets):
+//   FP64   6,000 x 80,000 x 8  11,886 / 9,498   x 16  11,975 / 11,430   x 32  11,983 / 13,634
+//          20,000 x 300,000 x 2  147,681 / 32,920   x 64  151,516 / 78,499   20,000 x 80,000 x 64  41,528 / 41,429
+//   mixed  20,000 x 80,000 x 8  8,078 / 7,022   x 16  8,157 / 8,717   12,000 x 80,000 x 4  5,070 / 4,413
+//          20,000 x 300,000 x 2  26,031 / 9,702   x 32  26,266 / 21,063   x 64  37,562 / 27,769 (there the flat pass's
+//          element weights no longer fit an XCD's L2)   6,000 x 300,000 x 16  11,265 / 10,029   x 32  11,382 / 11,934
+constexpr int64_t kTreeMaxSets = 65535;
+inline bool sets_pay(bool mixed, double n, double m, double nsets)
+{
+    const double each = n * m / nsets;
+    return mixed ? each >= (m >= 262144. && n >= 6000. ? 9e7 : 1.9e8) : each >= 3.5e7;
 }
 // wavefronts in all: kTreeWaves times p.slices of them per group of points.  Many more than the chip holds at once, since
 // groups differ in their work, a few by 10 times (400,000 points over 100,000 triangles: 18.2 ms at 8 per group,
@@ -743,47 +880,51 @@ constexpr int64_t kTreeLargeDoubles = (int64_t)512 << 20;
 // partial sums of one chunk of points
 constexpr int64_t kTreePartialDoubles = (int64_t)128 << 20;
 
-TreePlan plan_tree(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t npts)
+TreePlan plan_tree(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t nsets,
+                   int64_t npts)
 {
     TreePlan p;
-    if (policy != 0 || multi || m.axisym || !m.tree || !m.order || !m.clusters) return p;
+    if (policy != 0 || m.axisym || !m.tree || !m.order || !m.clusters) return p;
     if (mixed && (fp64_ratio != 0. || !m.nodes32 || !m.far6 || !m.far6_cl)) return p;
     if (npts < kTreeMinPoints || !tree_pays(mixed, (double)m.n, (double)npts) || npts > INT32_MAX ||
         m.n > ((int64_t)1 << KEM_TREE_INDEX_BITS))
         return p;
+    if (multi && (nsets > kTreeMaxSets || !sets_pay(mixed, (double)m.n, (double)npts, (double)nsets))) return p;
+    p.sets = multi ? nsets : 1;
     TreeLevels& T = p.levels;
     tree_levels(m.n, T);
     const int P = mixed ? Orders<true>::P : Orders<false>::P;
-    const int64_t limit = npts <= kTreeSmallPoints ? kTreeSmallDoubles : kTreeLargeDoubles;
+    const int64_t limit = !multi && npts <= kTreeSmallPoints ? kTreeSmallDoubles : kTreeLargeDoubles;
     const int64_t total = T.first[T.levels - 1] + T.count[T.levels - 1];
     for (T.low = 0; T.low < T.levels; T.low++) {
-        p.moments = (total - T.first[T.low]) * 2 * entries(P);
+        p.moments = p.sets * (total - T.first[T.low]) * 2 * entries(P);
         if (p.moments <= limit) break;
     }
     if (T.low >= T.levels) return TreePlan();
     T.run = KEM_TREE_LEAF;
     for (int k = 0; k < T.low; k++) T.run *= KEM_TREE_FAN;
-    p.per_lane = npts >= kTreePairPoints ? 2 : 1;
+    p.per_lane = !multi && npts >= kTreePairPoints ? 2 : 1;
     const int64_t groups = (npts + 64 * p.per_lane - 1) / (64 * p.per_lane);
     int64_t slices =
         std::min<int64_t>(kTreeMaxSlices, std::max<int64_t>(1, kTreeWavefronts / (kTreeWaves * groups)));
-    if (npts <= kTreeSmallPoints) slices = std::min(slices, kTreeSmallPartials / (4 * npts));
+    if (!multi && npts <= kTreeSmallPoints) slices = std::min(slices, kTreeSmallPartials / (4 * npts));
     p.slices = (int)slices;
     const int64_t unit = 64 * p.per_lane;
     p.chunk = std::min(npts, kTreePartialDoubles / (4 * slices) / unit * unit);
     p.partials = 4 * slices * p.chunk;
-    p.ranges = (p.chunk + unit - 1) / unit * (p.per_lane == 2 ? sizeof(Ranges<2>) : sizeof(Ranges<1>)) / sizeof(double);
+    p.ranges = (p.chunk + unit - 1) / unit * (multi ? sizeof(Ranges<1, true>) : p.per_lane == 2 ? sizeof(Ranges<2, false>) : sizeof(Ranges<1, false>)) /
+               sizeof(double);
     p.use = true;
     return p;
 }
 
 hipError_t launch_tree(hipStream_t st, const FieldMesh& m, const TreePlan& p, bool mixed, const double* sigma,
-                       const double* px, const double* py, const double* pz, int64_t npts, double* mom, double* ranges,
-                       double* out, bool moments)
+                       const int32_t* pset, const double* px, const double* py, const double* pz, int64_t npts,
+                       double* mom, double* ranges, double* out, bool moments)
 {
     if (npts <= 0) return hipSuccess;
-    return mixed ? tree_passes<true>(st, m, p, sigma, px, py, pz, npts, mom, ranges, out, moments)
-                 : tree_passes<false>(st, m, p, sigma, px, py, pz, npts, mom, ranges, out, moments);
+    return mixed ? tree_passes<true>(st, m, p, sigma, pset, px, py, pz, npts, mom, ranges, out, moments)
+                 : tree_passes<false>(st, m, p, sigma, pset, px, py, pz, npts, mom, ranges, out, moments);
 }
 
 }  // namespace kem
