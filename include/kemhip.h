@@ -380,7 +380,7 @@ int kem_cache_find(const char* directory, int64_t n, const int32_t* shape_type, 
                    int64_t file_cap);
 
 /* Y = A X for nrhs vectors (host, column-major n x nrhs): KSquareMatrix::Multiply
-   (KMatrix.hh:92-111) over a block; KEM_MIXED uses the FP32 matrix on FP32 MFMA, KEM_MIXED_BF16
+   (KMatrix.hh:92-111) over a block; KEM_MIXED uses the FP32 matrix on the matrix cores, KEM_MIXED_BF16
    the BF16 matrix on BF16 MFMA (X rounded to BF16, FP32 accumulation, FP64 sum of the split-K
    partials). */
 int kem_matrix_multiply_batch(kem_matrix* A, int precision, int64_t nrhs, const double* X, double* Y);

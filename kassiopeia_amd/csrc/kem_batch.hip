@@ -300,20 +300,73 @@ __device__ __forceinline__ void wait_vmcnt()
 }
 
 constexpr int kStreamRows = 256;  // rows per workgroup
-constexpr int kStreamKC = 16;     // FP32: matrix columns per chunk (3 buffers: 60 KB of LDS)
 constexpr int kStreamG = 4;       // BF16: column groups of 8 per chunk (3 buffers: 60 KB)
 
-// FP32 matrix (n % 4 == 0, A and Vt 16-byte aligned), KP = 64.  Chunk: KC columns x 256 rows
-// of A (one 1 KB load per column: lane l takes rows 4l .. 4l + 3) and KC panel rows (4 per 1 KB
-// load).  Splits start at multiples of KC columns.
-__global__ __launch_bounds__(kBlock) void k_bmm32s(const float* __restrict__ A, int64_t n,
-                                                   const float* __restrict__ Vt, int64_t per_split,
-                                                   float* __restrict__ part, const int* __restrict__ skip)
+// FP32 matrix (n % 4 == 0, A and the panel 16-byte aligned), KP = 64.  An FP32 number is three BF16 numbers exactly
+// (8 bits of significand each, cut off, not rounded), and a product of two is nine BF16 products, of which all but
+// low x low (2^-32 of the product) are summed on the BF16 matrix cores: 8 x 32 cycles for 32 x 32 x 16 entries
+// against 8 x 64 on the FP32 ones.  The matrix is split in registers as it passes, the panel once per product.  The
+// matrix cores cut their sums off, which adds up over a long row of one sign (4.5e-6 over 17,568 columns of positive
+// terms), so runs of kSplitRun chunks are added to sums of their own: against 64-bit sums 1,280 to 17,568 columns
+// give 3e-9 to 6e-9 of the sum of magnitudes for terms of random sign and 3.1e-8 to 4.7e-8 for positive ones, FP32
+// matrix cores 8e-9 to 1.5e-8 and 6e-8 to 2.8e-7.  Between the stream of the matrix (0.28 ms at 5.7 TB/s for 20,000 rows) and
+// the matrix cores and the splitting together (0.25 ms): 0.39 ms for 64 right-hand sides, 0.54 ms on FP32 cores.
+constexpr int kSplitChunk = 16;                      // columns of the matrix per chunk (one MFMA's)
+constexpr int kSplitRun = 4;                         // chunks summed on the matrix cores at a time
+constexpr int kSplitPanel = 3 * 2 * 64;              // 16-byte operands of a chunk's panel rows
+
+// the three parts of eight FP32 numbers as MFMA operands
+__device__ __forceinline__ void split8(const float (&v)[8], bf8v (&o)[3])
+{
+    uint32_t w[3][4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        uint32_t h[2], m[2], l[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const float x = v[2 * q + e];
+            h[e] = __float_as_uint(x);
+            const float r = x - __uint_as_float(h[e] & 0xffff0000u);
+            m[e] = __float_as_uint(r);
+            l[e] = __float_as_uint(r - __uint_as_float(m[e] & 0xffff0000u));
+        }
+        w[0][q] = __builtin_amdgcn_perm(h[1], h[0], 0x07060302);
+        w[1][q] = __builtin_amdgcn_perm(m[1], m[0], 0x07060302);
+        w[2][q] = __builtin_amdgcn_perm(l[1], l[0], 0x07060302);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; k++) o[k] = __builtin_bit_cast(bf8v, uint4{w[k][0], w[k][1], w[k][2], w[k][3]});
+}
+
+// the panel's parts in operand order: [chunk][part][tile of 32 columns][lane], rows past n zero.  A block takes two
+// chunks: thread = chunk, tile, lane.
+__global__ __launch_bounds__(kBlock) void k_split_panel(const float* __restrict__ P, int64_t n, int64_t nchunks,
+                                                        bf8v* __restrict__ out, const int* __restrict__ skip)
 {
     if (skip && *skip) return;
-    constexpr int KP = 64, KC = kStreamKC, CH = KC * kStreamRows + KC * KP, NW = KC / 4 + KC / 16;
-    static_assert(KC % 16 == 0, "one panel load per wavefront and chunk");
-    __shared__ float lds[3 * CH];
+    const int64_t c = (int64_t)blockIdx.x * 2 + (threadIdx.x >> 7);
+    if (c >= nchunks) return;
+    const int t = (threadIdx.x >> 6) & 1, lane = threadIdx.x & 63;
+    const int64_t j0 = c * kSplitChunk + 8 * (lane >> 5);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) v[e] = j0 + e < n ? P[(j0 + e) * 64 + 32 * t + (lane & 31)] : 0.f;
+    bf8v o[3];
+    split8(v, o);
+#pragma unroll
+    for (int k = 0; k < 3; k++) out[c * kSplitPanel + (k * 2 + t) * 64 + lane] = o[k];
+}
+
+// Chunk: 16 columns x 256 rows of A (one 1 KB load per column: lane l takes rows 4l .. 4l + 3; the upper eight
+// columns lie 32 banks further, so the two half-wavefronts read different banks) and the panel's six 1 KB loads.
+// Splits start at multiples of a chunk.
+__global__ __launch_bounds__(kBlock, 2) void k_bmm32s(const float* __restrict__ A, int64_t n,
+                                                      const bf8v* __restrict__ V3, int64_t per_split,
+                                                      float* __restrict__ part, const int* __restrict__ skip)
+{
+    if (skip && *skip) return;
+    constexpr int KP = 64, KC = kSplitChunk, AW = KC * kStreamRows + 32, CH = AW + 4 * kSplitPanel, NW = KC / 4 + 2;
+    __shared__ __attribute__((aligned(16))) float lds[3 * CH];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int lr = lane & 31, lk = lane >> 5;
     const int64_t r0 = (int64_t)blockIdx.x * kStreamRows;
@@ -328,23 +381,18 @@ __global__ __launch_bounds__(kBlock) void k_bmm32s(const float* __restrict__ A, 
         const int64_t jc = j0 + k * KC;
         for (int q = 0; q < KC / 4; q++) {
             const int c = wave + 4 * q;
-            const int64_t col = std::min<int64_t>(jc + c, j1 - 1);  // past j1: a valid column, unused
-            __builtin_amdgcn_global_load_lds(A + col * n + rr, buf + c * kStreamRows, 16, 0, 0);
+            const int64_t col = std::min<int64_t>(jc + c, n - 1);  // past n: a valid column against zero panel rows
+            __builtin_amdgcn_global_load_lds(A + col * n + rr, buf + c * kStreamRows + (c >= 8 ? 32 : 0), 16, 0, 0);
         }
-        for (int q = 0; q < KC / 16; q++) {
-            // panel rows jc + 16 q + 4 wave .. + 3; jc and n are multiples of 4, so a group of
-            // rows is either below n or wholly past it (then clamped, unused)
-            const int rb = 16 * q + 4 * wave;
-            const int64_t row = std::min<int64_t>(jc + rb, n - 4);
-            __builtin_amdgcn_global_load_lds(Vt + row * KP + lane * 4, buf + KC * kStreamRows + rb * KP, 16, 0, 0);
+        const bf8v* pv = V3 + (jc / KC) * kSplitPanel;
+        for (int q = 0; q < 2; q++) {
+            const int u = std::min(wave + 4 * q, 5);  // wavefronts 2 and 3 bring the last part again
+            __builtin_amdgcn_global_load_lds(pv + u * 64 + lane, buf + AW + u * 256, 16, 0, 0);
         }
     };
-    f16v acc0[2], acc1[2];
+    f16v acc0[2], acc1[2], sum0[2], sum1[2];
     for (int t = 0; t < 2; t++)
-        for (int v = 0; v < 16; v++) {
-            acc0[t][v] = 0.f;
-            acc1[t][v] = 0.f;
-        }
+        for (int v = 0; v < 16; v++) acc0[t][v] = acc1[t][v] = sum0[t][v] = sum1[t][v] = 0.f;
     issue(0);
     if (nch > 1) issue(1);
     for (int64_t k = 0; k < nch; k++) {
@@ -355,22 +403,41 @@ __global__ __launch_bounds__(kBlock) void k_bmm32s(const float* __restrict__ A, 
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const float* buf = lds + (k % 3) * CH;
-        const int kv = (int)std::min<int64_t>(KC, j1 - (j0 + k * KC));  // valid columns
-        float a0[KC / 2], a1[KC / 2], b[KC / 2][2];
-        for (int p = 0; p < KC / 2; p++) {
-            const int col = 2 * p + lk;
-            a0[p] = buf[col * kStreamRows + wave * 64 + lr];
-            a1[p] = buf[col * kStreamRows + wave * 64 + 32 + lr];
-            b[p][0] = buf[KC * kStreamRows + col * KP + lr];
-            b[p][1] = buf[KC * kStreamRows + col * KP + 32 + lr];
-            if (col >= kv) a0[p] = a1[p] = 0.f;
+        float x0[8], x1[8];
+        bf8v a0[3], a1[3], b[3][2];
+        const float* ab = buf + lk * (8 * kStreamRows + 32) + wave * 64 + lr;
+        for (int e = 0; e < 8; e++) {
+            x0[e] = ab[e * kStreamRows];
+            x1[e] = ab[e * kStreamRows + 32];
         }
+        const bf8v* pb = reinterpret_cast<const bf8v*>(buf + AW) + lane;
+        for (int u = 0; u < 3; u++)
+            for (int t = 0; t < 2; t++) b[u][t] = pb[(2 * u + t) * 64];
         if (k + 2 < nch) issue(k + 2);
-        for (int p = 0; p < KC / 2; p++)
+        split8(x0, a0);
+        split8(x1, a1);
+        // the small products first
+        auto add = [&](int u, int w) {
             for (int t = 0; t < 2; t++) {
-                acc0[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[p], b[p][t], acc0[t], 0, 0, 0);
-                acc1[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[p], b[p][t], acc1[t], 0, 0, 0);
+                acc0[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[u], b[w][t], acc0[t], 0, 0, 0);
+                acc1[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[u], b[w][t], acc1[t], 0, 0, 0);
             }
+        };
+        add(1, 2);
+        add(2, 1);
+        add(0, 2);
+        add(1, 1);
+        add(2, 0);
+        add(0, 1);
+        add(1, 0);
+        add(0, 0);
+        if ((k & (kSplitRun - 1)) == kSplitRun - 1 || k + 1 == nch)
+            for (int t = 0; t < 2; t++)
+                for (int v = 0; v < 16; v++) {
+                    sum0[t][v] += acc0[t][v];
+                    sum1[t][v] += acc1[t][v];
+                    acc0[t][v] = acc1[t][v] = 0.f;
+                }
     }
     const int64_t i0 = r0 + wave * 64;
     if (i0 >= n) return;
@@ -379,8 +446,8 @@ __global__ __launch_bounds__(kBlock) void k_bmm32s(const float* __restrict__ A, 
     for (int t = 0; t < 2; t++)
         for (int v = 0; v < 16; v++) {
             const int rr2 = 8 * (v >> 2) + (v & 3);
-            if (rr2 < lim) out[rr2 * KP + 32 * t] = acc0[t][v];
-            if (rr2 + 32 < lim) out[(rr2 + 32) * KP + 32 * t] = acc1[t][v];
+            if (rr2 < lim) out[rr2 * KP + 32 * t] = sum0[t][v];
+            if (rr2 + 32 < lim) out[(rr2 + 32) * KP + 32 * t] = sum1[t][v];
         }
 }
 
@@ -1070,7 +1137,9 @@ size_t bmm_workspace_bytes(int64_t n, int nrhs, int prec)
         const int64_t tiles = (n + 63) / 64;
         const int s = std::max({bmm_splits(n, tiles), kp == 64 ? bmm_stream_splits(n) : 1,
                                 kp <= 32 && n % 4 == 0 ? bmm_tile_splits(n, kp, 4) : 1});
-        return sizeof(float) * ((size_t)s * n * kp + (size_t)n * kp) + 256;
+        // a panel of 64 columns once more as its BF16 parts
+        const size_t parts = kp == 64 ? (size_t)((n + kSplitChunk - 1) / kSplitChunk) * kSplitPanel * 16 + 256 : 0;
+        return sizeof(float) * ((size_t)s * n * kp + (size_t)n * kp) + parts + 256;
     }
     const int64_t blocks = (n + kBlock - 1) / kBlock;
     const int s = std::max(bmm_splits(n, blocks * 4), n % 2 == 0 ? bmm_tile_splits(n, kp, 8) : 1);
@@ -1121,10 +1190,13 @@ hipError_t launch_bmm(hipStream_t st, const float* A32, const double* A64, int64
             // streamed through LDS; splits start at multiples of the chunk width
             const int ss = bmm_stream_splits(n);
             int64_t pc = (n + ss - 1) / ss;
-            pc = (pc + kStreamKC - 1) / kStreamKC * kStreamKC;
+            pc = (pc + kSplitChunk - 1) / kSplitChunk * kSplitChunk;
             const int nc = (int)((n + pc - 1) / pc);
             dim3 grid((unsigned)((n + kStreamRows - 1) / kStreamRows), (unsigned)nc);
-            k_bmm32s<<<grid, kBlock, 0, st>>>(A32, n, P, pc, part, skip);
+            const int64_t nchunks = (n + kSplitChunk - 1) / kSplitChunk;
+            bf8v* V3 = (bf8v*)(((uintptr_t)(Vt + (size_t)n * 64) + 255) / 256 * 256);
+            k_split_panel<<<(unsigned)((nchunks + 1) / 2), kBlock, 0, st>>>(P, n, nchunks, V3, skip);
+            k_bmm32s<<<grid, kBlock, 0, st>>>(A32, n, V3, pc, part, skip);
             k_bmm32_reduce<64><<<(unsigned)((n + kReduceRows - 1) / kReduceRows), kBlock, 0, st>>>(part, nc, n, nrhs, Y, ldy, skip);
             return hipGetLastError();
         }

@@ -245,8 +245,8 @@ hipError_t launch_pack_bf16(hipStream_t st, const double* A64, const float* A32,
 hipError_t launch_bmm16(hipStream_t st, const uint16_t* A16, int64_t n, const void* X, int64_t ldx, int nrhs,
                         double* Y, int64_t ldy, void* ws, size_t ws_bytes, bool x_is_panel,
                         const int* skip = nullptr);
-// Y[c*ldy + i] = sum_j A(i, j) X(j, c) for c < nrhs <= 64: A32 != null selects the FP32 MFMA
-// product (X rounded to FP32), else the FP64 product with A64.  x_is_panel: X already is the
+// Y[c*ldy + i] = sum_j A(i, j) X(j, c) for c < nrhs <= 64: A32 != null selects the FP32
+// product on the matrix cores (X rounded to FP32), else the FP64 product with A64.  x_is_panel: X already is the
 // row-major panel (FP32: n x (nrhs <= 32 ? 32 : 64) floats; FP64: n x (nrhs <= 16 ? 16 : 64)).
 hipError_t launch_bmm(hipStream_t st, const float* A32, const double* A64, int64_t n, const double* X, int64_t ldx,
                       int nrhs, double* Y, int64_t ldy, void* ws, size_t ws_bytes, bool x_is_panel,

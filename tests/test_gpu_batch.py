@@ -157,6 +157,28 @@ def test_block_product_fp32_mfma(coax, k):
     assert np.all(np.abs(Y - ref) <= 2e-6 * scale)
 
 
+@pytest.mark.parametrize("n", [4, 16, 20, 64, 68, 260, 1280])
+@pytest.mark.parametrize("rhs", ["positive", "wide"])
+def test_block_product_fp32_split(ctx, coax, n, rhs):
+    """33-64 right-hand sides against an FP32 matrix go through three BF16 parts per number: partial and whole chunks of 16
+    columns and runs of 4 chunks; sums of one sign, where the matrix cores' cut-off sums drift, and right-hand sides
+    from 2^-60 to 2^60.  The parts are exact and the products left out 2^-32, so the bound is that of the sums: 32
+    truncations (2^-23) in a run, one rounding (2^-24) per run, one per split, one of the result."""
+    from kassiopeia_amd import kemfield as K
+
+    m = _first_elements(coax[0], n)
+    A = K.KBoundaryIntegralMatrix(K.KSurfaceContainer(ctx, m), fp64=True, fp32=True)
+    A32 = A.to_numpy().astype(np.float32).astype(np.float64)
+    rng = np.random.default_rng(n)
+    X = rng.uniform(0.5, 1.0, size=(n, 40))
+    if rhs == "wide":
+        X *= np.exp2(rng.integers(-60, 61, size=X.shape)) * rng.choice([-1.0, 1.0], size=X.shape)
+    X = X.astype(np.float32).astype(np.float64)
+    Y = A.MultiplyBatch(X, "mixed")
+    bound = (32 + 0.5 * (n / 64 + 8)) * 2.0 ** -23
+    assert np.all(np.abs(Y - A32 @ X) <= bound * (np.abs(A32) @ np.abs(X)))
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_solve_batch_voltage_sets(coax, precision):
     """16 ring groups x 12 voltage sets (U[-1000, 0] V per group): every column converges to
