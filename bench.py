@@ -35,28 +35,11 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-# FLOPs per (point, element) pair for field + potential, by regime (add/sub/mul = 1, FMA = 2,
-# sqrt/div/rsqrt/log/atan2 = 1): cubature 14 + 21 n_q; closed form 260 (convention);
-# segments 14 + 21 n_nodes, analytic 100.  Census order: triangle 7/12/33/closed,
-# rectangle 7/12/33/closed, segment 4/16/analytic, triangle 6-point (FP32 ladder).
-FLOPS_PER_PAIR = np.array([161, 266, 707, 260, 161, 266, 707, 260, 98, 350, 100, 140], dtype=np.float64)
-FAR = np.ones(12)
-FAR[[3, 7, 10]] = 0.0  # the far kernels evaluate every pair but the closed-form ones
 PEAK_FP64_TFLOPS = 78.6  # MI355X FP64 vector peak
-PEAK_FP32_TFLOPS = 157.3  # MI355X FP32 vector peak (published; it needs packed FP32)
 PEAK_HBM_GBS = 8000.0
 # the oracle's per-core field rate over the compiled reference's, measured on one core of the
 # same host type: 3.68 / 2.95 M point-element pairs/s (1,728-triangle cube, 4,096 points)
 CPU_ORACLE_OVER_REFERENCE = 3.68 / 2.95
-
-# HBM bytes per launch of the mixed far kernel on the headline workload, by element-range size
-# (which sets the dispatch: 640 -> 208,384 points x 160 ranges, 2,560 -> 818,176 x 40, 10,240 ->
-# 1,973,760 x 16), from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs scaled by the readings of
-# a 1 GiB device copy (FETCH_SIZE x 1.99990, WRITE_SIZE x 1.0): 640: 0.847 GB read, 1.067 GB
-# written; 2,560: 0.885 / 1.047 GB; 10,240: 0.996 / 1.011 GB (the writes are the partial-sum
-# slices of the ranges).  Source: the profile named here; other sizes not measured (null).
-TRAFFIC = {"bytes": {640: 1.914e9, 2560: 1.932e9, 10240: 2.006e9},
-           "profile": "profiles/pmc_traffic_k_field_far32c_bore100k_10Mpts.md"}
 
 METRIC = "point-element field evals/s + solve time, mixed vs FP64 at 1e-6 rel. error"
 
@@ -184,30 +167,6 @@ def _kernel_time(ctx):
     return kt.value, kn.value
 
 
-def _plan(ctx, n, npts, range_elems, precision):
-    out = (ctypes.c_int64 * 8)()
-    ctx.check(ctx.lib.kem_field_plan(0, 1, precision, 0, n, 1, npts, range_elems, -1, out))
-    return {"ranges": out[3], "slices": out[4], "chunk": out[5], "xcd": out[6]}
-
-
-# FLOPs per pair of each path of the mixed cluster far pass (kem_field_census_paths order):
-# 3-point cluster pairs, 6-point record pairs, per-pair path by the pair's own rule (6, 7, 12,
-# 33 points; segments 4, 16 nodes); near pairs belong to the near pass
-FLOPS_PER_PATH = np.array([14 + 21 * 3, 140, 140, 161, 266, 707, 98, 350, 0, 0], dtype=np.float64)
-
-
-def _census_paths(ctx, cont, X, m):
-    """pairs per path of the mixed cluster far pass, in the order the pass visits the points;
-    returns (counts, algorithmic FLOPs = each pair at the rule its path evaluates (per-pair
-    pairs at their own rule), executed FLOPs (the per-pair path at its wavefront rule))"""
-    c = (ctypes.c_int64 * 10)()
-    ctx.check(ctx.lib.kem_field_census_paths(ctx.h, cont.h, m, X[0].ptr, X[1].ptr, X[2].ptr, c))
-    c = np.array(c[:], dtype=np.float64)
-    alg = float((c * FLOPS_PER_PATH).sum())
-    executed = float(c[0] * FLOPS_PER_PATH[0] + c[1] * FLOPS_PER_PATH[1] + 14.0 * c[2:8].sum() + 21.0 * c[9])
-    return c, alg, executed
-
-
 # FLOPs of one collocation entry (Dirichlet row: potential only) by regime, census order
 # (triangle 7/12/33/closed, rectangle 7/12/33/closed, segment 4/16/analytic, unused)
 ASM_FLOPS = np.array([95, 155, 407, 200, 95, 155, 407, 200, 59, 203, 100, 0], dtype=np.float64)
@@ -303,9 +262,8 @@ def field_only(ctx, args):
         ctx.sync()
         times.append(time.perf_counter() - t0)
     rng_used = T.get(ctx, "far_range_" + args.field_only)
-    plan = _plan(ctx, N, M, rng_used, prec)
     print(json.dumps({"field_only": args.field_only, "elements": N, "points": M, "pass_s": times,
-                      "far_range": rng_used, "plan": plan}), flush=True)
+                      "far_range": rng_used}), flush=True)
     for a in X + O + [S]:
         a.close()
     cont.close()
@@ -332,10 +290,7 @@ def run_bore(ctx, args):
         t0 = time.perf_counter()
         sig0 = np.full(N, 1e-9)  # the time per pair does not depend on the charge densities
         sample = pts[:min(args.tune_points, M)] if args.tune_points > 0 else pts
-        # the same candidates for both precisions, on the whole point set: the chunking of the
-        # per-XCD element ranges depends on the point count (10 M points, s per pass: mixed
-        # {640: 2.10, 1280: 2.13, 2560: 2.14, 5120: 2.19, 10240: 2.19}, FP64 {640: 9.67,
-        # 1280: 9.70, 2560: 9.85, 5120: 9.98, 10240: 10.16})
+        # the ranges of the flat far passes; a hierarchical pass (this size) does not depend on them
         cands = (640, 2560, 10240)
         tuning = {"far_range_mixed": T.tune_field(cont, sig0, sample, "mixed", repeats=1, candidates=cands),
                   "far_range_fp64": T.tune_field(cont, sig0, sample, "fp64", repeats=1, candidates=cands)}
@@ -431,16 +386,19 @@ def run_bore(ctx, args):
                mixed_err_phi_max_over_V=err["phi_max_over_V"], mixed_err_E_pointwise_p99=err["E_pointwise_p99"],
                mixed_within_1e6=mixed_ok)
 
-    # ------------------------------------------------------------ roofline of the mixed far kernel
-    prec_mx = _lib.KEM_MIXED
-    cmx, far_flops, far_flops_executed = _census_paths(ctx, cont, X, M)
+    # ------------------------------------------------------------ roofline of the step's dominant kernel
+    # the FP32 matrix-vector product of the inner solves: its time from the HIP events of the tuning sweep on this
+    # matrix, else the solve's time per product (an upper bound that holds the projections too)
     far_ms = float(np.mean([s["far_ms"] / max(s["far_regions"], 1) for s in steps]))
-    rng_used = T.get(ctx, "far_range_mixed")
-    plan = _plan(ctx, N, M, rng_used, prec_mx)
-    launches = -(-M // plan["chunk"]) if plan["xcd"] else 1
-    achieved = far_flops / (far_ms * 1e-3) / 1e12
-    log(f"far kernel (mixed): {far_ms:.1f} ms per pass in {launches} launches, census {far_flops:.3e} FLOP "
-        f"-> {achieved:.1f} TFLOP/s; pairs by regime {cmx.astype(int).tolist()}")
+    log(f"field pass (mixed): kernels up to the partial sums {far_ms:.1f} ms, pass {pm['field'] * 1e3:.1f} ms")
+    mv_ms = pm["solve"] * 1e3 / max(pm["iterations"], 1)
+    mv_source = "solve time / iterations"
+    if tuning is not None:
+        mv_ms = float(tuning["gemv_blocks_fp32"]["ms"][tuning["gemv_blocks_fp32"]["best"]])
+        mv_source = "HIP events"
+    achieved = 4.0 * N * N / (mv_ms * 1e-3) / 1e9
+    log(f"FP32 matrix-vector product: {mv_ms:.2f} ms = {achieved:.0f} GB/s ({mv_source})")
+    out.update(field_kernels_ms_mixed=far_ms)
 
     # ------------------------------------------------------------ the assembly kernels' roofline
     asm_ms = pm["asm_ms"]
@@ -490,7 +448,7 @@ def run_bore(ctx, args):
         out.update(mixed_field_only_err_E_l2=ef["E_l2"], mixed_field_only_err_E_max_over_rms=ef["E_max_over_rms"],
                    mixed_solve_only_err_E_l2=es["E_l2"], mixed_solve_only_err_E_max_over_rms=es["E_max_over_rms"],
                    sigma_mixed_vs_fp64=float(np.linalg.norm(pm["sigma"] - sig64) / np.linalg.norm(sig64)))
-        # 16 voltage sets in lockstep (mixed: FP32 MFMA block products, FP64 refinement)
+        # 16 voltage sets in lockstep (mixed: FP32 block products, FP64 refinement)
         groups = mesh.group
         V16 = rng.uniform(-20000.0, 0.0, size=(33, 16))
         V16[32, :] = 0.0
@@ -584,22 +542,12 @@ def run_bore(ctx, args):
                                f"(FP32 inner solves, FP64 refinement), FP32-far-field pass; value = field "
                                f"pairs per second of the whole step",
                    "elements": N, "points": M, "gmres_tolerance": 1e-10},
-        # the far kernel is bound by the vector ALU (no matrix-shaped work): achieved = census
-        # FLOPs of its pairs (the pairs of each regime x 14 + 21 n_q) / its time from HIP events
-        # on the library's stream over the timed steps; one pass is `launches` dispatches (chunks
-        # of points), so this equals FLOPs per dispatch / average dispatch duration
-        "roofline": {"bound": "valu", "compute": "vector ALU, fp32 (unpacked)", "achieved": achieved,
-                     "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s", "frac": achieved / PEAK_FP32_TFLOPS,
-                     "traffic": TRAFFIC["bytes"].get(rng_used) if (N == 100_000 and M == 10_000_000) else None,
-                     "traffic_unit": "HBM bytes per dispatch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-calibrated)",
-                     "traffic_source": TRAFFIC["profile"], "kernel": "k_field_far32c", "kernel_ms_per_pass": far_ms,
-                     "launches_per_pass": launches, "kernel_ms_per_launch": far_ms / launches,
-                     "flops_per_pass": far_flops, "frac_of_unpacked_fp32_peak": achieved / PEAK_FP64_TFLOPS,
-                     "flops_executed_per_pass": far_flops_executed,
-                     "pairs_by_path": cmx.astype(int).tolist(),
-                     "pairs_by_path_keys": ["3-point cluster", "6-point record", "per-pair 6", "per-pair 7",
-                                            "per-pair 12", "per-pair 33", "segment 4", "segment 16", "near",
-                                            "per-pair nodes executed"]},
+        # the step's largest part is the GMRES solve, and that is the stream of the FP32 matrix; the field pass is
+        # hierarchical, so its time is not pairs times a cost per pair
+        "roofline": {"bound": "hbm", "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
+                     "frac": achieved / PEAK_HBM_GBS, "kernel": "k_gemv_part_vec<float, 2>", "kernel_ms": mv_ms,
+                     "kernel_ms_source": mv_source, "bytes_per_launch": 4.0 * N * N,
+                     "launches_per_step": pm["iterations"], "share_of_step": mv_ms * pm["iterations"] / (t_step * 1e3)},
         "cpu_baseline": cpu,
         "tuning": None if tuning is None else {k: v["best"] for k, v in tuning.items()},
     }
@@ -671,19 +619,15 @@ def run_coax(ctx, args):
 
     ms64, kms64 = timed(_lib.KEM_FP64, O, 2)
     msmx, kmsmx = timed(_lib.KEM_MIXED, Om, 5)
-    c64 = _census(ctx, cont, X, M, _lib.KEM_FP64)
-    f64 = float((c64 * FLOPS_PER_PAIR * FAR).sum())
-    _, fmx, _ = _census_paths(ctx, cont, X, M)
     phi = O[0].get()
     E = np.stack([O[k].get() for k in (1, 2, 3)], 1)
     err = _errors(E, phi, np.stack([Om[k].get() for k in (1, 2, 3)], 1), Om[0].get(), 18600.0)
-    log(f"coax20k field: fp64 {ms64:.1f} ms (far {kms64:.1f} ms, {f64 / kms64 / 1e9:.1f} TFLOP/s), mixed "
-        f"{msmx:.2f} ms (far {kmsmx:.2f} ms, {fmx / kmsmx / 1e9:.1f} TFLOP/s), {ms64 / msmx:.2f}x; error "
+    log(f"coax20k field: fp64 {ms64:.1f} ms (kernels {kms64:.1f} ms), mixed "
+        f"{msmx:.2f} ms (kernels {kmsmx:.2f} ms), {ms64 / msmx:.2f}x; error "
         f"l2 {err['E_l2']:.1e} max/rms {err['E_max_over_rms']:.1e} phi/V {err['phi_max_over_V']:.1e}")
     out.update(coax20k_field_ms_fp64=ms64, coax20k_field_ms_mixed=msmx,
                coax20k_pairs_per_s_mixed=N * M / msmx * 1e3, coax20k_pairs_per_s_fp64=N * M / ms64 * 1e3,
-               coax20k_field_speedup=ms64 / msmx, coax20k_far_frac_fp64=f64 / kms64 / 1e9 / PEAK_FP64_TFLOPS,
-               coax20k_far_frac_mixed=fmx / kmsmx / 1e9 / PEAK_FP32_TFLOPS, coax20k_mixed_err_E_l2=err["E_l2"],
+               coax20k_field_speedup=ms64 / msmx, coax20k_mixed_err_E_l2=err["E_l2"],
                coax20k_mixed_err_E_max_over_rms=err["E_max_over_rms"],
                coax20k_mixed_err_phi_max_over_V=err["phi_max_over_V"],
                coax20k_pipeline_speedup=(t_asm + st64.seconds + ms64 * 1e-3) / (t_asm + stmx.seconds + msmx * 1e-3))

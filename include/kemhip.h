@@ -112,7 +112,8 @@ int kem_ctx_set_mixed_fp64_ratio(kem_ctx* ctx, double ratio);
 /* Launch tuning (no reference counterpart; kassiopeia_amd/autotune.py measures and sets them):
    KEM_TUNE_FAR_RANGE_FP64 / _MIXED = elements per element range of the far pass over 262,144
    or more points of one charge-density set; the elements split into 8 R ranges, R per XCD, so
-   each XCD's range stays in its L2 (0: no split; default 2560).  KEM_TUNE_GEMV_BLOCKS /
+   each XCD's range stays in its L2 (0: no split; default 2560).  It shapes the flat passes only, not the
+   hierarchical pass that serves most calls of this size.  KEM_TUNE_GEMV_BLOCKS /
    KEM_TUNE_BMM_BLOCKS = target block counts of the split-K matrix-vector product (default 2048)
    and of the register-loaded multi-RHS block products in 64-row tiles times column splits
    (FP32 with n % 4 != 0, FP64 with n odd; default 2560);
@@ -260,9 +261,9 @@ int kem_field_eval_sets(kem_ctx* ctx, const kem_mesh* mesh, int64_t nsets, const
 int kem_field_census(kem_ctx* ctx, const kem_mesh* mesh, int64_t npts, const double* d_x, const double* d_y,
                      const double* d_z, int precision, int64_t* counts);
 
-/* Instrumentation (no reference counterpart): the paths of the mixed-precision cluster far
-   pass (single charge-density set, numeric policy) over device points, visited in the order a
-   kem_field_eval_device pass of the same points visits them.  counts[10] = (point, element)
+/* Instrumentation (no reference counterpart): the paths of the flat mixed-precision cluster far
+   pass (single charge-density set, numeric policy) over device points, visited in the order of the
+   space-filling curve.  Calls that the hierarchical pass serves do not evaluate these pairs one by one.  counts[10] = (point, element)
    pairs on the 3-point cluster path, on the 6-point record path, on the per-pair path by the
    rule each pair's own ladder picks (6, 7, 12, 33 points; segments 4, 16 nodes), near pairs
    left to the near pass, and the node evaluations the per-pair path runs (its wavefront rule
@@ -270,7 +271,7 @@ int kem_field_census(kem_ctx* ctx, const kem_mesh* mesh, int64_t npts, const dou
 int kem_field_census_paths(kem_ctx* ctx, const kem_mesh* mesh, int64_t npts, const double* d_x, const double* d_y,
                            const double* d_z, int64_t* counts);
 
-/* Instrumentation (no reference counterpart; host arithmetic only, no device access): how a
+/* Instrumentation (no reference counterpart; host arithmetic only, no device access): how the flat passes of a
    field evaluation of npts points over nelem elements splits into element ranges and partial
    sums, for a mesh with (clustered = 1: triangles / rectangles / segments, numeric policy) or
    without element clusters, at a precision, with per-point set indices (multi = 1, as
