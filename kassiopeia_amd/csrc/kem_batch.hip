@@ -308,11 +308,13 @@ constexpr int kStreamG = 4;       // BF16: column groups of 8 per chunk (3 buffe
 // against 8 x 64 on the FP32 ones.  The matrix is split in registers as it passes, the panel once per product.  The
 // matrix cores cut their sums off, which adds up over a long row of one sign (4.5e-6 over 17,568 columns of positive
 // terms), so runs of kSplitRun chunks are added to sums of their own: against 64-bit sums 1,280 to 17,568 columns
-// give 3e-9 to 6e-9 of the sum of magnitudes for terms of random sign and 3.1e-8 to 4.7e-8 for positive ones, FP32
+// give 3e-9 to 9e-9 of the sum of magnitudes for terms of random sign and 4e-8 to 6e-8 for positive ones, FP32
 // matrix cores 8e-9 to 1.5e-8 and 6e-8 to 2.8e-7.  Between the stream of the matrix (0.28 ms at 5.7 TB/s for 20,000 rows) and
-// the matrix cores and the splitting together (0.25 ms): 0.39 ms for 64 right-hand sides, 0.54 ms on FP32 cores.
+// the matrix cores and the splitting together (0.25 ms): 0.36 ms for 64 right-hand sides (4.5 TB/s), 0.54 ms on FP32
+// cores.  Half of a chunk's splitting is put between matrix instructions (0.40 ms with all of it before them, sums every
+// four chunks and 64-bit address arithmetic per lane).
 constexpr int kSplitChunk = 16;                      // columns of the matrix per chunk (one MFMA's)
-constexpr int kSplitRun = 4;                         // chunks summed on the matrix cores at a time
+constexpr int kSplitRun = 8;                         // chunks summed on the matrix cores at a time
 constexpr int kSplitPanel = 3 * 2 * 64;              // 16-byte operands of a chunk's panel rows
 
 // the three parts of eight FP32 numbers as MFMA operands
@@ -367,7 +369,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_bmm32s(const float* __restrict__ 
     if (skip && *skip) return;
     constexpr int KP = 64, KC = kSplitChunk, AW = KC * kStreamRows + 32, CH = AW + 4 * kSplitPanel, NW = KC / 4 + 2;
     __shared__ __attribute__((aligned(16))) float lds[3 * CH];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 31, lk = lane >> 5;
     const int64_t r0 = (int64_t)blockIdx.x * kStreamRows;
     const int64_t j0 = (int64_t)blockIdx.y * per_split;
@@ -375,69 +377,79 @@ __global__ __launch_bounds__(kBlock, 2) void k_bmm32s(const float* __restrict__ 
     if (j0 >= j1) return;
     const int64_t nch = (j1 - j0 + KC - 1) / KC;
     // this lane's 4 rows of a column (rows past n read the last 4 rows; never stored)
-    const int64_t rr = std::min<int64_t>(r0 + 4 * lane, n - 4);
-    auto issue = [&](int64_t k) {
-        float* buf = lds + (k % 3) * CH;
+    const uint32_t rr = (uint32_t)std::min<int64_t>(r0 + 4 * lane, n - 4);
+    auto issue = [&](int64_t k, int slot) {
+        float* buf = lds + slot * CH;
         const int64_t jc = j0 + k * KC;
         for (int q = 0; q < KC / 4; q++) {
             const int c = wave + 4 * q;
             const int64_t col = std::min<int64_t>(jc + c, n - 1);  // past n: a valid column against zero panel rows
-            __builtin_amdgcn_global_load_lds(A + col * n + rr, buf + c * kStreamRows + (c >= 8 ? 32 : 0), 16, 0, 0);
+            const float* column = A + col * n;
+            __builtin_amdgcn_global_load_lds(column + rr, buf + c * kStreamRows + (c >= 8 ? 32 : 0), 16, 0, 0);
         }
         const bf8v* pv = V3 + (jc / KC) * kSplitPanel;
         for (int q = 0; q < 2; q++) {
             const int u = std::min(wave + 4 * q, 5);  // wavefronts 2 and 3 bring the last part again
-            __builtin_amdgcn_global_load_lds(pv + u * 64 + lane, buf + AW + u * 256, 16, 0, 0);
+            const bf8v* piece = pv + u * 64;
+            __builtin_amdgcn_global_load_lds(piece + (uint32_t)lane, buf + AW + u * 256, 16, 0, 0);
         }
     };
     f16v acc0[2], acc1[2], sum0[2], sum1[2];
     for (int t = 0; t < 2; t++)
-        for (int v = 0; v < 16; v++) acc0[t][v] = acc1[t][v] = sum0[t][v] = sum1[t][v] = 0.f;
-    issue(0);
-    if (nch > 1) issue(1);
-    for (int64_t k = 0; k < nch; k++) {
-        if (k + 1 < nch)
-            wait_vmcnt<NW>();
-        else
-            wait_vmcnt<0>();
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const float* buf = lds + (k % 3) * CH;
-        float x0[8], x1[8];
-        bf8v a0[3], a1[3], b[3][2];
-        const float* ab = buf + lk * (8 * kStreamRows + 32) + wave * 64 + lr;
-        for (int e = 0; e < 8; e++) {
-            x0[e] = ab[e * kStreamRows];
-            x1[e] = ab[e * kStreamRows + 32];
-        }
-        const bf8v* pb = reinterpret_cast<const bf8v*>(buf + AW) + lane;
-        for (int u = 0; u < 3; u++)
-            for (int t = 0; t < 2; t++) b[u][t] = pb[(2 * u + t) * 64];
-        if (k + 2 < nch) issue(k + 2);
-        split8(x0, a0);
-        split8(x1, a1);
-        // the small products first
-        auto add = [&](int u, int w) {
-            for (int t = 0; t < 2; t++) {
-                acc0[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[u], b[w][t], acc0[t], 0, 0, 0);
-                acc1[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[u], b[w][t], acc1[t], 0, 0, 0);
+        for (int v = 0; v < 16; v++) sum0[t][v] = sum1[t][v] = 0.f;
+    issue(0, 0);
+    if (nch > 1) issue(1, 1);
+    int slot = 0;
+    for (int64_t k0 = 0; k0 < nch; k0 += kSplitRun) {
+        for (int t = 0; t < 2; t++)
+            for (int v = 0; v < 16; v++) acc0[t][v] = acc1[t][v] = 0.f;
+        const int64_t ke = std::min<int64_t>(nch, k0 + kSplitRun);
+#pragma unroll 1
+        for (int64_t k = k0; k < ke; k++) {
+            if (k + 1 < nch)
+                wait_vmcnt<NW>();
+            else
+                wait_vmcnt<0>();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const float* buf = lds + slot * CH;
+            float x0[8], x1[8];
+            bf8v a0[3], a1[3], b[3][2];
+            const float* ab = buf + lk * (8 * kStreamRows + 32) + wave * 64 + lr;
+            for (int e = 0; e < 8; e++) {
+                x0[e] = ab[e * kStreamRows];
+                x1[e] = ab[e * kStreamRows + 32];
             }
-        };
-        add(1, 2);
-        add(2, 1);
-        add(0, 2);
-        add(1, 1);
-        add(2, 0);
-        add(0, 1);
-        add(1, 0);
-        add(0, 0);
-        if ((k & (kSplitRun - 1)) == kSplitRun - 1 || k + 1 == nch)
-            for (int t = 0; t < 2; t++)
-                for (int v = 0; v < 16; v++) {
-                    sum0[t][v] += acc0[t][v];
-                    sum1[t][v] += acc1[t][v];
-                    acc0[t][v] = acc1[t][v] = 0.f;
-                }
+            const bf8v* pb = reinterpret_cast<const bf8v*>(buf + AW) + lane;
+            for (int u = 0; u < 3; u++)
+                for (int t = 0; t < 2; t++) b[u][t] = pb[(2 * u + t) * 64];
+            if (k + 2 < nch) issue(k + 2, slot == 0 ? 2 : slot - 1);
+            slot = slot == 2 ? 0 : slot + 1;
+            split8(x0, a0);
+            split8(x1, a1);
+            // the small products first; the second tile's splitting goes between the first one's products
+            constexpr int kOf[8][2] = {{1, 2}, {2, 1}, {0, 2}, {1, 1}, {2, 0}, {0, 1}, {1, 0}, {0, 0}};
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                for (int t = 0; t < 2; t++)
+                    acc0[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a0[kOf[q][0]], b[kOf[q][1]][t], acc0[t], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < 8; q++)
+                for (int t = 0; t < 2; t++)
+                    acc1[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1[kOf[q][0]], b[kOf[q][1]][t], acc1[t], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 44, 0);
+#pragma unroll
+            for (int q = 0; q < 16; q++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
+        }
+        for (int t = 0; t < 2; t++)
+            for (int v = 0; v < 16; v++) {
+                sum0[t][v] += acc0[t][v];
+                sum1[t][v] += acc1[t][v];
+            }
     }
     const int64_t i0 = r0 + wave * 64;
     if (i0 >= n) return;
