@@ -199,6 +199,23 @@ def test_solve_batch_voltage_sets(coax, precision):
         assert st.refinements >= 2
 
 
+@pytest.mark.parametrize("n", [63, 64, 132, 1280])
+@pytest.mark.parametrize("k", [2, 17, 33, 64])
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "bf16"])
+def test_solve_batch_rows(ctx, coax, n, k, precision):
+    """The lockstep step's normalisation turns 64 rows of every right-hand side at a time into the panel: whole and partial
+    row blocks, every panel width and storage; each solution meets the tolerance it was solved to (twice, for the
+    residual's own rounding) and right-hand sides that differ get solutions of their own."""
+    from kassiopeia_amd import kemfield as K
+
+    m = _first_elements(coax[0], n)
+    A = K.KBoundaryIntegralMatrix(K.KSurfaceContainer(ctx, m), fp64=True, fp32=True, bf16=precision == "bf16")
+    Ah = A.to_numpy()
+    B = np.random.default_rng(n + k).uniform(0.5, 1.0, size=(n, k)) * np.linspace(1.0, 1000.0, k)
+    X, res, st, _ = A.solve_batch(B, tolerance=1e-9, precision=precision)
+    assert np.all(np.linalg.norm(Ah @ X - B, axis=0) <= 2e-9 * np.linalg.norm(B, axis=0))
+
+
 def test_solve_batch_more_than_64(coax):
     """Groups of 64 right-hand sides; zero columns stay zero; initial guesses are used."""
     m, cont, A, Ah = coax
