@@ -265,21 +265,22 @@ __device__ __forceinline__ double wave_sum(double v)
 
 // ------------------------------------------------------------------ field term
 // Far pairs of the field term: partV[s][j][10] = (sum_k g_k G_kj, sum_k g_k sigma_j dG_kj/dv) over the points of
-// split s.  Lane = element; the four wavefronts of a block share 64 elements and take 64 points of the split at a
-// time.  The sums over points are linear in the nodes' own sums A_q = sum_k g_k / R_kq and B_q = sum_k g_k r_kq /
+// split s.  Lane = element; the four wavefronts of a block share 64 elements and take chunk <= 64 points of the split at
+// a time.  The sums over points are linear in the nodes' own sums A_q = sum_k g_k / R_kq and B_q = sum_k g_k r_kq /
 // R_kq^3, so a wavefront runs over the points inside and over the nodes outside: a pair costs 22 operations a
 // node, and the node's position and the nine derivatives are formed once per 64 points.  Bound by FP64 issue: 1.24 ms
 // for 5,000 elements and 10,000 points, 2.36 ms with the nodes inside (36 operations a node and each lane its own
 // rule).  All lanes take the rule with the most nodes that any of them needs for a point, as in the assembly; the
 // points are put in LDS by rule.  Near pairs are left out, and near[group * splits + s] says whether there were any,
-// so that k_vjp_field_near passes over the others (28 us where there are none, 230 us with its own test of each pair).
+// so that k_vjp_field_near passes over the others (32 us where there are few, 230 us with its own test of each pair).
 constexpr int kVjpWaves = 4;
 __global__ __launch_bounds__(64 * kVjpWaves) void k_vjp_field_far(const double* __restrict__ geom,
                                                                   const double* __restrict__ sigma,
                                                                   const double* __restrict__ rule, int64_t n,
                                                                   const double* __restrict__ pts,
                                                                   const double* __restrict__ gk, int64_t npts,
-                                                                  int64_t per_split, double* __restrict__ partV,
+                                                                  int64_t per_split, int chunk,
+                                                                  double* __restrict__ partV,
                                                                   int* __restrict__ near)
 {
     __shared__ double4 lp[kVjpWaves][64];
@@ -303,8 +304,8 @@ __global__ __launch_bounds__(64 * kVjpWaves) void k_vjp_field_far(const double* 
     int* K = lk[wv];
     double S = 0., F[3][3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
     bool any_near = false;
-    for (int64_t c0 = k0 + 64 * wv; c0 < k1; c0 += 64 * kVjpWaves) {
-        const int cnt = (int)std::min<int64_t>(64, k1 - c0);
+    for (int64_t c0 = k0 + chunk * wv; c0 < k1; c0 += chunk * kVjpWaves) {
+        const int cnt = (int)std::min<int64_t>(chunk, k1 - c0);
         const int64_t kl = c0 + std::min(lane, cnt - 1);
         const double4 mine{pts[3 * kl], pts[3 * kl + 1], pts[3 * kl + 2], gk[kl]};
         // the rule that the wavefront takes for each point (lane k keeps point k's), and the lane's near pairs
@@ -417,28 +418,35 @@ __global__ __launch_bounds__(64 * kVjpWaves) void k_vjp_field_far(const double* 
             out[1 + 3 * m + c] = act ? E.sig * (E.da[m][c] * S + E.pref * F[m][c]) : 0.;
 }
 
-// Near pairs of the field term, added to k_vjp_field_far's sums where it saw any
-__global__ __launch_bounds__(kBlock) void k_vjp_field_near(const double* __restrict__ geom,
-                                                           const double* __restrict__ sigma, int64_t n,
-                                                           const double* __restrict__ pts,
-                                                           const double* __restrict__ gk, int64_t npts,
-                                                           int64_t per_split, double* __restrict__ partV,
-                                                           const int* __restrict__ near)
+// Near pairs of the field term, added to k_vjp_field_far's sums where it saw any.  Each wavefront takes a quarter of the
+// split's points for the block's 64 elements: one closed-form derivative is thousands of operations, so a block's
+// time is that of its longest run of them.
+__global__ __launch_bounds__(64 * kVjpWaves) void k_vjp_field_near(const double* __restrict__ geom,
+                                                                   const double* __restrict__ sigma, int64_t n,
+                                                                   const double* __restrict__ pts,
+                                                                   const double* __restrict__ gk, int64_t npts,
+                                                                   int64_t per_split, double* __restrict__ partV,
+                                                                   const int* __restrict__ near)
 {
-    const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-    if (j >= n || !near[(j >> 6) * gridDim.y + blockIdx.y]) return;
+    if (!near[(int64_t)blockIdx.x * gridDim.y + blockIdx.y]) return;
+    __shared__ double part[kVjpWaves - 1][10][64];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int64_t j = (int64_t)blockIdx.x * 64 + lane;
+    const bool live = j < n;
+    if (!live) j = n - 1;
     const double* g = geom + j * KG_STRIDE;
     Elem E;
     load_elem(g, sigma[j], E);
-    if (!E.tri) return;
-    const int64_t k0 = (int64_t)blockIdx.y * per_split;
-    const int64_t k1 = std::min<int64_t>(npts, k0 + per_split);
+    const int64_t quarter = (per_split + kVjpWaves - 1) / kVjpWaves;
+    const int64_t end = std::min<int64_t>(npts, (blockIdx.y + 1) * per_split);
+    const int64_t k0 = std::min<int64_t>(end, blockIdx.y * per_split + wv * quarter);
+    const int64_t k1 = std::min<int64_t>(end, k0 + quarter);
     double acc[10];
-    double* out = partV + ((int64_t)blockIdx.y * n + j) * 10;
-    for (int c = 0; c < 10; c++) acc[c] = out[c];
+    for (int c = 0; c < 10; c++) acc[c] = 0.;
     for (int64_t k = k0; k < k1; k++) {
         const double px = pts[3 * k], py = pts[3 * k + 1], pz = pts[3 * k + 2], wk = gk[k];
-        if (tri_regime_field(g, px, py, pz) != 0) continue;
+        if (!live || !E.tri || tri_regime_field(g, px, py, pz) != 0) continue;
         Dual<9> V[3][3], P[3];
         for (int m = 0; m < 3; m++)
             for (int c = 0; c < 3; c++) {
@@ -453,7 +461,16 @@ __global__ __launch_bounds__(kBlock) void k_vjp_field_near(const double* __restr
         const double ws = wk * E.sig;
         for (int c = 0; c < 9; c++) acc[1 + c] += ws * G.d[c];
     }
-    for (int c = 0; c < 10; c++) out[c] = acc[c];
+    if (wv > 0)
+        for (int c = 0; c < 10; c++) part[wv - 1][c][lane] = acc[c];
+    __syncthreads();
+    if (wv > 0 || !live || !E.tri) return;
+    double* out = partV + ((int64_t)blockIdx.y * n + j) * 10;
+    for (int c = 0; c < 10; c++) {
+        double v = out[c] + acc[c];
+        for (int k = 0; k < kVjpWaves - 1; k++) v += part[k][c][lane];
+        out[c] = v;
+    }
 }
 
 // ------------------------------------------------------------------ matrix term
@@ -593,15 +610,22 @@ hipError_t launch_field_vjp(hipStream_t st, const double* geom, const double* si
     if (n <= 0) return hipSuccess;
     if (ws_doubles < vjp_workspace_doubles(n, npts)) return hipErrorInvalidValue;
     const int64_t nbx = nblocks(n), sf = vjp_splits(nbx, npts);
-    // splits of whole rounds of the block's wavefronts (256 points), within the workspace's and 256
-    constexpr int64_t kRound = 64 * kVjpWaves;
-    const int64_t rounds = std::max<int64_t>(1, (npts + kRound - 1) / kRound);
-    const int64_t per = (rounds + sf - 1) / sf * kRound;
+    // Chunks of 64 points a wavefront where that gives kVjpBlocks blocks, down to 4 points below (a node's own work is
+    // about that of two pairs): the closed forms and small calls need the blocks.  Splits within the workspace's.
+    // Calls, us, with a thread per element and 16 to 100 points / so: rings 200 elements x 5,000 points 790 / 591,
+    // coax 5,000 x 20,000 9,069 / 7,290, cube 700 x 10 215 / 186.  Rounds of 256 points a block throughout were
+    // 2.6 times slower than the former on a call of a few hundred elements.
+    constexpr int64_t kVjpBlocks = 2048;
+    const int64_t groups = (n + 63) / 64;
+    int64_t chunk = std::clamp<int64_t>(npts * groups / (kVjpWaves * kVjpBlocks), 4, 64);
+    int64_t per = std::max<int64_t>(kVjpWaves * chunk, (npts + sf - 1) / sf);
+    chunk = std::min<int64_t>(64, (per + kVjpWaves - 1) / kVjpWaves);
+    per = (per + kVjpWaves * chunk - 1) / (kVjpWaves * chunk) * (kVjpWaves * chunk);
     const int ns = (int)std::max<int64_t>(1, (npts + per - 1) / per);
     int* near = reinterpret_cast<int*>(ws + (size_t)sf * n * 10);
-    k_vjp_field_far<<<dim3((unsigned)((n + 63) / 64), (unsigned)ns), kRound, 0, st>>>(geom, sigma, rule, n, pts, gk, npts,
-                                                                                     per, ws, near);
-    k_vjp_field_near<<<dim3((unsigned)nbx, (unsigned)ns), kBlock, 0, st>>>(geom, sigma, n, pts, gk, npts, per, ws, near);
+    const dim3 grid((unsigned)groups, (unsigned)ns);
+    k_vjp_field_far<<<grid, 64 * kVjpWaves, 0, st>>>(geom, sigma, rule, n, pts, gk, npts, per, (int)chunk, ws, near);
+    k_vjp_field_near<<<grid, 64 * kVjpWaves, 0, st>>>(geom, sigma, n, pts, gk, npts, per, ws, near);
     k_vjp_reduce_v<<<dim3((unsigned)nbx, 10), kBlock, 0, st>>>(ws, ns, n, dsig, dvert);
     return hipGetLastError();
 }

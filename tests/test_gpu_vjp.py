@@ -47,3 +47,25 @@ def test_field_vjp_splits(ctx, n, npts):
     assert np.abs(ds - rs).max() <= 1e-13 * np.abs(rs).max()
     assert np.abs(dv - rv).max() <= 1e-12 * np.abs(rv).max()
     cont.close()
+
+
+def test_field_vjp_chunks(ctx):
+    """Enough pairs for chunks of 64 points, and a ragged last one, against batches of 125 points (chunks of a few)."""
+    from kassiopeia_amd import kemfield as K
+
+    m = G.cube_mesh(21)  # 5,292 triangles of 0.05: sizes about 0.06
+    cont = K.KSurfaceContainer(ctx, m)
+    rng = np.random.default_rng(11)
+    npts = 7013
+    sigma = rng.uniform(0.5, 1.0, size=m.n) * 1e-9
+    pts = np.concatenate([G.points_shell(npts, a, b, npts) for a, b in ((0.45, 0.9), (0.9, 3.0), (3.0, 20.0))])
+    pts = pts[rng.permutation(len(pts))[:npts]]
+    g = rng.uniform(0.5, 1.0, size=npts)
+    ds, dv = vjp(ctx, cont, sigma, pts, g)
+    parts = [vjp(ctx, cont, sigma, pts[k:k + 125], g[k:k + 125]) for k in range(0, npts, 125)]
+    rs, rv = sum(o[0] for o in parts), sum(o[1] for o in parts)
+    # sums of 7,013 terms in another order: 7,013 x 2^-53 = 8e-13 of the sum of magnitudes, which for the densities'
+    # positive terms is the sum, and for the vertices' at most ten times the largest
+    assert np.abs(ds - rs).max() <= 1e-12 * np.abs(rs).max()
+    assert np.abs(dv - rv).max() <= 1e-11 * np.abs(rv).max()
+    cont.close()
