@@ -992,24 +992,25 @@ __global__ __launch_bounds__(64) void k_bproj_sum(const double* __restrict__ par
     }
 }
 
-// row and column of position e of the panel's 64 rows from a multiple of 8 on (kp = 1 << sh columns)
+// row and column of entry e of a block of the panel, kNormCols columns wide, in the panel's own order
+constexpr int kNormRows = 64, kNormCols = 16;
 template <typename T>
-__device__ __forceinline__ void panel_place(int e, int sh, int& i, int& r)
+__device__ __forceinline__ void panel_place(int e, int& i, int& r)
 {
-    i = e >> sh;
-    r = e & ((1 << sh) - 1);
+    i = e / kNormCols;
+    r = e % kNormCols;
 }
 template <>
-__device__ __forceinline__ void panel_place<uint16_t>(int e, int sh, int& i, int& r)
+__device__ __forceinline__ void panel_place<uint16_t>(int e, int& i, int& r)
 {
-    r = (e >> 3) & ((1 << sh) - 1);
-    i = (e >> (3 + sh)) * 8 + (e & 7);
+    r = e / 8 % kNormCols;
+    i = e / (8 * kNormCols) * 8 + e % 8;
 }
 
-// V_r (j+1) = W_r / nrm_r; panel column r = that for active r, 0 otherwise.  A block takes 64 rows of all right-hand
-// sides and turns them through LDS, so the panel, too, is written in whole lines (20,000 rows x 64: 13.0 us, 18.8 with a
-// panel entry per lane, each in a line of its own).
-constexpr int kNormRows = 64;
+// V_r (j+1) = W_r / nrm_r; panel column r = that for active r, 0 otherwise.  A block takes 64 rows of 16 right-hand
+// sides and turns them through LDS, so the panel, too, is written in runs of 64 bytes or more (20,000 rows x 64: 7.0 us, 18.8 with a
+// panel entry per lane, each in a line of its own, and 13.0 with all right-hand sides in one block, which also left calls
+// of 1,000 to 2,000 rows with too few blocks: BF16 x 64 8,260 before, 8,787 so, 8,288 us now).
 template <typename T, typename VT>
 __global__ __launch_bounds__(kBlock) void k_bnormalize_idx(const double* __restrict__ W,
                                                            const double* __restrict__ nrm,
@@ -1018,24 +1019,27 @@ __global__ __launch_bounds__(kBlock) void k_bnormalize_idx(const double* __restr
                                                            T* __restrict__ Vt, const int* __restrict__ ints)
 {
     if (ints[1]) return;
-    __shared__ T tile[64][kNormRows + 1];
-    const int lane = threadIdx.x & 63;
+    __shared__ T tile[kNormCols][kNormRows + 1];
+    const int lane = threadIdx.x & 63, r0 = blockIdx.y * kNormCols, cols = min(kNormCols, nrhs - r0);
     const int64_t i0 = (int64_t)blockIdx.x * kNormRows, i = i0 + lane;
     const int64_t at = (int64_t)(ints[0] + 1) * n + i;
     if (i < n) {
-#pragma unroll 4
-        for (int r = threadIdx.x >> 6; r < nrhs; r += kBlock / 64) {
+#pragma unroll
+        for (int c = threadIdx.x >> 6; c < kNormCols; c += kBlock / 64) {
+            if (c >= cols) break;
+            const int r = r0 + c;
             const double v = active[r] ? W[(int64_t)r * n + i] * (1.0 / nrm[r]) : 0.;
             V[r * vstride + at] = (VT)v;
-            tile[r][lane] = panel_value<T>(v);
+            tile[c][lane] = panel_value<T>(v);
         }
     }
     __syncthreads();
-    const int sh = 31 - __clz(kp), rows = (int)std::min<int64_t>(kNormRows, n - i0);
-    for (int e = threadIdx.x; e < (kNormRows << sh); e += kBlock) {
-        int ii, r;
-        panel_place<T>(e, sh, ii, r);
-        if (ii < rows && r < nrhs) Vt[i0 * kp + e] = tile[r][ii];
+    const int rows = (int)std::min<int64_t>(kNormRows, n - i0);
+#pragma unroll
+    for (int e = threadIdx.x; e < kNormRows * kNormCols; e += kBlock) {
+        int ii, c;
+        panel_place<T>(e, ii, c);
+        if (ii < rows && c < cols) Vt[panel_index<T>(i0 + ii, r0 + c, kp)] = tile[c][ii];
     }
 }
 
@@ -1441,7 +1445,7 @@ void batch_orthonormalize(hipStream_t st, const BatchArnoldi& a, VT* V)
                                                                           a.W, stop);
     }
     k_bnorm<<<(unsigned)nrhs, kNormBlock, 0, st>>>(a.W, n, a.nrm, 1, stop);
-    const unsigned grid = (unsigned)((n + kNormRows - 1) / kNormRows);
+    const dim3 grid((unsigned)((n + kNormRows - 1) / kNormRows), (unsigned)((nrhs + kNormCols - 1) / kNormCols));
     if (a.A16)
         k_bnormalize_idx<uint16_t, VT><<<grid, kBlock, 0, st>>>(a.W, a.nrm, a.active, n, nrhs, V, a.vstride, a.kp,
                                                                a.P16, a.ints);
