@@ -485,30 +485,36 @@ __global__ __launch_bounds__(64) void k_tree_ranges(const double* __restrict__ p
         y[n] = py[i];
         z[n] = pz[i];
     }
+    // A point with a coordinate that is not a number gives values that are not, whatever is summed, and is left out of
+    // the spheres; an infinite coordinate, or a distance past the largest number, makes a range's radius infinite, so
+    // that nothing is taken for it and its elements go pair by pair, as in the flat passes.
+    bool some[NP];
+#pragma unroll
+    for (int n = 0; n < NP; n++) some[n] = x[n] == x[n] && y[n] == y[n] && z[n] == z[n];
     double c[3];
     auto sphere = [&](int a, int b) {
         double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        auto in = [&](int n) { return n * 64 + lane >= a && n * 64 + lane < b && some[n]; };
 #pragma unroll
         for (int n = 0; n < NP; n++)
-            if (n * 64 + lane >= a && n * 64 + lane < b) {
+            if (in(n)) {
                 lo[0] = fmin(lo[0], x[n]), lo[1] = fmin(lo[1], y[n]), lo[2] = fmin(lo[2], z[n]);
                 hi[0] = fmax(hi[0], x[n]), hi[1] = fmax(hi[1], y[n]), hi[2] = fmax(hi[2], z[n]);
             }
 #pragma unroll
-        for (int k = 0; k < 3; k++) c[k] = 0.5 * (dev::wave_min(lo[k]) + dev::wave_max(hi[k]));
+        for (int k = 0; k < 3; k++) {
+            const double least = dev::wave_min(lo[k]), most = dev::wave_max(hi[k]);
+            c[k] = least <= most ? 0.5 * (least + most) : 0.;  // no point but such: anything
+        }
         double far = 0.;
 #pragma unroll
         for (int n = 0; n < NP; n++)
-            if (n * 64 + lane >= a && n * 64 + lane < b) {
+            if (in(n)) {
                 const double dx = x[n] - c[0], dy = y[n] - c[1], dz = z[n] - c[2];
                 const double d2 = dx * dx + dy * dy + dz * dz;
-                far = d2 <= far ? far : d2;  // not a number stays: nothing is taken for such a range
+                far = d2 == d2 ? fmax(far, d2) : INFINITY;
             }
-        for (int o = 32; o > 0; o >>= 1) {
-            const double v = __shfl_xor(far, o, 64);
-            far = v <= far ? far : v;
-        }
-        return dev::uniform(sqrt(far));
+        return dev::uniform(sqrt(dev::wave_max(far)));
     };
     int a = 0, len = 64 * NP, k = 0;
     Ranges<NP, SETS>* o = out + grp;

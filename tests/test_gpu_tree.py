@@ -104,6 +104,37 @@ def test_tree_hard_points(ctx):
     cont.close()
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("npts", [16384, 70000])
+@pytest.mark.parametrize("lane", [5, 31, 32, 60, 62, 63])
+def test_tree_points_that_are_not_finite(ctx, lane, npts, precision):
+    """One coordinate of one point in each second group not a number, in lanes of both halves of a wavefront, with one and two
+    points per lane: alone, so that the others stay in curve order, and beside an infinite coordinate, which leaves all
+    points in the caller's order, where every second one lies far from its neighbours."""
+    from kassiopeia_amd import kemfield as K
+
+    m = mesh_of("triangles", 4007)
+    cont = K.KSurfaceContainer(ctx, m)
+    sigma = 1e-9 * np.random.default_rng(5).normal(size=m.n)
+    tol = 1e-13 if precision == "fp64" else 1e-6  # as for finite points
+    for infinite in (False, True):
+        pts = points_of("triangles", npts, 6)
+        pts[lane::128, 0] = np.nan
+        if infinite:
+            pts[1::2] = 0.0
+            pts[lane::128, 0] = np.nan
+            pts[npts // 2, 1] = np.inf
+        some = np.unique(np.concatenate([np.arange(npts // 2 - 64, npts // 2 + 64), np.arange(0, npts, 5)]))
+        E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, precision).ElectricFieldAndPotential(pts)
+        E0, p0 = flat(cont, sigma, pts[some], "fp64")
+        ok = np.isfinite(pts[some]).all(1)
+        E, phi = E[some], phi[some]
+        assert not np.isfinite(E[np.isnan(pts[some]).any(1)]).any()
+        assert np.linalg.norm(E[ok] - E0[ok]) <= tol * np.linalg.norm(E0[ok]), infinite
+        assert np.linalg.norm(phi[ok] - p0[ok]) <= tol * np.linalg.norm(p0[ok]), infinite
+    cont.close()
+
+
 @pytest.mark.parametrize("kind,n,npts,sets,precision", [
     ("triangles", 4007, 40001, 4, "fp64"), ("frame", 3219, 262147, 24, "fp64"), ("groups", 4800, 33000, 3, "fp64"),
     ("triangles", 4007, 150001, 3, "mixed"), ("triangles", 4992, 262149, 6, "mixed"),
