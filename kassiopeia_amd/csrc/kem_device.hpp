@@ -244,11 +244,20 @@ __device__ __forceinline__ F4 line_analytic(const double* __restrict__ g, double
 // tan(Omega / 2) = |a0.(a1 x a2)| / (R0 R1 R2 + (a0.a1) R2 + (a1.a2) R0 + (a2.a0) R1), the triple product
 // being twice the area times |h|; a rectangle's two triangles P0P1P2 and P2P3P0 add as angles of complex
 // numbers; signed by h.  Triangle: 2 pi at the centroid; rectangle: in the plane 2 pi inside, 0 outside.
+// For a triangle and a point in its plane both numbers are roundings on an edge's line, and there the angle is what the
+// reference's own operations, on unit corner vectors, make of them.
 //
 // NEAR: the pair is in the numeric policy's near set (within 4.6 sizes), and the logarithm is that of the
 // quotient.  The rwg policy also evaluates distant pairs, whose terms cancel like eps dr^2: there the difference
 // of two logarithms keeps the roundings of the reference (the quotient's is closer to the truth, and 1.4 times
 // further from the reference at dr = 2,000).
+// whether height h over an element's plane is no more than the roundings of the distance c from its centre and of the
+// coordinates, by which the corners' own rounding takes them out of the plane
+__device__ __forceinline__ bool in_plane(double h, double cx, double cy, double cz, double px, double py, double pz)
+{
+    return fabs(h) <= 1.e-12 + 1.e-14 * (fabs(cx) + fabs(cy) + fabs(cz) + fabs(px) + fabs(py) + fabs(pz));
+}
+
 template <int NE, bool FIELD, bool NEAR>
 __device__ __forceinline__ F4 closed_form_at(const double* __restrict__ g, double px, double py, double pz, int count,
                                              int line, double dist)
@@ -274,7 +283,25 @@ __device__ __forceinline__ F4 closed_form_at(const double* __restrict__ g, doubl
         // g[KG_PREF] = area / (4 pi eps0): twice the triangle's area (each half of a rectangle: its area)
         const double y = g[KG_PREF] * ((NE == 3 ? 2. : 1.) / kK) * fabs(h);
         if (NE == 3) {
-            om = 2. * angle_acc(y, low(0, 1, 2));
+            double top = y, bottom = low(0, 1, 2);
+            if (in_plane(h, cx, cy, cz, px, py, pz)) {
+                double u[3][3];
+#pragma unroll
+                for (int v = 0; v < 3; v++) {
+                    const double im = rsqrt_acc(ax[v] * ax[v] + ay[v] * ay[v] + az[v] * az[v]);
+                    u[v][0] = im * ax[v];
+                    u[v][1] = im * ay[v];
+                    u[v][2] = im * az[v];
+                }
+                bottom = 1. + (u[0][0] * u[1][0] + u[0][1] * u[1][1] + u[0][2] * u[1][2]) +
+                         (u[0][0] * u[2][0] + u[0][1] * u[2][1] + u[0][2] * u[2][2]) +
+                         (u[1][0] * u[2][0] + u[1][1] * u[2][1] + u[1][2] * u[2][2]);
+                const double a0 = u[1][1] * u[2][2] - u[1][2] * u[2][1];
+                const double a1 = u[1][2] * u[2][0] - u[1][0] * u[2][2];
+                const double a2 = u[1][0] * u[2][1] - u[1][1] * u[2][0];
+                top = fabs(u[0][0] * a0 + u[0][1] * a1 + u[0][2] * a2);
+            }
+            om = 2. * angle_acc(top, bottom);
             if (cx * cx + cy * cy + cz * cz <= 1.e-24) om = 2. * kPi;
         } else {
             const double x1 = low(0, 1, 2), x2 = low(2, NE - 1, 0);
@@ -344,11 +371,11 @@ __device__ __forceinline__ F4 closed_form(const double* __restrict__ g, double p
 {
     int count = 0, line = 99;
     double dmin = 0.;
-    // Only a point in the element's plane can lie on an edge: kMinDistToLine is far below the height bound,
-    // which leaves room for h's own rounding (a few ulps of the distance), so most wavefronts skip the test.
+    // only a point in the element's plane can lie on an edge (kMinDistToLine is far below the bound on the height), so
+    // most wavefronts skip the test
     const double cx = px - g[KG_HX], cy = py - g[KG_HY], cz = pz - g[KG_HZ];
     const double h = g[KG_NX] * cx + g[KG_NY] * cy + g[KG_NZ] * cz;
-    if (fabs(h) <= 1.e-12 + 1.e-14 * (fabs(cx) + fabs(cy) + fabs(cz))) {
+    if (in_plane(h, cx, cy, cz, px, py, pz)) {
 #pragma unroll 1
         for (int e = 0; e < NE; e++) {
             const double dx = g[KG_V + 3 * e] - px, dy = g[KG_V + 3 * e + 1] - py, dz = g[KG_V + 3 * e + 2] - pz;

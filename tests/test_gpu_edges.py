@@ -1,7 +1,7 @@
 """Edge cases of the C-ABI on the GPU: empty point sets, a one-element mesh, point counts on
-either side of the wavefront (64), block (256) and Morton-sort (4,096) boundaries, which must
-all give the same answers as one large call and as the oracle, and the rejection of degenerate
-or unknown shapes."""
+either side of the wavefront (64), block (256) and point-ordering (4,096) boundaries, which must
+all give the same answers as one large call and as the oracle, points on corners and edges, and the
+rejection of degenerate or unknown shapes."""
 import ctypes
 
 import numpy as np
@@ -72,6 +72,24 @@ def test_ragged_point_counts(ctx, oracle, precision):
         E, phi = solver.ElectricFieldAndPotential(P[:n])
         assert np.abs(phi - phi_all[:n]).max() <= tol * np.abs(phi_all).max(), n
         assert np.abs(E - E_all[:n]).max() <= 10 * tol * np.abs(E_all).max(), n
+
+
+def test_points_on_corners_and_edges(ctx, oracle):
+    """On a triangle's edge the solid angle is 0 / 0, so the normal field there is what the reference's own operations make
+    of the roundings: the oracle's values, not merely one of the two sides' limits."""
+    from kassiopeia_amd import kemfield as K
+
+    m = G.cube_mesh(3)
+    cont = K.KSurfaceContainer(ctx, m)
+    sigma = 1e-9 * np.random.default_rng(1).uniform(0.5, 1.5, m.n)
+    r = m.recs
+    p0, p1, p2 = r[:, 2:5], r[:, 2:5] + r[:, 0:1] * r[:, 5:8], r[:, 2:5] + r[:, 1:2] * r[:, 8:11]
+    P = np.concatenate([p0, p1, p2, 0.5 * (p0 + p1)])
+    E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma).ElectricFieldAndPotential(P)
+    pr, Er = oracle.field(m.shapes, m.recs, sigma, P)
+    # corners are evaluated 1e-7 off the plane, where the logarithms of nearby edges lose up to 1e-7 / 1e-16
+    assert np.abs(phi - pr).max() <= 1e-12 * np.abs(pr).max()
+    assert np.linalg.norm(E - Er, axis=1).max() <= 1e-10 * np.linalg.norm(Er, axis=1).max()
 
 
 def test_rejected_shapes(ctx):
