@@ -58,16 +58,16 @@ FieldPlan plan_field(int policy, const FieldMesh& m, bool mixed, double fp64_rat
                      int64_t npts, int64_t range_elems, int64_t ws_doubles);
 
 // How launch_field evaluates far pairs hierarchically (kem_tree.hip; host arithmetic): expansions of moments
-// doubles at the start of ws, then the point groups' ranges, then partials doubles of partial sums, the latter two
-// for chunk points at a time.
+// doubles at the start of ws, then the runs' charge radii, the point groups' ranges and partials doubles of partial sums,
+// the latter two for chunk points at a time.
 struct TreePlan {
     bool use = false;
     TreeLevels levels;
     int per_lane = 1;      // points per lane
     int64_t sets = 1;      // charge-density sets, each with its expansions
     int slices = 1;        // blocks per group of 64 per_lane points, each with a slice of the partial sums
-    int64_t moments = 0, ranges = 0, partials = 0, chunk = 0;
-    int64_t doubles() const { return moments + ranges + partials; }
+    int64_t moments = 0, reach = 0, ranges = 0, partials = 0, chunk = 0;
+    int64_t doubles() const { return moments + reach + ranges + partials; }
 };
 TreePlan plan_tree(int policy, const FieldMesh& m, bool mixed, double fp64_ratio, bool multi, int64_t nsets,
                    int64_t npts);

@@ -1985,18 +1985,19 @@ int64_t field_workspace_doubles(int policy, const FieldMesh& m, bool mixed, doub
 }
 
 namespace {
-// The hierarchical pass over points in curve order: expansions at the start of ws, then the point groups' ranges
-// and the partial sums of a chunk of points.
+// The hierarchical pass over points in curve order: expansions at the start of ws, then the runs' charge radii, the
+// point groups' ranges and the partial sums of a chunk of points.
 hipError_t tree_field(hipStream_t st, const FieldMesh& m, const TreePlan& p, bool mixed, const double* sigma,
                       const int32_t* pset, const double* px, const double* py, const double* pz, int64_t npts, double* phi, double* ex,
                       double* ey, double* ez, double* ws, hipEvent_t far_begin, hipEvent_t far_end)
 {
-    double* q = ws + p.moments + p.ranges;
+    double* ranges = ws + p.moments + p.reach;
+    double* q = ranges + p.ranges;
     if (far_begin) (void)hipEventRecord(far_begin, st);
     for (int64_t p0 = 0; p0 < npts; p0 += p.chunk) {
         const int64_t np = std::min(p.chunk, npts - p0);
         const hipError_t e = launch_tree(st, m, p, mixed, sigma, pset ? pset + p0 : nullptr, px + p0, py + p0, pz + p0,
-                                         np, ws, ws + p.moments, q, p0 == 0);
+                                         np, ws, ranges, q, p0 == 0);
         if (e != hipSuccess) return e;
         if (far_end && p0 + np >= npts) (void)hipEventRecord(far_end, st);
         k_field_combine<<<dim3(nblocks(np), 4), kBlock, 0, st>>>(q, p.slices, np, phi + p0, ex + p0, ey + p0, ez + p0);

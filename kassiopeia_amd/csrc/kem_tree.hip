@@ -37,18 +37,27 @@ __host__ __device__ constexpr int entry(int P, int l, int m) { return line_start
 __host__ __device__ constexpr int entries(int P) { return line_start(P, P + 2); }
 __host__ __device__ constexpr int tri_index(int l, int m) { return l * (l + 1) / 2 + m; }
 
-// The order stored, and the tolerance that chooses the order summed.  Order p serves a run of radius a
-// at distance d from the sphere around a range of points when (a / d)^(p+1) <= tol.  The first omitted term is
-// below that against the run's charge by magnitude, and its coefficients decay besides: at 8e-14 (FP64) and 7e-7
-// (mixed) the error against 64-bit sums is that of the pairs' own rules and rounding, the same as at a tolerance
-// 80 times smaller, for smooth densities and for densities of random sign (20,000-triangle coax, 40,000-triangle
-// bore, a cube of 3,072 and 5,047 rectangles and wires: 1.5e-15 to 9.6e-15 and 0.8e-8 to 7.5e-8 of the field, all
-// within the flat passes').  The orders: 100,000 points over 20,000 triangles 18.2 ms at 22, 14.6 at 26 (FP64);
-// a million, mixed, 24.3 ms at 16, 21.8 at 20, no faster at 24.
+// The order stored, and the tolerance that chooses the order summed.  With T_l = sum_q |q| (r_q / a)^l over a run's
+// charges (r_q from its centre), the terms of order l are at most T_l (a / d)^l of the potential and (l + 1) T_l (a / d)^l
+// of the field, tight for a single charge.  By convexity T_l <= rho^l T_0 up to order L for rho^L = T_L / T_0, so order
+// p serves a run at distance d from the sphere around a range of points when, with q = rho a / d,
+//   sum_{l > p} (l + 1) q^l (1 - q)^2 = ((p + 2) - (p + 1) q) q^(p+1) <= tol,
+// the field's omitted part against the field of the charge rho a from the centre on the points' side (L past the order
+// stored and a / d < widest bound what rho does not).  Each call finds rho a of each run (k_tree_reach): at the rim it
+// is a, for the elements of a surface 0.85 of it, which saves two orders.
+// The tolerances keep every point's field as good as the pairs' own rules do it, whatever the charges: one
+// charged element at the rim of a run of any level (of 16 to 4,096 elements: 20,000-triangle coax, 100,000-triangle bore, a
+// cube, rectangles and wires), points in clumps beyond it, worst / root mean square error of the field: FP64 3.3e-14 / 2.8e-15
+// both here and in the flat passes, mixed 4.0e-7 / 1.0e-7 in both (with (a / d)^(p+1) <= 8e-14 and 7e-7, the bound of the
+// potential, 8.5e-13 and 4.5e-6).
+// The orders: a million points over 20,000 triangles, mixed, 19.5 ms at 20, 19.2 at 21, 19.0 at 22, where 400,000
+// over 100,000 take 9.0 instead of 8.7; 100,000 points over 20,000 triangles, FP64, 14.9 ms at 26, 13.5 at 28, 13.0 at 30.
 template <bool MIXED>
 struct Orders {
-    static constexpr int P = MIXED ? 20 : 26;
-    static constexpr float log2_tol = MIXED ? -20.5f : -43.5f;
+    static constexpr int P = MIXED ? 21 : 30;
+    static constexpr float log2_tol = MIXED ? -21.7f : -47.2f;
+    static constexpr float widest = 0.6f;
+    static constexpr int H = (P + 2) / 2;  // L / 2
 };
 
 // ------------------------------------------------------------------ expansions
@@ -348,6 +357,67 @@ __global__ __launch_bounds__(2 * kM2MGroup) void k_tree_m2m(const double* __rest
     }
 }
 
+// rho a of each run from the lowest stored level up, and of each set (blockIdx.y); L = 2 H.  The mean of r^L over an element
+// is at most that over its corners, since it is convex.  Bound by the elements' records, read once per level: 14 us
+// for 20,000 triangles, 70 us for 100,000.
+template <int H>
+__global__ __launch_bounds__(kP2MBlock) void k_tree_reach(const double* __restrict__ geom,
+                                                          const int32_t* __restrict__ order,
+                                                          const double* __restrict__ sigma,
+                                                          const double* __restrict__ tnode, TreeLevels T, int64_t nelem,
+                                                          float* __restrict__ reach, int64_t reach_set)
+{
+    __shared__ double red[kP2MBlock / 64][2];
+    const int64_t base = T.first[T.low], node = base + blockIdx.x;
+    int lev = T.low;
+    int64_t run = T.run;
+    while (node >= (int64_t)T.first[lev] + T.count[lev]) {
+        lev++;
+        run *= KEM_TREE_FAN;
+    }
+    const int64_t e0 = (node - T.first[lev]) * run, e1 = e0 + run < nelem ? e0 + run : nelem;
+    const double* t = tnode + node * KEM_TREE_STRIDE;
+    const double* sg = sigma + blockIdx.y * nelem;
+    const double cx = t[0], cy = t[1], cz = t[2], ia2 = t[5] * t[5];
+    double all = 0., far = 0.;
+    for (int64_t e = e0 + threadIdx.x; e < e1; e += kP2MBlock) {
+        const int64_t j = order[e];
+        const double* g = geom + j * KG_STRIDE;
+        const int type = (int)g[KG_TYPE], nv = type == KEM_TRIANGLE ? 3 : type == KEM_RECTANGLE ? 4 : 2;
+        double corners = 0.;
+        for (int v = 0; v < nv; v++) {
+            const double dx = g[KG_V + 3 * v] - cx, dy = g[KG_V + 3 * v + 1] - cy, dz = g[KG_V + 3 * v + 2] - cz;
+            double f = 1., b = (dx * dx + dy * dy + dz * dz) * ia2;
+#pragma unroll
+            for (int k = H; k; k >>= 1) {
+                if (k & 1) f *= b;
+                b *= b;
+            }
+            corners += f;
+        }
+        const double w = fabs(g[KG_PREF] * sg[j]);
+        all += w;
+        far += w * corners / nv;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        all += __shfl_xor(all, o, 64);
+        far += __shfl_xor(far, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        red[threadIdx.x >> 6][0] = all;
+        red[threadIdx.x >> 6][1] = far;
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < kP2MBlock / 64; k++) {
+        all += red[k][0];
+        far += red[k][1];
+    }
+    // rounded up, and no less than a mean whose power is still a 32-bit number; charges that are not finite: the radius
+    const float rho = all == 0. ? 0.f : exp2f(log2f((float)(far / all)) * (0.5f / H)) * 1.0001f;
+    reach[blockIdx.y * reach_set + blockIdx.x] = (float)t[3] * 1.0001f * (rho < 1.f ? fmaxf(rho, 0.0625f) : 1.f);
+}
+
 // ------------------------------------------------------------------ evaluation
 typedef double Pair __attribute__((ext_vector_type(2)));
 
@@ -578,9 +648,10 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
     const double* __restrict__ geom, const double* __restrict__ nodes, const float* __restrict__ nodes32,
     const float* __restrict__ far6, const double* __restrict__ far6_cl, const int32_t* __restrict__ order,
     const double* __restrict__ sigma, const double* __restrict__ tnode, const double* __restrict__ mom,
-    TreeLevels T, int64_t nelem, const double* __restrict__ px, const double* __restrict__ py,
-    const double* __restrict__ pz, const Ranges<NP, SETS>* __restrict__ ranges, int64_t npts, int64_t ngroups,
-    int slices, double* __restrict__ out, int64_t comp_stride, int64_t mom_set)
+    const float* __restrict__ reach, TreeLevels T, int64_t nelem, const double* __restrict__ px,
+    const double* __restrict__ py, const double* __restrict__ pz, const Ranges<NP, SETS>* __restrict__ ranges,
+    int64_t npts, int64_t ngroups, int slices, double* __restrict__ out, int64_t comp_stride, int64_t mom_set,
+    int64_t reach_set)
 {
     using O = Orders<MIXED>;
     constexpr int E = entries(O::P);
@@ -617,10 +688,12 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
         const double wx = rg[0], wy = rg[1], wz = rg[2], wr = rg[3];
         const double* sg = sigma;
         const double* ms = mom;
+        const float* rs = reach - T.first[T.low];
         if constexpr (SETS) {
             const int64_t set = (int64_t)rg[6];
             sg += set * nelem;
             ms += set * mom_set;
+            rs += set * reach_set;
         }
         bool in[NP];  // the lane's points that belong to the range
 #pragma unroll
@@ -649,9 +722,13 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
             const double* t = tnode + (int64_t)at * KEM_TREE_STRIDE;
             const double dx = t[0] - wx, dy = t[1] - wy, dz = t[2] - wz;
             const double d = sqrt(dx * dx + dy * dy + dz * dz) * (1. - 1e-9) - wr;
-            // the smallest order with (a / d)^(p+1) <= tol
-            const float lg = __log2f((float)(t[3] / d));
-            const int ord = lg < -1.f ? (int)ceilf(O::log2_tol / lg) - 1 : O::P + 1;
+            // the smallest order whose omitted terms stay below the tolerance (Orders), by fixed-point steps: the
+            // factor before the power changes slowly with the order, and two steps leave 0.01 of one
+            const float id = 1.f / (float)d, q = rs[at] * id, lg = __log2f(q);
+            float need = O::log2_tol / lg - 1.f;
+#pragma unroll
+            for (int k = 0; k < 2; k++) need = (O::log2_tol - __log2f(need + 2.f - (need + 1.f) * q)) / lg - 1.f;
+            const int ord = lg < -1.f && (float)t[3] * id < O::widest ? (int)ceilf(need) : O::P + 1;
             const bool take = have && d > t[4] && ord <= O::P;
             const bool open = have && !take && lev > T.low;
             const bool pairs = have && !take && lev == T.low;
@@ -798,8 +875,12 @@ hipError_t tree_passes(hipStream_t st, const FieldMesh& m, const TreePlan& p, co
     const TreeLevels& T = p.levels;
     const int64_t stride = 2 * entries(P);
     const int64_t base = T.first[T.low], mom_set = p.moments / p.sets;
+    const int64_t runs = T.first[T.levels - 1] + T.count[T.levels - 1] - base;
+    float* reach = reinterpret_cast<float*>(mom + p.moments);
     if (moments) {
         const double* low = m.tree + base * KEM_TREE_STRIDE;
+        k_tree_reach<Orders<MIXED>::H><<<dim3((unsigned)runs, (unsigned)p.sets), kP2MBlock, 0, st>>>(
+            m.geom, m.order, sigma, m.tree, T, m.n, reach, runs);
         if (pset)
             k_tree_p2m_sets<P><<<(unsigned)T.count[T.low], kP2MBlock, 0, st>>>(m.geom, m.nodes, m.order, sigma, p.sets,
                                                                               low, m.n, T.run, mom, mom_set);
@@ -821,8 +902,8 @@ hipError_t tree_passes(hipStream_t st, const FieldMesh& m, const TreePlan& p, co
         k_tree_ranges<NP, SETS><<<(unsigned)groups, 64, 0, st>>>(px, py, pz, pset, npts, rg);
         auto run = [&](auto triangles) {
             k_field_tree<MIXED, NP, decltype(triangles)::value, SETS><<<grid, 64 * kTreeWaves, 0, st>>>(
-                m.geom, m.nodes, m.nodes32, m.far6, m.far6_cl, m.order, sigma, m.tree, mom, T, m.n, px, py, pz, rg,
-                npts, groups, p.slices, out, p.slices * npts, mom_set);
+                m.geom, m.nodes, m.nodes32, m.far6, m.far6_cl, m.order, sigma, m.tree, mom, reach, T, m.n, px, py, pz, rg,
+                npts, groups, p.slices, out, p.slices * npts, mom_set, runs);
         };
         if (m.triangles)
             run(std::true_type());
@@ -878,10 +959,11 @@ constexpr int kTreeMaxSlices = 16;
 // mixed: 16,384 points 2.51 ms with two, 1.99 with one; 65,536 points 4.15 and 3.93).
 constexpr int64_t kTreePairPoints = 65537;
 // Expansions of calls that the no-allocation entry point may serve (up to 65,536 points) fit its scratch beside
-// the points' ordering and partial sums; other calls' are bounded by 4 GiB.  Runs of the lowest level grow until
-// they do.
+// the points' ordering, partial sums and the group members' charge densities; other calls' are bounded by 4 GiB.  Runs of
+// the lowest level grow until they do: from 33,000 elements on in FP64, 58,000 in mixed precision.  The entry points that
+// allocate keep to the same sizes at these points, as their results are the same bit for bit.
 constexpr int64_t kTreeSmallPoints = 65536;
-constexpr int64_t kTreeSmallDoubles = (int64_t)5 << 19, kTreeSmallPartials = (int64_t)3 << 19;
+constexpr int64_t kTreeSmallDoubles = (int64_t)7 << 19, kTreeSmallPartials = (int64_t)3 << 19;
 constexpr int64_t kTreeLargeDoubles = (int64_t)512 << 20;
 // partial sums of one chunk of points
 constexpr int64_t kTreePartialDoubles = (int64_t)128 << 20;
@@ -900,13 +982,14 @@ TreePlan plan_tree(int policy, const FieldMesh& m, bool mixed, double fp64_ratio
     TreeLevels& T = p.levels;
     tree_levels(m.n, T);
     const int P = mixed ? Orders<true>::P : Orders<false>::P;
-    const int64_t limit = !multi && npts <= kTreeSmallPoints ? kTreeSmallDoubles : kTreeLargeDoubles;
+    const int64_t limit = !multi && npts <= kTreeSmallPoints ? kTreeSmallDoubles - m.n : kTreeLargeDoubles;
     const int64_t total = T.first[T.levels - 1] + T.count[T.levels - 1];
     for (T.low = 0; T.low < T.levels; T.low++) {
         p.moments = p.sets * (total - T.first[T.low]) * 2 * entries(P);
         if (p.moments <= limit) break;
     }
     if (T.low >= T.levels) return TreePlan();
+    p.reach = (p.sets * (total - T.first[T.low]) + 1) / 2;
     T.run = KEM_TREE_LEAF;
     for (int k = 0; k < T.low; k++) T.run *= KEM_TREE_FAN;
     p.per_lane = !multi && npts >= kTreePairPoints ? 2 : 1;

@@ -68,7 +68,7 @@ def test_tree_against_flat(ctx, kind, n, npts, rough):
     E0, p0 = flat(cont, sigma, pts[some], "fp64")
     for precision, tol in (("fp64", 1e-13), ("mixed", 1e-6)):
         E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, precision).ElectricFieldAndPotential(pts)
-        # FP64: expansions to 8e-14 of each run's field, before the decay of their coefficients; mixed: its bar
+        # FP64: expansions to 6e-15 of each run's field and the pairs' own rules to 3e-14; mixed: its bar
         assert np.linalg.norm(E[some] - E0) <= tol * np.linalg.norm(E0), precision
         assert np.linalg.norm(phi[some] - p0) <= tol * np.linalg.norm(p0), precision
         assert np.abs(phi[some] - p0).max() <= 10 * tol * np.abs(p0).max(), precision
@@ -132,6 +132,34 @@ def test_tree_points_that_are_not_finite(ctx, lane, npts, precision):
         assert not np.isfinite(E[np.isnan(pts[some]).any(1)]).any()
         assert np.linalg.norm(E[ok] - E0[ok]) <= tol * np.linalg.norm(E0[ok]), infinite
         assert np.linalg.norm(phi[ok] - p0[ok]) <= tol * np.linalg.norm(p0[ok]), infinite
+    cont.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind,n", [("triangles", 4992), ("frame", 3219), ("cube", 3072)])
+def test_tree_one_charged_element(ctx, kind, n, precision):
+    """One charged element at a time, where the coefficients of the expansions of a run that has it at its rim do not decay:
+    clumps of points all around it, where runs are taken near and far, point by point."""
+    from kassiopeia_amd import kemfield as K
+
+    m = G.cube_mesh(16) if kind == "cube" else mesh_of(kind, n)
+    cont = K.KSurfaceContainer(ctx, m)
+    c = m.centroids()
+    size = np.ptp(c, axis=0).max()
+    # each run's terms are omitted below 6e-15 (FP64) and 3e-7 (mixed) of the element's field at the point, and the rules of
+    # the pairs err by up to 3e-14 (FP64, in either evaluation) and 4e-7 (mixed)
+    tol = 6e-14 if precision == "fp64" else 6e-7
+    for j in np.random.default_rng(n).integers(0, m.n, 24):
+        rng = np.random.default_rng(j)
+        sigma = np.zeros(m.n)
+        sigma[j] = 1e-9
+        out = rng.normal(size=(1100, 3))
+        out *= (size * np.exp(rng.uniform(np.log(0.03), np.log(3.0), 1100)) / np.linalg.norm(out, axis=1))[:, None]
+        pts = np.repeat(c[j] + out, 32, 0) + 1e-7 * rng.normal(size=(1100 * 32, 3))
+        E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, precision).ElectricFieldAndPotential(pts)
+        E0, p0 = flat(cont, sigma, pts, "fp64")
+        assert (np.linalg.norm(E - E0, axis=1) / np.linalg.norm(E0, axis=1)).max() <= tol, j
+        assert (np.abs(phi - p0) / np.abs(p0)).max() <= tol, j
     cont.close()
 
 
