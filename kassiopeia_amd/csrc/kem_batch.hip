@@ -183,11 +183,14 @@ constexpr int kReduceRows = 16;  // rows per block of k_bmm32_reduce
 // its kReduceRows KP / 256 entries before adding them, so a reduce is about one round trip to
 // memory (one split per round trip: 9 splits of a 20,000 x 64 block in 41 us; 32 rows and
 // four splits per round trip: 20 us for 6 splits); the sums are transposed through LDS so that
-// the writes run along rows.
-template <int KP, typename P = float>
+// the writes run along rows.  WHOLE (a caller's right-hand sides through k_bmm32s): column c was multiplied with scale[c],
+// and sums that are not numbers are formed again from matrix and panel.
+template <int KP, typename P = float, bool WHOLE = false>
 __global__ __launch_bounds__(kBlock) void k_bmm32_reduce(const P* __restrict__ part, int nsplit, int64_t n,
                                                          int ncols, double* __restrict__ W, int64_t ldw,
-                                                         const int* __restrict__ skip)
+                                                         const int* __restrict__ skip, const float* __restrict__ A = nullptr,
+                                                         const float* __restrict__ panel = nullptr,
+                                                         const float* __restrict__ scale = nullptr)
 {
     if (skip && *skip) return;
     constexpr int R = kReduceRows, E = R * KP / kBlock;
@@ -213,6 +216,16 @@ __global__ __launch_bounds__(kBlock) void k_bmm32_reduce(const P* __restrict__ p
             if (k0 + kk < nsplit)
                 for (int m = 0; m < E; m++) s[m] += (double)v[kk][m];
     }
+    if constexpr (WHOLE)
+        for (int m = 0; m < E; m++) {
+            const int e = threadIdx.x + kBlock * m, c = e % KP;
+            s[m] *= 1. / (double)scale[c];
+            if (s[m] == s[m] || e >= lim || c >= ncols) continue;
+            const float* a = A + i0 + e / KP;
+            double t = 0.;
+            for (int64_t j = 0; j < n; j++) t += (double)(a[j * n] * panel[j * KP + c]);
+            s[m] = t;
+        }
     for (int m = 0; m < E; m++) {
         const int e = threadIdx.x + kBlock * m;
         sh[e % KP][e / KP] = s[m];
@@ -313,6 +326,10 @@ constexpr int kStreamG = 4;       // BF16: column groups of 8 per chunk (3 buffe
 // the matrix cores and the splitting together (0.25 ms): 0.36 ms for 64 right-hand sides (4.5 TB/s), 0.54 ms on FP32
 // cores.  Half of a chunk's splitting is put between matrix instructions (0.40 ms with all of it before them, sums every
 // four chunks and 64-bit address arithmetic per lane).
+// What the parts cannot hold: the rest of an infinite number is inf - inf, so a product that comes out as not a number is
+// formed again without them (k_bmm32_reduce), and the third part of a number below 2^-110 lies below the smallest BF16
+// number, so right-hand sides of nothing but numbers below 2^-64 are multiplied with 2^64 first (k_column_scale).  Both
+// for a caller's right-hand sides only: those of the solver are normalised.
 constexpr int kSplitChunk = 16;                      // columns of the matrix per chunk (one MFMA's)
 constexpr int kSplitRun = 8;                         // chunks summed on the matrix cores at a time
 constexpr int kSplitPanel = 3 * 2 * 64;              // 16-byte operands of a chunk's panel rows
@@ -340,19 +357,40 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf8v (&o)[3])
     for (int k = 0; k < 3; k++) o[k] = __builtin_bit_cast(bf8v, uint4{w[k][0], w[k][1], w[k][2], w[k][3]});
 }
 
-// the panel's parts in operand order: [chunk][part][tile of 32 columns][lane], rows past n zero.  A block takes two
-// chunks: thread = chunk, tile, lane.
+// scale[c] = 2^64 where the column's largest number, as FP32, is below 2^-64 (and not 0), else 1: one block per column of the
+// panel, those from ncols on 1
+constexpr int kScaleBlock = 1024;
+__global__ __launch_bounds__(kScaleBlock) void k_column_scale(const double* __restrict__ X, int64_t ldx, int64_t n,
+                                                              int ncols, float* __restrict__ scale)
+{
+    __shared__ float sh[kScaleBlock / 64];
+    const int c = blockIdx.x;
+    float top = 0.f;
+    if (c < ncols)
+        for (int64_t i = threadIdx.x; i < n; i += kScaleBlock) top = fmaxf(top, fabsf((float)X[c * ldx + i]));
+    for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 1; k < kScaleBlock / 64; k++) top = fmaxf(top, sh[k]);
+    scale[c] = top > 0.f && top < 0x1p-64f ? 0x1p64f : 1.f;
+}
+
+// the panel's parts in operand order: [chunk][part][tile of 32 columns][lane], rows past n zero, column c times scale[c]
+// (nullable).  A block takes two chunks: thread = chunk, tile, lane.
 __global__ __launch_bounds__(kBlock) void k_split_panel(const float* __restrict__ P, int64_t n, int64_t nchunks,
-                                                        bf8v* __restrict__ out, const int* __restrict__ skip)
+                                                        const float* __restrict__ scale, bf8v* __restrict__ out,
+                                                        const int* __restrict__ skip)
 {
     if (skip && *skip) return;
     const int64_t c = (int64_t)blockIdx.x * 2 + (threadIdx.x >> 7);
     if (c >= nchunks) return;
     const int t = (threadIdx.x >> 6) & 1, lane = threadIdx.x & 63;
     const int64_t j0 = c * kSplitChunk + 8 * (lane >> 5);
+    const float f = scale ? scale[32 * t + (lane & 31)] : 1.f;
     float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = j0 + e < n ? P[(j0 + e) * 64 + 32 * t + (lane & 31)] : 0.f;
+    for (int e = 0; e < 8; e++) v[e] = j0 + e < n ? P[(j0 + e) * 64 + 32 * t + (lane & 31)] * f : 0.f;
     bf8v o[3];
     split8(v, o);
 #pragma unroll
@@ -1193,8 +1231,8 @@ size_t bmm_workspace_bytes(int64_t n, int nrhs, int prec)
         const int64_t tiles = (n + 63) / 64;
         const int s = std::max({bmm_splits(n, tiles), kp == 64 ? bmm_stream_splits(n) : 1,
                                 kp <= 32 && n % 4 == 0 ? bmm_tile_splits(n, kp, 4) : 1});
-        // a panel of 64 columns once more as its BF16 parts
-        const size_t parts = kp == 64 ? (size_t)((n + kSplitChunk - 1) / kSplitChunk) * kSplitPanel * 16 + 256 : 0;
+        // a panel of 64 columns once more as its BF16 parts, and its columns' scales
+        const size_t parts = kp == 64 ? (size_t)((n + kSplitChunk - 1) / kSplitChunk) * kSplitPanel * 16 + 512 : 0;
         return sizeof(float) * ((size_t)s * n * kp + (size_t)n * kp) + parts + 256;
     }
     const int64_t blocks = (n + kBlock - 1) / kBlock;
@@ -1251,9 +1289,15 @@ hipError_t launch_bmm(hipStream_t st, const float* A32, const double* A64, int64
             dim3 grid((unsigned)((n + kStreamRows - 1) / kStreamRows), (unsigned)nc);
             const int64_t nchunks = (n + kSplitChunk - 1) / kSplitChunk;
             bf8v* V3 = (bf8v*)(((uintptr_t)(Vt + (size_t)n * 64) + 255) / 256 * 256);
-            k_split_panel<<<(unsigned)((nchunks + 1) / 2), kBlock, 0, st>>>(P, n, nchunks, V3, skip);
+            float* scale = x_is_panel ? nullptr : (float*)(V3 + nchunks * kSplitPanel);
+            if (scale) k_column_scale<<<64, kScaleBlock, 0, st>>>(X, ldx, n, nrhs, scale);
+            k_split_panel<<<(unsigned)((nchunks + 1) / 2), kBlock, 0, st>>>(P, n, nchunks, scale, V3, skip);
             k_bmm32s<<<grid, kBlock, 0, st>>>(A32, n, V3, pc, part, skip);
-            k_bmm32_reduce<64><<<(unsigned)((n + kReduceRows - 1) / kReduceRows), kBlock, 0, st>>>(part, nc, n, nrhs, Y, ldy, skip);
+            const unsigned gr = (unsigned)((n + kReduceRows - 1) / kReduceRows);
+            if (scale)
+                k_bmm32_reduce<64, float, true><<<gr, kBlock, 0, st>>>(part, nc, n, nrhs, Y, ldy, skip, A32, P, scale);
+            else
+                k_bmm32_reduce<64><<<gr, kBlock, 0, st>>>(part, nc, n, nrhs, Y, ldy, skip);
             return hipGetLastError();
         }
         if (launch_tuning().bmm_rows == 128 && n % 4 == 0 && n >= 4) {

@@ -179,6 +179,38 @@ def test_block_product_fp32_split(ctx, coax, n, rhs):
     assert np.all(np.abs(Y - A32 @ X) <= bound * (np.abs(A32) @ np.abs(X)))
 
 
+@pytest.mark.parametrize("n", [20, 260, 1280])
+def test_block_product_fp32_split_outside_range(ctx, coax, n):
+    """What the three BF16 parts of a number cannot hold: infinite right-hand sides, those past the largest FP32 number, and
+    columns of numbers so small that their third parts underflow.  The same results as 32 right-hand sides give, whose
+    kernel takes FP32 numbers whole."""
+    from kassiopeia_amd import kemfield as K
+
+    m = _first_elements(coax[0], n)
+    A = K.KBoundaryIntegralMatrix(K.KSurfaceContainer(ctx, m), fp64=True, fp32=True)
+    X = np.random.default_rng(n).normal(size=(n, 64))
+    X[7, 3], X[9, 4], X[0, 6], X[5, 40] = np.inf, 1e60, -np.inf, np.inf
+    X[6, 40] = -np.inf  # of both signs: not a number
+    X[2, 41] = np.nan
+    for c, e in ((10, -66), (11, -100), (12, -112), (50, -118), (51, -126)):
+        X[:, c] *= 2.0 ** e
+    X[:, 52] = 0.0
+    Y = A.MultiplyBatch(X, "mixed")
+    ref = np.hstack([A.MultiplyBatch(X[:, :32], "mixed"), A.MultiplyBatch(X[:, 32:], "mixed")])
+    assert np.array_equal(np.isnan(Y), np.isnan(ref)) and np.isnan(Y[:, 40:42]).all()
+    inf = np.isinf(ref)
+    assert np.array_equal(Y[inf], ref[inf]) and inf[:, [3, 4, 6]].all()
+    ok = np.isfinite(ref).all(0)
+    assert np.isfinite(Y[:, ok]).all()
+    # both sum FP32 numbers: as test_block_product_fp32_split and test_block_product_fp32_mfma have it
+    scale = np.abs(A.to_numpy()) @ np.abs(X[:, ok])
+    assert np.all(np.abs(Y[:, ok] - ref[:, ok]) <= 2.5e-6 * scale)
+    A32 = A.to_numpy().astype(np.float32).astype(np.float64)
+    exact = A32 @ X[:, ok].astype(np.float32).astype(np.float64)
+    bound = (64 + 0.5 * (n / 128 + 8)) * 2.0 ** -23
+    assert np.all(np.abs(Y[:, ok] - exact) <= bound * (np.abs(A32) @ np.abs(X[:, ok])))
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_solve_batch_voltage_sets(coax, precision):
     """16 ring groups x 12 voltage sets (U[-1000, 0] V per group): every column converges to
