@@ -27,7 +27,7 @@ constexpr double kMixedFp64RatioDefault = 0.0;
 // the inner tolerance of BF16-matrix solves: the BF16 product rounds its input vector to 8
 // significant bits, so an inner solve cannot reduce its true residual much below 2^-8
 constexpr double kBf16InnerTolerance = 1.0 / 256.0;
-// host-array calls of up to this size go through page-locked memory
+// host-array calls of up to this size go through memory kept on the context
 constexpr size_t kStageBytes = (size_t)16 << 20;
 // elements per XCD range of the large single-set far passes (kem::launch_field); 0 = no split
 constexpr int64_t kFarRangeDefault = 2560;
@@ -80,7 +80,7 @@ struct kem_ctx {
     double* scal = nullptr;  // small device scalars (dot products, Hessenberg column)
     int64_t scal_doubles = 0;
     FieldWs fws;  // workspace of eager field evaluations (grow-only)
-    // staging of host-array calls: device memory, and page-locked host memory for calls of up to kStageBytes (grow-only)
+    // staging of host-array calls of up to kStageBytes, in device memory and page-locked host memory (grow-only)
     double* io = nullptr;
     int64_t io_doubles = 0;
     double* pin = nullptr;
@@ -189,8 +189,10 @@ void dfree(T*& p)
     p = nullptr;
 }
 
+void ws_release(FieldWs& w);
+
 // matrix storage: a cached block of exactly this size, else a new allocation (after releasing
-// the cache if the first attempt fails)
+// the cache, and what field calls keep on the context, if the first attempt fails)
 template <typename T>
 hipError_t store_alloc(kem_ctx* c, T** p, int64_t count)
 {
@@ -204,10 +206,14 @@ hipError_t store_alloc(kem_ctx* c, T** p, int64_t count)
             return hipSuccess;
         }
     hipError_t e = hipMalloc((void**)p, bytes);
-    if (e != hipSuccess && !c->store_cache.empty()) {
+    if (e != hipSuccess) {
         (void)hipGetLastError();
         for (auto& b : c->store_cache) (void)hipFree(b.first);
         c->store_cache.clear();
+        // hipFree waits for the device, so no call still reads these
+        ws_release(c->fws);
+        dfree(c->io);
+        c->io_doubles = 0;
         e = hipMalloc((void**)p, bytes);
     }
     return e;
@@ -1119,13 +1125,16 @@ int kem_field_eval(kem_ctx* c, const kem_mesh* m, const double* sigma, int64_t n
     if (!c || !m || !sigma || (npts > 0 && !P)) return KEM_E_ARG;
     if (npts <= 0) return KEM_OK;
     KEM_CK(c, enter(c));
-    // sigma, x, y, z in one block of device memory, then phi, Ex, Ey, Ez; kept on the context, as is a page-locked
-    // block of host memory that small calls pass through in one copy each way (allocating, freeing and copying
-    // pageable memory took 120 us of a call of 64 points)
+    // sigma, x, y, z in one block of device memory, then phi, Ex, Ey, Ez.  For calls of up to kStageBytes it is kept on the
+    // context, as is a page-locked block of host memory that they pass through in one copy each way (allocating, freeing
+    // and copying pageable memory took 120 us of a call of 64 points); larger calls allocate and free theirs.
     const int64_t in = m->n + 3 * npts, total = in + 4 * npts;
     const bool staged = sizeof(double) * (size_t)total <= kStageBytes;
+    DVec own;
     hipError_t e = hipSuccess;
-    if (c->io_doubles < total) {
+    if (!staged) {
+        e = dalloc(&own.p, total);
+    } else if (c->io_doubles < total) {
         dfree(c->io);
         c->io_doubles = 0;
         e = dalloc(&c->io, total);
@@ -1135,21 +1144,27 @@ int kem_field_eval(kem_ctx* c, const kem_mesh* m, const double* sigma, int64_t n
         if (c->pin) (void)hipHostFree(c->pin);
         c->pin = nullptr;
         c->pin_doubles = 0;
-        e = hipHostMalloc((void**)&c->pin, sizeof(double) * (size_t)total, hipHostMallocDefault);
-        if (e == hipSuccess) c->pin_doubles = total;
+        if (hipHostMalloc((void**)&c->pin, sizeof(double) * (size_t)total, hipHostMallocDefault) == hipSuccess) {
+            c->pin_doubles = total;
+        } else {
+            c->pin = nullptr;  // pageable memory then
+            (void)hipGetLastError();
+        }
     }
     if (e != hipSuccess) return fail(c, KEM_E_HIP, std::string("field_eval: ") + hipGetErrorString(e));
-    std::vector<double> pageable(staged ? 0 : (size_t)total);
-    double* h = staged ? c->pin : pageable.data();
+    const bool pinned = staged && c->pin_doubles >= total;
+    double* io = staged ? c->io : own.p;
+    std::vector<double> pageable(pinned ? 0 : (size_t)total);
+    double* h = pinned ? c->pin : pageable.data();
     std::memcpy(h, sigma, sizeof(double) * (size_t)m->n);
     double* hx = h + m->n;
     for (int64_t i = 0; i < npts; i++)
         for (int k = 0; k < 3; k++) hx[(size_t)k * npts + i] = P[3 * i + k];
-    e = hipMemcpyAsync(c->io, h, sizeof(double) * (size_t)in, hipMemcpyHostToDevice, c->stream);
+    e = hipMemcpyAsync(io, h, sizeof(double) * (size_t)in, hipMemcpyHostToDevice, c->stream);
     int rc = KEM_OK;
     if (e == hipSuccess) {
-        double *dP = c->io + m->n, *dO = c->io + in;
-        rc = kem_field_eval_device(c, m, c->io, npts, dP, dP + npts, dP + 2 * npts, precision, dO, dO + npts,
+        double *dP = io + m->n, *dO = io + in;
+        rc = kem_field_eval_device(c, m, io, npts, dP, dP + npts, dP + 2 * npts, precision, dO, dO + npts,
                                    dO + 2 * npts, dO + 3 * npts);
         if (rc == KEM_OK) {
             const double* o = h + in;

@@ -1,7 +1,10 @@
 """Matrix storage handed back to the context on kem_matrix_destroy and reused by the next
 assembly of the same size: a matrix assembled into reused storage equals, bit for bit, the same
 matrix assembled into fresh storage on another context (every entry rewritten, nothing of the
-previous matrix left), in FP64, FP32 and BF16, with a matrix of another size in between."""
+previous matrix left), in FP64, FP32 and BF16, with a matrix of another size in between.  Host-array
+field calls: what they allocate beyond a few MiB goes back when they return."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -45,3 +48,55 @@ def test_matrix_storage_reuse():
     finally:
         ctx.close()
         fresh.close()
+
+
+def _free_memory():
+    """Bytes free on the device, from the runtime that the library has loaded."""
+    with open("/proc/self/maps") as maps:
+        path = next(line.split()[-1] for line in maps if "libamdhip64" in line)
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+def test_host_field_calls_give_memory_back():
+    from kassiopeia_amd import kemfield as K
+
+    m = G.cube_mesh(4)
+    ctx = K.Context(0)
+    try:
+        cont = K.KSurfaceContainer(ctx, m)
+        solver = K.KIntegratingElectrostaticFieldSolver(cont, np.full(m.n, 1e-9))
+        npts = 1_000_000  # 56 MB of points and results
+        pts = G.points_shell(npts, 1.0, 2.0, 1)
+        E, phi = solver.ElectricFieldAndPotential(pts)  # and the workspace of such calls, which stays
+        few = solver.ElectricFieldAndPotential(pts[:1000])
+        free = _free_memory()
+        own = 8 * (m.n + 7 * npts)
+        # the workspace through device arrays alone, on a context that never took host arrays
+        other = K.Context(0)
+        oc = K.KSurfaceContainer(other, m)
+        S = K.DeviceArray(other, np.full(m.n, 1e-9))
+        X = [K.DeviceArray(other, np.ascontiguousarray(pts[:, k])) for k in range(3)]
+        O = [K.DeviceArray.empty(other, npts) for _ in range(4)]
+        before = _free_memory()
+        other.check(other.lib.kem_field_eval_device(other.h, oc.h, S.ptr, npts, X[0].ptr, X[1].ptr, X[2].ptr, 0,
+                                                    O[0].ptr, O[1].ptr, O[2].ptr, O[3].ptr))
+        other.sync()
+        workspace = before - _free_memory()
+        assert np.array_equal(np.stack([o.get() for o in O[1:]], 1), E) and np.array_equal(O[0].get(), phi)
+        assert np.allclose(few[1], phi[:1000], rtol=1e-12)
+        for a in X + O + [S]:
+            a.close()
+        oc.close()
+        other.close()
+        cont.close()
+        ctx.close()
+        ctx = None
+        # what the host-array context still held: its workspace, and of the staging no more than 16 MiB (and as much slack
+        # for the allocator's pages)
+        held = _free_memory() - free
+        assert held <= workspace + (32 << 20) < workspace + own
+    finally:
+        if ctx is not None:
+            ctx.close()
