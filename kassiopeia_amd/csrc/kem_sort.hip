@@ -7,9 +7,12 @@
 // 64 points of a wavefront neighbours, so they almost always share one regime, and close to each other, so
 // the hierarchical pass accepts more expansions for them.  (A Morton curve's jumps left groups of points up to
 // 8 times the usual size, whose wavefronts ran 20 times longer than the others.)
-// The results are gathered back to the caller's order; each point's value does not depend on
-// the ordering.
+// The results are gathered back to the caller's order.  In its last digits a point's value depends on the
+// ordering, and so on the call's other points: which pairs of a wavefront share a rule, and which runs of elements are
+// taken as expansions, follows from the points visited with it.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 #include <hipcub/hipcub.hpp>
 
 #include <cstdint>
@@ -64,14 +67,17 @@ __device__ __forceinline__ uint64_t spread3(uint64_t a)
     return v;
 }
 
-// Hilbert key (kCurveBits bits per axis) of each point in the cube over the box spanned by the block
-// partials: J. Skilling, "Programming the Hilbert curve" (2004), axes to transposed index.  pset (nullable): the set
+// Hilbert key (bits per axis) of each point in the cube over the box spanned by the block
+// partials: as many bits as the key holds, up to 21, since a stray point far from the others (a lost particle) widens the
+// cube: at 1e5 times their extent it leaves them 21 cells per axis, and at 16 bits one, with
+// which 200,000 points in a random order over 20,000 triangles took 61.5 ms instead of 7.0 (mixed).  J. Skilling, "Programming the Hilbert curve" (2004), axes to transposed index.  pset (nullable): the set
 // above the curve's bits, for the hierarchical pass.  The flat passes' points of several charge-density sets sort
 // together: their kernels read the sets element-major, so a wavefront may mix sets.
-constexpr int kCurveBits = 16;
+constexpr int kCurveBits = 21;
+inline int curve_bits(int set_bits) { return std::min(kCurveBits, (64 - set_bits) / 3); }
 __global__ __launch_bounds__(kBlock) void k_curve(const double* __restrict__ x, const double* __restrict__ y,
                                                   const double* __restrict__ z, int64_t n,
-                                                  const int32_t* __restrict__ pset,
+                                                  const int32_t* __restrict__ pset, int bits,
                                                   const double* __restrict__ part, int nparts,
                                                   uint64_t* __restrict__ key, int32_t* __restrict__ idx)
 {
@@ -96,14 +102,14 @@ __global__ __launch_bounds__(kBlock) void k_curve(const double* __restrict__ x, 
     const double v[3] = {x[i], y[i], z[i]};
     double span = 0.;
     for (int k = 0; k < 3; k++) span = fmax(span, sh[3 + k][0] - sh[k][0]);
-    constexpr double kMost = (1 << kCurveBits) - 1;
+    const double most = (1 << bits) - 1;
     uint32_t a[3];
     for (int k = 0; k < 3; k++) {
-        double q = span > 0. ? (v[k] - sh[k][0]) / span * kMost : 0.;
-        q = q > 0. ? (q > kMost ? kMost : q) : 0.;
+        double q = span > 0. ? (v[k] - sh[k][0]) / span * most : 0.;
+        q = q > 0. ? (q > most ? most : q) : 0.;
         a[k] = (uint32_t)q;
     }
-    for (uint32_t q = 1u << (kCurveBits - 1); q > 1; q >>= 1) {
+    for (uint32_t q = 1u << (bits - 1); q > 1; q >>= 1) {
         const uint32_t p = q - 1;
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -119,9 +125,9 @@ __global__ __launch_bounds__(kBlock) void k_curve(const double* __restrict__ x, 
     a[1] ^= a[0];
     a[2] ^= a[1];
     uint32_t t = 0;
-    for (uint32_t q = 1u << (kCurveBits - 1); q > 1; q >>= 1)
+    for (uint32_t q = 1u << (bits - 1); q > 1; q >>= 1)
         if (a[2] & q) t ^= q - 1;
-    const uint64_t set = pset ? (uint64_t)(uint32_t)pset[i] << (3 * kCurveBits) : 0;
+    const uint64_t set = pset ? (uint64_t)(uint32_t)pset[i] << (3 * bits) : 0;
     key[i] = set | spread3(a[2] ^ t) | spread3(a[1] ^ t) << 1 | spread3(a[0] ^ t) << 2;
     idx[i] = (int32_t)i;
 }
@@ -210,13 +216,14 @@ hipError_t launch_field_sorted(hipStream_t st, int policy, const FieldMesh& m, b
     if (nb > kBoxParts) nb = kBoxParts;
     k_bbox_part<<<nb, kBlock, 0, st>>>(px, py, pz, npts, box);
     // the hierarchical pass takes the points set by set (as launch_field decides)
-    int bits = 3 * kCurveBits;
+    int set_bits = 0;
     const TreePlan tp = plan_tree(policy, m, mixed, fp64_ratio, pset != nullptr, nsets, npts);
     const bool by_set = pset && tp.use && tp.doubles() <= ws_doubles;
     if (by_set)
-        for (int64_t v = nsets - 1; v > 0; v >>= 1) bits++;
-    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, by_set ? pset : nullptr, box, nb, k0, i0);
-    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, bits, st);
+        for (int64_t v = nsets - 1; v > 0; v >>= 1) set_bits++;
+    const int bits = curve_bits(set_bits);
+    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, by_set ? pset : nullptr, bits, box, nb, k0, i0);
+    hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 3 * bits + set_bits, st);
     if (e != hipSuccess) return e;
     k_gather3<<<nblocks(npts), kBlock, 0, st>>>(i1, px, py, pz, pset, npts, sx, sy, sz, ss);
     e = launch_field(st, policy, m, mixed, fp64_ratio, sigma, pset ? ss : nullptr, nsets, sx, sy, sz, npts, o[0], o[1],
@@ -255,7 +262,7 @@ hipError_t launch_census_paths_sorted(hipStream_t st, const FieldMesh& m, const 
     int nb = (int)((npts + kBlock - 1) / kBlock);
     if (nb > kBoxParts) nb = kBoxParts;
     k_bbox_part<<<nb, kBlock, 0, st>>>(px, py, pz, npts, box);
-    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, nullptr, box, nb, k0, i0);
+    k_curve<<<nblocks(npts), kBlock, 0, st>>>(px, py, pz, npts, nullptr, kCurveBits, box, nb, k0, i0);
     hipError_t e = hipcub::DeviceRadixSort::SortPairs(tmp, tb, k0, k1, i0, i1, (int)npts, 0, 3 * kCurveBits, st);
     if (e != hipSuccess) return e;
     k_gather3<<<nblocks(npts), kBlock, 0, st>>>(i1, px, py, pz, nullptr, npts, sx, sy, sz, ss);

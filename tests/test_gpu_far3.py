@@ -58,6 +58,18 @@ def test_far3_against_fp64(sphere, shell):
         assert c[0] == 0 and c[1] > 0, c
 
 
+def test_order_with_a_stray_point(ctx, sphere):
+    """One point 1e5 times as far away as the others leaves these enough cells of the curve's cube to be grouped: the pairs that
+    compact groups take by the clusters' 3-point rule stay with it."""
+    m, cont, x = sphere
+    pts = G.points_shell(20000, 10.0, 40.0, seed=41)
+    alone = paths(cont, pts)[0]
+    stray = pts.copy()
+    stray[777] = [4e6, -3e6, 2e6]
+    # 21 cells along each axis against groups of a seventh of it
+    assert paths(cont, stray)[0] >= 0.9 * alone > 0
+
+
 def paths(cont, pts):
     import ctypes
 
