@@ -290,7 +290,7 @@ def run_bore(ctx, args):
         t0 = time.perf_counter()
         sig0 = np.full(N, 1e-9)  # the time per pair does not depend on the charge densities
         sample = pts[:min(args.tune_points, M)] if args.tune_points > 0 else pts
-        # the ranges of the flat far passes; a hierarchical pass (this size) does not depend on them
+        # the ranges of the flat far passes; nothing is swept where the hierarchical pass serves the points (this size)
         cands = (640, 2560, 10240)
         tuning = {"far_range_mixed": T.tune_field(cont, sig0, sample, "mixed", repeats=1, candidates=cands),
                   "far_range_fp64": T.tune_field(cont, sig0, sample, "fp64", repeats=1, candidates=cands)}

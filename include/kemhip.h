@@ -271,6 +271,11 @@ int kem_field_census(kem_ctx* ctx, const kem_mesh* mesh, int64_t npts, const dou
 int kem_field_census_paths(kem_ctx* ctx, const kem_mesh* mesh, int64_t npts, const double* d_x, const double* d_y,
                            const double* d_z, int64_t* counts);
 
+/* 1 when a field evaluation of npts points of the mesh takes the hierarchical pass, which has no element
+   ranges and no near pass of its own to tune (nsets = 0: kem_field_eval_device and its kin; else
+   kem_field_eval_sets), 0 when it takes the flat ones.  No reference counterpart; host arithmetic only. */
+int kem_field_hierarchical(kem_ctx* ctx, const kem_mesh* mesh, int64_t nsets, int64_t npts, int precision);
+
 /* Instrumentation (no reference counterpart; host arithmetic only, no device access): how the flat passes of a
    field evaluation of npts points over nelem elements splits into element ranges and partial
    sums, for a mesh with (clustered = 1: triangles / rectangles / segments, numeric policy) or

@@ -111,6 +111,7 @@ SIGNATURES = {
     "kem_field_eval_fields": (_INT, [_P, _I64, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _P]),
     "kem_field_eval_sets": (_INT, [_P, _P, _I64, _P, _P, _I64, _P, _P, _P, _INT, _P, _P, _P, _P]),
     "kem_field_census": (_INT, [_P, _P, _I64, _P, _P, _P, _INT, _P]),
+    "kem_field_hierarchical": (_INT, [_P, _P, _I64, _I64, _INT]),
     "kem_field_census_paths": (_INT, [_P, _P, _I64, _P, _P, _P, _P]),
     "kem_zh_params_default": (None, [ctypes.POINTER(ZHParams)]),
     "kem_zh_create": (_INT, [_P, _P, _P, ctypes.POINTER(ZHParams), ctypes.POINTER(_P)]),

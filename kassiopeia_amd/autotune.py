@@ -3,7 +3,7 @@
 The C-ABI exposes these launch-shape knobs (``kem_ctx_set_tuning``):
 
 * ``KEM_TUNE_FAR_RANGE_FP64`` / ``KEM_TUNE_FAR_RANGE_MIXED``: elements per element range of the
-  far field pass over large point sets.  The elements split into 8 R ranges, R per XCD, so the
+  flat far field pass over large point sets.  The elements split into 8 R ranges, R per XCD, so the
   range an XCD works on stays in its L2; 0 disables the split.
 * ``KEM_TUNE_GEMV_BLOCKS``: target block count of the split-K matrix-vector product (GMRES,
   Robin Hood residuals, ``KSquareMatrix::Multiply``).
@@ -14,7 +14,7 @@ The C-ABI exposes these launch-shape knobs (``kem_ctx_set_tuning``):
 * ``KEM_TUNE_BMM_TILE_BLOCKS``: largest workgroup count of the streamed block products of up
   to 32 right-hand sides (16 x 16 MFMA tiles: FP32 when n % 4 == 0, FP64 when n is even; one
   32-column tile: BF16).
-* ``KEM_TUNE_NEAR_BLOCKS``: blocks of the near pass that runs beside the mixed far pass on a
+* ``KEM_TUNE_NEAR_BLOCKS``: blocks of the near pass that runs beside the flat mixed far pass on a
   second stream (0: one per 256 points).  Its timed region is the whole field pass.
 * ``KEM_TUNE_BMM_ROWS``: the wavefront tile of the FP32 MFMA block product, 64 rows (one float
   per lane and column) or 128 rows (a 16-byte load of four rows per lane feeding four MFMAs).
@@ -92,13 +92,26 @@ def _sweep(ctx, name, candidates, run, repeats, wall=False):
     return {"best": best, "ms": times}
 
 
+def _hierarchical(container: K.KSurfaceContainer, npts: int, precision: str) -> bool:
+    """Whether a field call of npts points takes the hierarchical pass, which the far and near knobs do not shape."""
+    ctx = container.ctx
+    r = ctx.lib.kem_field_hierarchical(ctx.h, container.h, 0, npts,
+                                       {"fp64": _lib.KEM_FP64, "mixed": _lib.KEM_MIXED}[precision])
+    if r < 0:
+        ctx.check(r)
+    return bool(r)
+
+
 def tune_field(container: K.KSurfaceContainer, sigma, points, precision="mixed", repeats=2,
                candidates=FAR_RANGE_CANDIDATES):
     """Element-range size of the far pass for this container, charge densities and points
-    (points: (m, 3) array; the split applies from 262,144 points on)."""
+    (points: (m, 3) array; the split applies from 262,144 points on).  Nothing is run, and the knob stays, where
+    the hierarchical pass serves the call."""
     ctx = container.ctx
     P = np.asarray(points, dtype=np.float64).reshape(-1, 3)
     m = P.shape[0]
+    if _hierarchical(container, m, precision):
+        return {"best": get(ctx, "far_range_" + precision), "ms": {}}
     X = [K.DeviceArray(ctx, np.ascontiguousarray(P[:, k])) for k in range(3)]
     S = K.DeviceArray(ctx, np.asarray(sigma, dtype=np.float64))
     O = [K.DeviceArray.empty(ctx, m) for _ in range(4)]
@@ -116,10 +129,13 @@ def tune_field(container: K.KSurfaceContainer, sigma, points, precision="mixed",
 
 
 def tune_near(container: K.KSurfaceContainer, sigma, points, repeats=3, candidates=NEAR_CANDIDATES):
-    """Grid of the near pass beside the mixed far pass, timed over the whole field pass."""
+    """Grid of the near pass beside the mixed far pass, timed over the whole field pass.  Nothing is run, and the knob
+    stays, where the hierarchical pass serves the call."""
     ctx = container.ctx
     P = np.asarray(points, dtype=np.float64).reshape(-1, 3)
     m = P.shape[0]
+    if _hierarchical(container, m, "mixed"):
+        return {"best": get(ctx, "near_blocks"), "ms": {}}
     X = [K.DeviceArray(ctx, np.ascontiguousarray(P[:, k])) for k in range(3)]
     S = K.DeviceArray(ctx, np.asarray(sigma, dtype=np.float64))
     O = [K.DeviceArray.empty(ctx, m) for _ in range(4)]

@@ -1035,6 +1035,20 @@ int kem_field_eval_sets(kem_ctx* c, const kem_mesh* m, int64_t nsets, const doub
     return field_eval(c, m, sigma, set, nsets, npts, x, y, z, precision, phi, ex, ey, ez, c->fws, true);
 }
 
+int kem_field_hierarchical(kem_ctx* c, const kem_mesh* m, int64_t nsets, int64_t npts, int precision)
+{
+    if (!c || !m || nsets < 0 || npts < 0) return KEM_E_ARG;
+    if (m->ctx != c) return fail(c, KEM_E_STATE, "mesh belongs to another context");
+    if (precision != KEM_FP64 && precision != KEM_MIXED) return fail(c, KEM_E_ARG, "field: unknown precision mode");
+    kem::FieldMesh fm;
+    field_mesh(m, fm);
+    return kem::plan_tree(c->policy, fm, precision == KEM_MIXED, c->mixed_fp64_ratio, nsets > 0,
+                          std::max<int64_t>(nsets, 1), npts)
+                   .use
+               ? 1
+               : 0;
+}
+
 int kem_field_plan(int policy, int clustered, int precision, int multi, int64_t nelem, int64_t nsets, int64_t npts,
                    int64_t range_elems, int64_t ws_doubles, int64_t* out)
 {

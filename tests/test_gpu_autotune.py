@@ -47,6 +47,36 @@ def test_tune_field(setup, precision):
     T.set_knob(ctx, "far_range_" + precision, 2560)
 
 
+def test_hierarchical_calls_are_not_swept(setup):
+    """Calls that the hierarchical pass serves depend neither on the far ranges nor on the near grid: no sweep, and the knobs
+    stay as they are."""
+    from kassiopeia_amd import autotune as T
+    from kassiopeia_amd import kemfield as K
+
+    ctx = setup[0]
+    m = G.cube_mesh(18)  # 3,888 triangles
+    cont = K.KSurfaceContainer(ctx, m)
+    sigma = np.full(m.n, 1e-9)
+    pts = G.points_shell(300_000, 1.0, 2.0, 3)
+    try:
+        for knob in ("far_range_fp64", "far_range_mixed"):
+            T.set_knob(ctx, knob, 1280)
+        for precision in ("fp64", "mixed"):
+            assert T.tune_field(cont, sigma, pts, precision, candidates=(0, 640)) == {"best": 1280, "ms": {}}
+        near = T.get(ctx, "near_blocks")
+        assert T.tune_near(cont, sigma, pts) == {"best": near, "ms": {}} and T.get(ctx, "near_blocks") == near
+        lib = ctx.lib
+        assert lib.kem_field_hierarchical(ctx.h, cont.h, 0, 300_000, 0) == 1
+        assert lib.kem_field_hierarchical(ctx.h, cont.h, 0, 1000, 0) == 0
+        assert lib.kem_field_hierarchical(ctx.h, cont.h, 64, 300_000, 1) == 0
+        assert lib.kem_field_hierarchical(ctx.h, cont.h, 2, 300_000, 1) == 1
+        assert lib.kem_field_hierarchical(ctx.h, cont.h, 0, 300_000, 2) == -1
+    finally:
+        for knob in ("far_range_fp64", "far_range_mixed"):
+            T.set_knob(ctx, knob, 2560)
+        cont.close()
+
+
 def test_tune_products(setup):
     from kassiopeia_amd import autotune as T
 
