@@ -163,6 +163,28 @@ def test_tree_one_charged_element(ctx, kind, n, precision):
     cont.close()
 
 
+@pytest.mark.parametrize("n,npts,precision", [(36000, 20001, "fp64"), (64000, 20001, "mixed"), (140000, 8193, "fp64"),
+                                              (240000, 8193, "mixed")])
+def test_tree_coarser_lowest_runs(ctx, n, npts, precision):
+    """Up to 65,536 points the lowest runs expanded hold 64 elements from about 33,000 (FP64) or 58,000 (mixed) on, and
+    256 from four times as many: several rounds of 16 elements in each expansion, levels from the second or third on."""
+    from kassiopeia_amd import kemfield as K
+
+    m = G.ring_bore_mesh(n_target=n, volts=np.zeros(32))
+    cont = K.KSurfaceContainer(ctx, m)
+    rng = np.random.default_rng(n)
+    pts = G.points_annulus(npts, 0.0, 1.88, 4.0, 7)
+    some = np.unique(np.concatenate([[0, npts - 1], rng.integers(0, npts, 3000)]))
+    tol = 1e-13 if precision == "fp64" else 1e-6  # as for runs of 16
+    c = m.centroids()
+    for sigma in (1e-9 * rng.normal(size=m.n), 1e-9 * (1.0 + 0.5 * np.sin(3.0 * c[:, 2] + c[:, 0]))):
+        E0, p0 = flat(cont, sigma, pts[some], "fp64")
+        E, phi = K.KIntegratingElectrostaticFieldSolver(cont, sigma, precision).ElectricFieldAndPotential(pts)
+        assert np.linalg.norm(E[some] - E0) <= tol * np.linalg.norm(E0)
+        assert np.linalg.norm(phi[some] - p0) <= tol * np.linalg.norm(p0)
+    cont.close()
+
+
 @pytest.mark.parametrize("kind,n,npts,sets,precision", [
     ("triangles", 4007, 40001, 4, "fp64"), ("frame", 3219, 262147, 24, "fp64"), ("groups", 4800, 33000, 3, "fp64"),
     ("triangles", 4007, 150001, 3, "mixed"), ("triangles", 4992, 262149, 6, "mixed"),

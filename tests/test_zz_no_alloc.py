@@ -1,8 +1,9 @@
 """The no-allocation field entry point (kem_field_eval_device_noalloc) against the eager one
 (kem_field_eval_device), through the C-ABI: the same kernels and sums, so bit-equal outputs,
 on two calls in a row, the second with a smaller input (the static scratch keeps the first
-call's contents), in both precisions and on a mesh with symmetry groups; sizes beyond the
-scratch are refused before any device work."""
+call's contents), in both precisions and on a mesh with symmetry groups; calls that the hierarchical
+pass serves, whose expansions lie in the scratch too; sizes beyond the scratch are refused before any
+device work."""
 import ctypes
 
 import numpy as np
@@ -70,6 +71,33 @@ def test_noalloc_groups(ctx):
         pts = G.points_shell(npts, 0.9, 3.0, seed)
         ref = run(ctx, cont, S, pts, 0, False)
         got = run(ctx, cont, S, pts, 0, True)
+        assert np.array_equal(got, ref)
+    S.close()
+    cont.close()
+
+
+@pytest.mark.parametrize("kind", ["triangles", "many", "groups"])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_noalloc_hierarchical(ctx, kind, precision):
+    """Sizes that the hierarchical pass serves: the largest number of points, meshes whose lowest runs are coarsened for
+    the scratch, symmetry groups, whose charge densities lie beside the expansions."""
+    from kassiopeia_amd import kemfield as K
+
+    if kind == "triangles":
+        mesh = G.coax_mesh(nphi_in=24, nphi_out=48, nz=31, ncap_r=4, ncap_phi=33)
+    elif kind == "many":
+        mesh = G.ring_bore_mesh(n_target=70000, volts=np.zeros(32))
+    else:
+        mesh = G.mirror_groups(G.cube_mesh(20), [0.0, 0.0, 2.0], [0.0, 0.0, 1.0])
+    cont = K.KSurfaceContainer(ctx, mesh)
+    S = K.DeviceArray(ctx, np.random.default_rng(2).normal(size=cont.size()) * 1e-10)
+    for npts, seed in ((65536, 3), (24001, 4)):
+        assert ctx.lib.kem_field_hierarchical(ctx.h, cont.h, 0, npts, precision) == 1
+        pts = G.points_annulus(npts, 0.0, 1.88, 4.0, seed) if kind == "many" else G.points_shell(npts, 0.9, 3.0, seed)
+        print(f"noalloc: {kind}, precision {precision}, {npts} points", flush=True)
+        ref = run(ctx, cont, S, pts, precision, False)
+        got = run(ctx, cont, S, pts, precision, True)
+        assert np.all(np.isfinite(got))
         assert np.array_equal(got, ref)
     S.close()
     cont.close()
