@@ -51,11 +51,11 @@ def test_matrix_storage_reuse():
 
 
 def _free_memory():
-    """Bytes free on the device, from the runtime that the library has loaded."""
-    with open("/proc/self/maps") as maps:
-        path = next(line.split()[-1] for line in maps if "libamdhip64" in line)
+    """Bytes free on the device, from the runtime that the library is linked to."""
+    from kassiopeia_amd import _lib
+
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
-    assert ctypes.CDLL(path).hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    assert _lib.load().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
     return free.value
 
 
