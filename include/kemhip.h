@@ -43,7 +43,10 @@ extern "C" {
 #define KEM_POLICY_REFERENCE 3 /* nested 32-node Gauss-Legendre (segments: 8 x 32 nodes) */
 
 /* ---- precision modes */
-#define KEM_FP64 0  /* plain path: FP64 everywhere */
+#define KEM_FP64 0  /* plain path: FP64 everywhere.  Field calls of many points over many elements take far runs of
+                       elements as truncated expansions, to the accuracy of the pairs' own rules
+                       (kem_field_hierarchical says which); the last digits of a point's value there depend on the
+                       call's other points */
 #define KEM_MIXED 1 /* FP32 far-field cubature / FP32 matrix; FP64 near field, refinement, sums */
 #define KEM_MIXED_BF16 2 /* solves and block products only: BF16 matrix on BF16 MFMA (FP32 accumulation),
                             FP64 refinement */
@@ -196,7 +199,8 @@ int kem_element_eval(kem_ctx* ctx, const kem_mesh* mesh, int64_t npairs, const i
 /* ---- direct field: KIntegratingFieldSolver<KElectrostaticBoundaryIntegrator, Kind>::
    ElectricFieldAndPotential (FieldSolvers/Integrating/include/KElectrostaticIntegratingFieldSolver.hh:303-339),
    fused (one pass) and batched over points.  Host arrays, synchronous: P is npts x 3 (AoS),
-   sigma has mesh-size entries; phi (npts) and E (npts x 3) may be NULL to skip. */
+   sigma has mesh-size entries; phi (npts) and E (npts x 3) may be NULL to skip.  Calls of up to 16 MiB
+   (56 bytes a point) pass through memory kept on the context, larger ones allocate and free theirs. */
 int kem_field_eval(kem_ctx* ctx, const kem_mesh* mesh, const double* sigma, int64_t npts, const double* P,
                    int precision, double* phi, double* E);
 /* Same on device arrays (SoA point streams), asynchronous on the context's stream.

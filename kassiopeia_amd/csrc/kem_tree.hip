@@ -2,7 +2,8 @@
 //
 // A field evaluation at many points spends its time on pairs far apart.  Elements lie in
 // compact runs of KEM_TREE_LEAF, KEM_TREE_FAN of which make the next level's run (kem::build_tree).  Each call
-// expands the charge of every run about its centre (k_tree_p2m for the lowest level, k_tree_m2m upwards),
+// expands the charge of every run about its centre (k_tree_p2m for the lowest level, k_tree_m2m upwards), finds how far
+// from it the charge lies (k_tree_reach),
 // and each wavefront walks the tree for its 64 points: a run far enough from all of them is one expansion,
 // of the order that its distance asks for, and the rest of the elements go pair by pair through the
 // same rules as the flat far passes (k_field_far, k_field_far32c).  Expansions are FP64 in both precisions.
@@ -44,14 +45,14 @@ __host__ __device__ constexpr int tri_index(int l, int m) { return l * (l + 1) /
 //   sum_{l > p} (l + 1) q^l (1 - q)^2 = ((p + 2) - (p + 1) q) q^(p+1) <= tol,
 // the field's omitted part against the field of the charge rho a from the centre on the points' side (L past the order
 // stored and a / d < widest bound what rho does not).  Each call finds rho a of each run (k_tree_reach): at the rim it
-// is a, for the elements of a surface 0.85 of it, which saves two orders.
+// is a, for the elements of a surface 0.8 to 0.9 of it.
 // The tolerances keep every point's field as good as the pairs' own rules do it, whatever the charges: one
 // charged element at the rim of a run of any level (of 16 to 4,096 elements: 20,000-triangle coax, 100,000-triangle bore, a
 // cube, rectangles and wires), points in clumps beyond it, worst / root mean square error of the field: FP64 3.3e-14 / 2.8e-15
 // both here and in the flat passes, mixed 4.0e-7 / 1.0e-7 in both (with (a / d)^(p+1) <= 8e-14 and 7e-7, the bound of the
 // potential, 8.5e-13 and 4.5e-6).
-// The orders: a million points over 20,000 triangles, mixed, 19.5 ms at 20, 19.2 at 21, 19.0 at 22, where 400,000
-// over 100,000 take 9.0 instead of 8.7; 100,000 points over 20,000 triangles, FP64, 14.9 ms at 26, 13.5 at 28, 13.0 at 30.
+// The orders (at 2^-21.25 and 2^-45.2): a million points over 20,000 triangles, mixed, 19.5 ms at 20, 19.1 at 22, 19.0 at
+// 24, where 400,000 over 100,000 take 8.5, 8.7 and 8.7; 100,000 points over 20,000, FP64, 14.2 ms at 26, 13.5 at 28, 12.9 at 30.
 template <bool MIXED>
 struct Orders {
     static constexpr int P = MIXED ? 21 : 30;
@@ -185,7 +186,7 @@ __global__ __launch_bounds__(kP2MBlock) void k_tree_p2m(const double* __restrict
 
 // The same for several charge-density sets: one block per run expands each of its elements at unit charge density once
 // (half a wavefront per element, its nodes as above) and leaves the coefficients in LDS; the sets' expansions are sums
-// of them, a thread per coefficient (64 sets of 20,000 triangles 0.56 ms, and 2.7 ms the levels above).
+// of them, a thread per coefficient (64 sets of 20,000 triangles 0.56 ms, and 2.8 ms the levels above).
 template <int P>
 __global__ __launch_bounds__(kP2MBlock) void k_tree_p2m_sets(const double* __restrict__ geom,
                                                              const double* __restrict__ nodes,
@@ -642,7 +643,10 @@ constexpr int kTreeStack = 64 + 48 * (KEM_TREE_LEVELS + 1);
 // of their own).  The walk is the same for all of them, and the sums of a block's wavefronts are added in order
 // through LDS.  A run's coefficients pass through LDS too; the other wavefronts of the SIMD cover the wait for
 // them.  Three wavefronts per SIMD are asked for: a few registers spill, and the million mixed points over 20,000
-// triangles take 20.3 ms instead of 21.8 at two.  Bound by the vector ALU: half expansions, half pairs close by.
+// triangles take 18.8 ms instead of 22.2 at two, 100,000 in FP64 13.4 instead of 14.5.  Half expansions, half pairs close
+// by.  The vector ALU issues in 84 % of the cycles for the million, which binds it; in 60 to 70 % in FP64, for 64 sets and
+// for 400,000 points over 100,000 triangles, where chains of dependent FP64 operations and the loads of the coefficients
+// are not covered by three wavefronts.
 template <bool MIXED, int NP, bool TRIANGLES, bool SETS>
 __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu(3))) void k_field_tree(
     const double* __restrict__ geom, const double* __restrict__ nodes, const float* __restrict__ nodes32,
@@ -924,12 +928,18 @@ hipError_t tree_passes(hipStream_t st, const FieldMesh& m, const TreePlan& p, co
 // The hierarchical pass serves planar elements and wires under the numeric policy
 // (in mixed precision without an FP64 band), at 4,096 points or more, which the caller has put in curve order.
 // Below these sizes the flat pass is the faster one: its cost grows with elements times points, while here the
-// expansions take 0.2 ms and a group's walk its elements close by.  Measured, us flat / hierarchical:
-//   FP64   coax  5,000 x  8,192  1,566 / 1,814   10,000 x  8,192  3,061 / 2,450   20,000 x  4,096  3,405 / 3,781
-//          coax  2,500 x 16,384  1,418 / 1,494    5,000 x 16,384  2,654 / 2,495   20,000 x 65,536 34,820 / 13,273
-//          coax  1,000 x 131,072 3,453 / 3,694   cube 1,728 x 131,072  5,989 / 1,860
-//   mixed  coax  5,000 x 16,384  1,012 / 1,090    5,000 x 65,536  2,368 / 2,336   20,000 x 65,536  6,610 / 3,928
-//          coax  2,500 x 131,072 2,379 / 2,957   cube 3,072 x 131,072  1,958 / 820
+// expansions take 0.1 to 0.4 ms and a group's walk its elements close by.  Points in the gap of a closed surface (coax,
+// bore) have many of those, points around a body few, so the line lies between the sizes where either gains.  Measured,
+// us flat / hierarchical:
+//   FP64   coax  5,000 x  8,192  1,468 / 1,673   10,000 x  8,192  2,953 / 2,471   20,000 x  4,096  3,291 / 3,977
+//          coax  2,500 x 16,384  1,382 / 1,359    5,000 x 16,384  2,500 / 2,059   20,000 x 65,536 35,181 / 12,680
+//          coax  1,000 x 131,072 3,249 / 3,400    1,600 x 32,768  1,543 / 1,764    1,600 x 131,072 5,077 / 4,942
+//          cube  1,728 x 30,000  1,420 / 842      1,728 x 131,072 5,820 / 1,923
+//   mixed  coax  5,000 x 20,000  1,042 / 1,243    5,000 x 65,536  2,159 / 2,272    5,000 x 131,072 4,017 / 3,360
+//          coax  2,500 x 131,072 2,254 / 2,808    3,100 x 131,072 2,547 / 3,018   20,000 x 65,536  6,453 / 3,737
+//          bore  5,000 x 131,072 3,781 / 4,677   10,000 x 33,000  2,706 / 2,055   30,000 x 33,000  5,425 / 2,781
+//          cube  3,072 x 33,000    571 / 441      3,072 x 131,072 1,875 / 897
+//          rectangles and wires  3,200 x 33,000  778 / 637   x 131,072  2,567 / 1,615
 constexpr int64_t kTreeMinPoints = 4096;
 inline bool tree_pays(bool mixed, double n, double m)
 {
@@ -938,12 +948,18 @@ inline bool tree_pays(bool mixed, double n, double m)
 }
 // Points of several sets are visited set by set, so the groups are less compact the fewer points a set has, and each set
 // has its expansions: the pass serves them from a product of elements and points per set on.  Measured on the coax, us
-// flat / hierarchical (elements x points x sets):
-//   FP64   6,000 x 80,000 x 8  11,886 / 9,498   x 16  11,975 / 11,430   x 32  11,983 / 13,634
-//          20,000 x 300,000 x 2  147,681 / 32,920   x 64  151,516 / 78,499   20,000 x 80,000 x 64  41,528 / 41,429
-//   mixed  20,000 x 80,000 x 8  8,078 / 7,022   x 16  8,157 / 8,717   12,000 x 80,000 x 4  5,070 / 4,413
-//          20,000 x 300,000 x 2  26,031 / 9,702   x 32  26,266 / 21,063   x 64  37,562 / 27,769 (there the flat pass's
-//          element weights no longer fit an XCD's L2)   6,000 x 300,000 x 16  11,265 / 10,029   x 32  11,382 / 11,934
+// flat / hierarchical (elements x points x sets, product per set):
+//   FP64   6,000 x 80,000 x 16  3.0e7  13,101 / 11,503   x 32  1.5e7  13,110 / 13,104
+//          20,000 x 80,000 x 64  2.5e7  41,728 / 39,288   20,000 x 300,000 x 64  9.4e7  148,520 / 75,234
+//   mixed  20,000 x 80,000 x 8  2.0e8  7,903 / 6,352   x 16  1.0e8  7,835 / 8,596
+//          20,000 x 160,000 x 16  2.0e8  13,728 / 11,543   x 32  1.0e8  14,448 / 15,346
+//          12,000 x 80,000 x 4  2.4e8  5,072 / 4,422   x 8  1.2e8  5,038 / 5,081
+//          6,000 x 160,000 x 4  2.4e8  5,061 / 4,989   x 8  1.2e8  5,100 / 5,895
+//          and with 300,000 points, where the sides meet lower:
+//          20,000 x 32  1.9e8  25,841 / 19,989   x 64  9.4e7  36,158 / 26,060   12,000 x 32  1.1e8  17,160 / 15,845
+//          x 64  5.6e7  22,557 / 20,036   6,000 x 8  2.2e8  9,468 / 8,402   x 16  1.1e8  9,449 / 9,644
+// (the flat pass's own times rise with elements x sets: its weights, 6 and 10 MB for 64 sets of 12,000 and 20,000
+// elements, no longer fit an XCD's 4 MB of L2).
 constexpr int64_t kTreeMaxSets = 65535;
 inline bool sets_pay(bool mixed, double n, double m, double nsets)
 {
@@ -951,12 +967,13 @@ inline bool sets_pay(bool mixed, double n, double m, double nsets)
     return mixed ? each >= (m >= 262144. && n >= 6000. ? 9e7 : 1.9e8) : each >= 3.5e7;
 }
 // wavefronts in all: kTreeWaves times p.slices of them per group of points.  Many more than the chip holds at once, since
-// groups differ in their work, a few by 10 times (400,000 points over 100,000 triangles: 18.2 ms at 8 per group,
-// 14.1 at 16, 10.8 at 64; a million points over 20,000: 27.2, 25.2 at 8, 25.7 at 32).
+// groups differ in their work, a few by 10 times (400,000 points over 100,000 triangles: 15.5 ms at 8 per group,
+// 11.3 at 16, 9.3 at 32, 8.8 at the 40 that this gives, 8.4 at 64; a million points over 20,000: 21.0 at 8, 18.8 at the 16
+// that this gives, 19.2 at 32, 21.3 at 64).
 constexpr int64_t kTreeWavefronts = 131072;
 constexpr int kTreeMaxSlices = 16;
 // From this many points on, two per lane; below, groups of 64 points are the more compact ones (20,000-triangle coax,
-// mixed: 16,384 points 2.51 ms with two, 1.99 with one; 65,536 points 4.15 and 3.93).
+// mixed: 16,384 points 2.41 ms with two, 1.98 with one; 65,536 points 4.27 and 3.72; 131,072 points 4.90 and 5.00).
 constexpr int64_t kTreePairPoints = 65537;
 // Expansions of calls that the no-allocation entry point may serve (up to 65,536 points) fit its scratch beside
 // the points' ordering, partial sums and the group members' charge densities; other calls' are bounded by 4 GiB.  Runs of
