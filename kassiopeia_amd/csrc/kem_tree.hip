@@ -722,7 +722,7 @@ __global__ __launch_bounds__(64 * kTreeWaves) __attribute__((amdgpu_waves_per_eu
                 idx = (e & ((1 << KEM_TREE_INDEX_BITS) - 1)) * KEM_TREE_FAN + (lane & 3);
                 have = have && idx < T.count[lev];
             }
-            const int at = have ? T.first[lev] + idx : 0;
+            const int at = have ? T.first[lev] + idx : T.first[T.low];  // a lane without a run reads the first one
             const double* t = tnode + (int64_t)at * KEM_TREE_STRIDE;
             const double dx = t[0] - wx, dy = t[1] - wy, dz = t[2] - wz;
             const double d = sqrt(dx * dx + dy * dy + dz * dz) * (1. - 1e-9) - wr;
