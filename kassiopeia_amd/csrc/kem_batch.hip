@@ -184,7 +184,8 @@ constexpr int kReduceRows = 16;  // rows per block of k_bmm32_reduce
 // memory (one split per round trip: 9 splits of a 20,000 x 64 block in 41 us; 32 rows and
 // four splits per round trip: 20 us for 6 splits); the sums are transposed through LDS so that
 // the writes run along rows.  WHOLE (a caller's right-hand sides through k_bmm32s): column c was multiplied with scale[c],
-// and sums that are not numbers are formed again from matrix and panel.
+// and sums that are not numbers are formed again from matrix and panel (9 ms for 20,000 rows with an infinite right-hand side),
+// unless the column itself holds one (scale[c] < 0).
 template <int KP, typename P = float, bool WHOLE = false>
 __global__ __launch_bounds__(kBlock) void k_bmm32_reduce(const P* __restrict__ part, int nsplit, int64_t n,
                                                          int ncols, double* __restrict__ W, int64_t ldw,
@@ -220,9 +221,11 @@ __global__ __launch_bounds__(kBlock) void k_bmm32_reduce(const P* __restrict__ p
         for (int m = 0; m < E; m++) {
             const int e = threadIdx.x + kBlock * m, c = e % KP;
             s[m] *= 1. / (double)scale[c];
-            if (s[m] == s[m] || e >= lim || c >= ncols) continue;
+            if (scale[c] < 0.f) s[m] = __builtin_nan("");
+            if (s[m] == s[m] || scale[c] < 0.f || e >= lim || c >= ncols) continue;
             const float* a = A + i0 + e / KP;
             double t = 0.;
+#pragma unroll 8
             for (int64_t j = 0; j < n; j++) t += (double)(a[j * n] * panel[j * KP + c]);
             s[m] = t;
         }
@@ -357,8 +360,9 @@ __device__ __forceinline__ void split8(const float (&v)[8], bf8v (&o)[3])
     for (int k = 0; k < 3; k++) o[k] = __builtin_bit_cast(bf8v, uint4{w[k][0], w[k][1], w[k][2], w[k][3]});
 }
 
-// scale[c] = 2^64 where the column's largest number, as FP32, is below 2^-64 (and not 0), else 1: one block per column of the
-// panel, those from ncols on 1
+// scale[c] = 2^64 where the column's largest number, as FP32, is below 2^-64 (and not 0), -1 where it holds a not-a-number,
+// so that its products are not formed twice (k_bmm32_reduce), else 1: one block per column of the panel, those from ncols
+// on 1
 constexpr int kScaleBlock = 1024;
 __global__ __launch_bounds__(kScaleBlock) void k_column_scale(const double* __restrict__ X, int64_t ldx, int64_t n,
                                                               int ncols, float* __restrict__ scale)
@@ -366,14 +370,19 @@ __global__ __launch_bounds__(kScaleBlock) void k_column_scale(const double* __re
     __shared__ float sh[kScaleBlock / 64];
     const int c = blockIdx.x;
     float top = 0.f;
+    int nan = 0;
     if (c < ncols)
-        for (int64_t i = threadIdx.x; i < n; i += kScaleBlock) top = fmaxf(top, fabsf((float)X[c * ldx + i]));
+        for (int64_t i = threadIdx.x; i < n; i += kScaleBlock) {
+            const float v = (float)X[c * ldx + i];
+            top = fmaxf(top, fabsf(v));
+            nan |= v != v;
+        }
     for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o, 64));
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = top;
-    __syncthreads();
+    nan = __syncthreads_or(nan);
     if (threadIdx.x != 0) return;
     for (int k = 1; k < kScaleBlock / 64; k++) top = fmaxf(top, sh[k]);
-    scale[c] = top > 0.f && top < 0x1p-64f ? 0x1p64f : 1.f;
+    scale[c] = nan ? -1.f : top > 0.f && top < 0x1p-64f ? 0x1p64f : 1.f;
 }
 
 // the panel's parts in operand order: [chunk][part][tile of 32 columns][lane], rows past n zero, column c times scale[c]
